@@ -48,12 +48,6 @@ __device__ __forceinline__ double wave_sum_f64(double x) {
   return x;
 }
 
-__device__ __forceinline__ int64_t shfl_i64_bc(int64_t x, int src) {
-  const uint32_t lo = __shfl((uint32_t)((uint64_t)x & 0xFFFFFFFFull), src, 64);
-  const uint32_t hi = __shfl((uint32_t)((uint64_t)x >> 32), src, 64);
-  return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
 __global__ void level_keys_kernel(const int32_t* depth, int64_t n, int32_t nlevels, uint32_t* keys, int32_t* ids) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const int32_t d = depth[i];
@@ -124,7 +118,7 @@ __device__ __forceinline__ void gather_level(const int32_t* order, int64_t begin
     while (heavy) {
       const int k = __ffsll((unsigned long long)heavy) - 1;
       heavy &= heavy - 1;
-      const int64_t ka = shfl_i64_bc(a, k), kb = shfl_i64_bc(b, k);
+      const int64_t ka = (int64_t)wave_lane((uint64_t)a, k), kb = (int64_t)wave_lane((uint64_t)b, k);
       double part = 0.0;
       for (int64_t e = ka + lane; e < kb; e += 64) part += arc(e);
       part = wave_sum_f64(part);

@@ -126,7 +126,7 @@ __device__ __forceinline__ void pull_level(const BfsArgs<OffT>& a, int variant, 
     if (myw == a.w0 - 1 && tail_bits) myun &= (1ull << tail_bits) - 1ull;
     const uint32_t cnt = (uint32_t)__popcll(myun);
     const uint32_t incl = wave_inclusive_scan(cnt);
-    const uint32_t total = shfl(incl, 63);
+    const uint32_t total = wave_lane(incl, 63);
     wnew[lane] = 0ull;
     for (uint32_t t0 = 0; t0 < total; t0 += 64 * kPullBatch) {
       uint32_t vv[kPullBatch];
@@ -230,9 +230,9 @@ __device__ __forceinline__ void pull_level(const BfsArgs<OffT>& a, int variant, 
         while (pending) {
           const int k2 = __ffsll((unsigned long long)pending) - 1;
           pending &= pending - 1;
-          const int64_t jb = shfl_i64((int64_t)j, k2);
-          const int64_t je = shfl_i64((int64_t)e, k2);
-          const int64_t bb = shfl_i64((int64_t)b, k2);
+          const int64_t jb = (int64_t)wave_lane((uint64_t)j, k2);
+          const int64_t je = (int64_t)wave_lane((uint64_t)e, k2);
+          const int64_t bb = (int64_t)wave_lane((uint64_t)b, k2);
           int64_t hit_pos = -1;
           for (int64_t jj = jb; jj < je; jj += 64) {
             const int64_t my = jj + lane;
@@ -717,7 +717,7 @@ __device__ __forceinline__ void burst_visit_small(const BurstArgs<OffT>& a, cons
     qe.len = 0;
     if (base + lane < cnt) qe = ents[base + lane];
     const uint32_t incl = wave_inclusive_scan((uint32_t)qe.len);
-    const uint32_t total = __shfl(incl, 63, 64);
+    const uint32_t total = wave_lane(incl, 63);
     const uint32_t excl = incl - (uint32_t)qe.len;
     for (uint32_t t0 = 0; t0 < total; t0 += 4 * 64) {
       uint32_t y[4];
@@ -1029,7 +1029,7 @@ __device__ __forceinline__ void gb_claim4(const GbArgs<OffT>& a, const uint32_t 
     np += npc[k];
   }
   const uint32_t is = wave_inclusive_scan(ns), ip = wave_inclusive_scan(np);
-  const uint32_t ts = __shfl(is, 63, 64), tp = __shfl(ip, 63, 64);
+  const uint32_t ts = wave_lane(is, 63), tp = wave_lane(ip, 63);
   if ((ts | tp) == 0) return;
   unsigned long long bs = 0, bp = 0;
   if (lane == 63) {
@@ -1075,7 +1075,7 @@ __device__ __forceinline__ void gb_visit_small(const GbArgs<OffT>& a, const QEnt
       if (coherent) atomic_or(&a.prev[(uint32_t)qe.v >> 6], 1ull << (qe.v & 63));
     }
     const uint32_t incl = wave_inclusive_scan((uint32_t)qe.len);
-    const uint32_t total = __shfl(incl, 63, 64);
+    const uint32_t total = wave_lane(incl, 63);
     const uint32_t excl = incl - (uint32_t)qe.len;
     for (uint32_t t0 = 0; t0 < total; t0 += 4 * 64) {
       uint32_t y[4];

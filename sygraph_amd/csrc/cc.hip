@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(kBlock) sym_hash_kernel(const OffT* off, const
     while (heavy) {
       const int k = __ffsll((unsigned long long)heavy) - 1;
       heavy &= heavy - 1;
-      const int64_t kb = shfl_i64(b, k), ke = shfl_i64(e, k);
+      const int64_t kb = (int64_t)wave_lane((uint64_t)b, k), ke = (int64_t)wave_lane((uint64_t)e, k);
       const uint32_t ku = (uint32_t)(base + k);
       for (int64_t j = kb + lane; j < ke; j += 64) {
         const uint32_t v = (uint32_t)cols[j];
@@ -382,7 +382,7 @@ __device__ __forceinline__ void wave_word_arcs(const OffT* off, const int32_t* c
   while (heavy) {
     const int k = __ffsll((unsigned long long)heavy) - 1;
     heavy &= heavy - 1;
-    const int64_t kb = shfl_i64(b, k), ke = shfl_i64(e, k);
+    const int64_t kb = (int64_t)wave_lane((uint64_t)b, k), ke = (int64_t)wave_lane((uint64_t)e, k);
     const uint32_t ku = (uint32_t)(w * 64 + k);
     for (int64_t j = kb + lane; j < ke; j += 64) f(ku, (uint32_t)cols[j]);
   }

@@ -236,7 +236,7 @@ __device__ __noinline__ bool grid_sync(Ctl* c, uint32_t& t, uint64_t wait_ticks)
 /* this lane's first slot of k, with one atomic per wave (all lanes call) */
 __device__ __forceinline__ uint64_t wave_reserve(unsigned long long* ctr, uint32_t k) {
   const uint32_t incl = wave_inclusive_scan(k);
-  const uint32_t total = __shfl(incl, 63, 64);
+  const uint32_t total = wave_lane(incl, 63);
   unsigned long long base = 0;
   if (total) {
     if (lane_id() == 63) base = atomic_add(ctr, (unsigned long long)total);
@@ -488,7 +488,7 @@ __device__ __forceinline__ PairWalk pair_walk(uint64_t mine, int64_t len) {
   w.words = ballot(mine != 0);
   w.pc = (uint32_t)__popcll(mine);
   w.incl = wave_inclusive_scan(w.pc);
-  w.total = __shfl(w.incl, 63, 64);
+  w.total = wave_lane(w.incl, 63);
   const uint32_t flat_steps = (w.total + 63) / 64, word_steps = (uint32_t)__popcll(w.words);
   const uint64_t l = mine ? (uint64_t)len + 1 : 0ull;
   const uint64_t word_cost = wave_sum_u64(l), flat_cost = (uint64_t)flat_steps * wave_max_u64(l);
@@ -565,7 +565,7 @@ __device__ __forceinline__ void expand_push(const MsArgs<OffT>& a, int32_t d, in
       }
     }
     const uint32_t incl = wave_inclusive_scan(len);
-    const uint32_t total = __shfl(incl, 63, 64);
+    const uint32_t total = wave_lane(incl, 63);
     const uint32_t excl = incl - len;
     for (uint32_t t0 = 0; t0 < total; t0 += 4 * 64) {
       int32_t v[4];
@@ -642,8 +642,8 @@ __device__ __forceinline__ void expand_pull(const MsArgs<OffT>& a, const uint64_
     while (heavy) {
       const int k = __ffsll((unsigned long long)heavy) - 1;
       heavy &= heavy - 1;
-      const int64_t kb = shfl_i64(b, k), ke = shfl_i64(e, k);
-      const uint64_t kwant = shfl_u64(want, k);
+      const int64_t kb = (int64_t)wave_lane((uint64_t)b, k), ke = (int64_t)wave_lane((uint64_t)e, k);
+      const uint64_t kwant = wave_lane(want, k);
       uint64_t part = 0;
       for (int64_t j0 = kb; j0 < ke; j0 += 64) {
         if (j0 + lane < ke) part |= cld(&Mc[a.icols[j0 + lane]]);

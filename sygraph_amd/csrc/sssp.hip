@@ -125,7 +125,7 @@ __device__ __forceinline__ unsigned long long heavy_pull(const SsspArgs<OffT, W>
     if (myw == a.w0 - 1 && tail_bits) myun &= (1ull << tail_bits) - 1ull;
     const uint32_t c = (uint32_t)__popcll(myun);
     const uint32_t incl = wave_inclusive_scan(c);
-    const uint32_t total = __shfl(incl, 63, 64);
+    const uint32_t total = wave_lane(incl, 63);
     for (uint32_t t0 = 0; t0 < total; t0 += 64) {
       const uint32_t t = t0 + lane;
       const int owner = scan_owner(incl, t);
@@ -162,7 +162,7 @@ __device__ __forceinline__ unsigned long long heavy_pull(const SsspArgs<OffT, W>
       while (pending) {
         const int k2 = __ffsll((unsigned long long)pending) - 1;
         pending &= pending - 1;
-        const int64_t jb = shfl_i64(j, k2), je = shfl_i64(e, k2);
+        const int64_t jb = (int64_t)wave_lane((uint64_t)j, k2), je = (int64_t)wave_lane((uint64_t)e, k2);
         uint32_t m = 0xFFFFFFFFu;
         for (int64_t jj = jb + lane; jj < je; jj += 64) {
           const uint32_t u = (uint32_t)a.cols[jj];

@@ -185,7 +185,7 @@ __global__ void __launch_bounds__(kBlock) intersect_kernel(const int64_t* dag_of
         while (longs) {
           const int k2 = __ffsll((unsigned long long)longs) - 1;
           longs &= longs - 1;
-          const int64_t lb = shfl_i64(vb, k2);
+          const int64_t lb = (int64_t)wave_lane((uint64_t)vb, k2);
           const uint32_t ll = (uint32_t)__shfl((uint32_t)vlen, k2, 64);
           for (uint32_t j0 = 0; j0 < ll; j0 += kTcUnroll * 64) {
 #pragma unroll
@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(kBlock) intersect_kernel(const int64_t* dag_of
         /* short lists: laid end to end, a lane per arc */
         const uint32_t slen = is_long ? 0u : (uint32_t)vlen;
         const uint32_t incl = wave_inclusive_scan(slen);
-        const uint32_t tot = __shfl(incl, 63, 64);
+        const uint32_t tot = wave_lane(incl, 63);
         const uint32_t excl = incl - slen;
         for (uint32_t t0 = 0; t0 < tot; t0 += kTcUnroll * 64) {
 #pragma unroll

@@ -135,12 +135,7 @@ inline Tuning default_tuning() { return Tuning{64, 1024, 1024}; }
 
 /* ------------------------------------------------------------ helpers --- */
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t x) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    uint32_t t = __shfl_up(x, o, 64);
-    if (lane_id() >= o) x += t;
-  }
-  return x;
+  return wave_prefix(x, [](uint32_t a, uint32_t b) { return a + b; });
 }
 
 /* 64-bit value of lane `src` (src may differ per lane; all lanes active) */
@@ -248,7 +243,7 @@ __device__ __forceinline__ TileWalk tile_walk(uint64_t mine) {
   w.words = ballot(mine != 0);
   w.pc = (uint32_t)__popcll(mine);
   w.incl = wave_inclusive_scan(w.pc);
-  w.total = __shfl(w.incl, 63, 64);
+  w.total = wave_lane(w.incl, 63);
   const uint32_t flat_steps = (w.total + 63) / 64, word_steps = (uint32_t)__popcll(w.words);
   w.flat = flat_steps < word_steps;
   w.steps = w.flat ? flat_steps : word_steps;
@@ -269,7 +264,7 @@ __device__ __forceinline__ bool tile_walk_item(TileWalk& w, uint64_t mine, int64
   }
   const int k = __ffsll((unsigned long long)w.words) - 1; /* the step-th non-empty word */
   w.words &= w.words - 1;
-  const uint64_t word = shfl_u64(mine, k);
+  const uint64_t word = wave_lane(mine, k);
   v = (tile * 64 + k) * 64 + lane;
   return (word >> lane) & 1ull;
 }
@@ -542,7 +537,7 @@ __device__ __forceinline__ bool compact_write_body_at(const CompactArgs<OffT>& a
         a.qout[2][p + c] = ce;
       }
     }
-    pos2 += __shfl(incl, 63, 64);
+    pos2 += wave_lane(incl, 63);
   }
   return wrote;
 }
@@ -647,7 +642,7 @@ __device__ __forceinline__ void for_each_queued_arc4(QEntry* const q[3], const Q
       qe.len = 0;
       if (i < cnt) qe = qq[i];
       const uint32_t incl = wave_inclusive_scan((uint32_t)qe.len);
-      const uint32_t total = __shfl(incl, 63, 64);
+      const uint32_t total = wave_lane(incl, 63);
       const uint32_t excl = incl - (uint32_t)qe.len;
       for (uint32_t t0 = 0; t0 < total; t0 += 4 * 64) {
 #pragma unroll
@@ -712,7 +707,7 @@ __device__ __forceinline__ void for_each_queued_arc(QEntry* const q[3], const Qu
       qe.len = 0;
       if (i < cnt) qe = qq[i];
       const uint32_t incl = wave_inclusive_scan((uint32_t)qe.len);
-      const uint32_t total = __shfl(incl, 63, 64);
+      const uint32_t total = wave_lane(incl, 63);
       for (uint32_t t0 = 0; t0 < total; t0 += 64) {
         const uint32_t t = t0 + lane;
         const int owner = scan_owner(incl, t);
