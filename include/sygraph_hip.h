@@ -394,8 +394,9 @@ typedef struct sg_sssp_options {
                             from the settled set; push: every heavy arc of the settled set is
                             relaxed with an atomic minimum.  Directed graphs always push. */
   int32_t burst_arcs;    /* rounds of the reference's schedule (no buckets) with at most this many
-                            arcs run back to back inside one workgroup while they stay that small:
-                            0 = default (4,096), negative = never, at most 8,192 */
+                            arcs run back to back inside one workgroup while they stay that small,
+                            and larger ones of at most 2^17 arcs in one launch of resident
+                            workgroups: 0 = default (4,096), negative = neither, at most 8,192 */
   int32_t record_relax;  /* 1: time every relax launch on its own (two events per round; stats must
                             not be NULL): stats->relax_ms / relax_launches */
 } sg_sssp_options;

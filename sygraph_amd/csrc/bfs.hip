@@ -33,9 +33,11 @@
 using namespace sygraph::hipdev;
 
 #include "policy.hpp"
+#include "gridburst.hpp"
 #include "traverse.hpp"
 
 using namespace sg::trav;
+namespace gb = sg::gb;
 
 namespace {
 
@@ -931,10 +933,8 @@ __global__ void __launch_bounds__(kBurstThreads) write_dyn_kernel(CompactArgs<Of
 /* Push levels too large for one workgroup but far too small to fill the chip
  * (a 4096 x 4096 grid has ~8,000 levels of a few thousand arcs each) still
  * pay the ~25 us of a step's three launches.  A grid burst runs such levels
- * in one cooperative launch, with one grid barrier per level instead: every
- * workgroup of the launch is co-resident, the frontier lives in two global
- * lists, and the totals that decide the next level are summed with atomics
- * and read by every workgroup after the barrier, so all of them take the
+ * in one launch of resident workgroups (gridburst.hpp), one exchange per
+ * level, after which every workgroup knows the level's totals and takes the
  * same decision.  It starts from the queues the previous step wrote (like
  * level_kernel), keeps going while the policy pushes and the frontier has at
  * most gb_arcs arcs, and hands the level at which it stops back exactly like
@@ -942,311 +942,351 @@ __global__ void __launch_bounds__(kBurstThreads) write_dyn_kernel(CompactArgs<Of
  * discoveries in visited and depth but not in prev, so that the same step's
  * level_kernel skips it and its count pass counts and decides it.
  *
- * Lists: short adjacency lists (< kBurstBig arcs) as one entry each, laid
- * end to end 64 at a time by a wave (merge path); longer ones as pieces of
- * kGbPiece arcs, one wave per piece, so a hub is spread over many waves. */
-constexpr int kGbThreads = 512;
-constexpr int kGbWaves = kGbThreads / 64;
-constexpr int kGbPiece = 256;
+ * 3001 x 2999 grid: 10.4 -> 5.1 us a level (48.7 -> 24.1 ms), of which the
+ * visit's chain (entry, visited word and list bounds, claim and heads, the
+ * next entry) takes about 2.2 and the exchange the rest.  The 10.4 went to
+ * the lists' global counter, the merge path's searches, one load per offset
+ * and head, and a barrier of three round trips. */
 constexpr int64_t kGbDefaultArcs = 1 << 18;
 constexpr int64_t kGbMaxArcs = 1 << 24;
+constexpr int kGbMaxWgs = gb::kMaxWgs;
 
-/* per level: entries of the next short list and pieces of the next long
- * list (three rotating copies, so the copy a level adds into was cleared two
- * levels earlier and read one level earlier) */
-struct alignas(128) GbSums {
-  unsigned long long nsmall, npieces;
-  unsigned long long pad[14];
-};
-
-/* per workgroup and level: its discoveries, their arcs and their largest
- * degree, written by the workgroup and read by every workgroup after the
- * level's barrier (two rotating copies: a workgroup writes a copy only after
- * the barrier that follows every read of its previous contents).  One slot
- * per workgroup, not a shared atomic counter: hundreds of workgroups adding
- * into one line serialize for tens of microseconds per level. */
-constexpr int kGbMaxWgs = 1024;
-/* Default workgroups of a grid burst: the levels it takes have at most 2^18
- * arcs, sixteen per lane of 32 workgroups of 512; a level's time is its
- * busiest waves' memory round trips plus the barrier, and fewer workgroups
- * make the barrier cheaper (8 to 512 swept on the 4096^2 grid: 8 to 64
- * alike, 6 % slower at 256, 12 % at 512). */
-constexpr int kGbDefaultWgs = 32;
-struct alignas(32) GbSlot {
-  unsigned long long disc, deg, mx, pad;
-};
-
+/* List entries of short adjacency lists: vertex | length << 32, first arc,
+ * and for lists of at most gb::kInline arcs the heads themselves, loaded
+ * while the vertex's claim is in flight, so the next level starts at the
+ * claims instead of at the adjacency. */
 template<typename OffT>
 struct GbArgs {
   const OffT* off;
   const int32_t* cols;
+  int64_t m; /* arcs */
   uint64_t* visited;
   uint64_t* prev;
   int32_t* depth;
   QEntry* q[3]; /* the queues of the level about to run */
   const QueueHdr* hdr;
-  QEntry* small[2];
+  /* [parity]: `total` entries of two words (vertex and length; first arc),
+   * then `total` x gb::kInline heads; the segments of the workgroups, seg_cap
+   * entries each */
+  uint64_t* list[2];
+  int64_t total;
+  uint32_t seg_cap;
   QEntry* pieces[2];
-  int64_t cap_small, cap_pieces;
-  GbSums* sums;  /* [3] */
-  GbSlot* slots; /* [2][kGbMaxWgs] */
-  GridBar* bar;
+  int64_t cap_pieces;
+  gb::Exchange x;
+  LevelLog* log; /* the burst's level records, copied to the host's at its end */
   int64_t gb_arcs;
-  uint64_t wait_ticks;
+  uint32_t stride; /* the burst's workgroups are those with blockIdx.x % stride == 0 */
 };
 
-/* Claim the (up to) four arcs y[k] of each lane; new vertices get depth
- * level + 1 and join the short list or, cut into pieces, the long list. */
 template<typename OffT>
-__device__ __forceinline__ void gb_claim4(const GbArgs<OffT>& a, const uint32_t (&y)[4], const bool (&ok)[4],
-                                          int32_t level, QEntry* out_small, QEntry* out_pieces, GbSums* sm,
-                                          BurstAcc& acc) {
-  const int lane = lane_id();
-  uint64_t old[4];
-  int64_t vs[4], ve[4];
+struct GbOut {
+  uint64_t* list;
+  uint32_t rank, wgs;
+  QEntry* pieces;
+  gb::Sums* sums;
+  gb::Local* local;
+  int32_t level;
+};
+
+/* Claim the (up to) K arcs y[k] of each lane; new vertices get depth
+ * level + 1 and join the workgroup's segment or, cut into pieces, the long
+ * list.  Two memory round trips: the visited words with the heads' list
+ * bounds, then the claims with the heads of the short lists. */
+template<int K, typename OffT>
+__device__ __forceinline__ void gb_claim(const GbArgs<OffT>& a, const uint32_t (&y)[K], const bool (&ok)[K],
+                                         const GbOut<OffT>& o, gb::Acc& acc) {
+  uint64_t w[K];
+  int64_t vs[K], ve[K];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    old[k] = ~0ull;
+  for (int k = 0; k < K; ++k) {
+    w[k] = ~0ull;
     vs[k] = ve[k] = 0;
     if (ok[k]) {
-      const uint64_t bit = 1ull << (y[k] & 63);
-      const uint64_t w = a.visited[y[k] >> 6];
-      if (!(w & bit)) {
-        old[k] = atomic_or(&a.visited[y[k] >> 6], bit);
-        vs[k] = (int64_t)a.off[y[k]];
-        ve[k] = (int64_t)a.off[y[k] + 1];
-      }
+      w[k] = a.visited[y[k] >> 6];
+      list_bounds(a.off, y[k], vs[k], ve[k]);
     }
   }
-  bool nw[4];
-  uint32_t ns = 0, np = 0, npc[4];
+  uint64_t old[K];
+  uint32_t id[K][gb::kInline];
+  bool nw[K];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    nw[k] = ((old[k] >> (y[k] & 63)) & 1ull) == 0ull;
-    const int64_t len = ve[k] - vs[k];
-    npc[k] = (nw[k] && len >= kBurstBig) ? (uint32_t)((len + kGbPiece - 1) / kGbPiece) : 0u;
-    ns += (nw[k] && len < kBurstBig) ? 1u : 0u;
-    np += npc[k];
+  for (int k = 0; k < K; ++k) {
+    const uint64_t bit = 1ull << (y[k] & 63);
+    nw[k] = !(w[k] & bit);
+    old[k] = ~0ull;
+    if (nw[k]) old[k] = atomic_or(&a.visited[y[k] >> 6], bit);
+    if (nw[k] && ve[k] - vs[k] <= gb::kInline) load_ids4(a.cols, vs[k], a.m, id[k]);
   }
-  const uint32_t is = wave_inclusive_scan(ns), ip = wave_inclusive_scan(np);
-  const uint32_t ts = wave_lane(is, 63), tp = wave_lane(ip, 63);
-  if ((ts | tp) == 0) return;
-  unsigned long long bs = 0, bp = 0;
-  if (lane == 63) {
-    if (ts) bs = atomic_add(&sm->nsmall, (unsigned long long)ts);
-    if (tp) bp = atomic_add(&sm->npieces, (unsigned long long)tp);
-  }
-  bs = (unsigned long long)shfl_i64((int64_t)bs, 63) + (is - ns);
-  bp = (unsigned long long)shfl_i64((int64_t)bp, 63) + (ip - np);
+  uint64_t ms[K];
+  uint32_t cs = 0;
+  bool pieces = false;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (!nw[k]) continue;
-    const uint32_t v = y[k];
-    const int64_t len = ve[k] - vs[k];
-    a.depth[v] = level + 1;
-    ++acc.disc;
-    acc.deg += (unsigned long long)len;
-    acc.mx = (unsigned long long)len > acc.mx ? (unsigned long long)len : acc.mx;
-    if (npc[k] == 0) {
-      if ((int64_t)bs < a.cap_small) store_entry_coherent(out_small + bs, QEntry{vs[k], (int32_t)v, (int32_t)len});
-      ++bs;
-    } else {
-      for (uint32_t c = 0; c < npc[k]; ++c, ++bp) {
-        const int64_t o = (int64_t)c * kGbPiece;
-        const int64_t l = len - o < kGbPiece ? len - o : kGbPiece;
-        if ((int64_t)bp < a.cap_pieces) store_entry_coherent(out_pieces + bp, QEntry{vs[k] + o, (int32_t)v, (int32_t)l});
+  for (int k = 0; k < K; ++k) {
+    nw[k] = nw[k] && ((old[k] >> (y[k] & 63)) & 1ull) == 0ull;
+    const bool big = ve[k] - vs[k] >= kBurstBig;
+    ms[k] = ballot(nw[k] && !big);
+    cs += (uint32_t)__popcll(ms[k]);
+    pieces = pieces || (nw[k] && big);
+  }
+  const bool any_pieces = ballot(pieces) != 0;
+  if (cs == 0 && !any_pieces) return;
+  uint32_t at = 0;
+  if (cs) {
+    if (lane_id() == 0) at = atomicAdd(&o.local->cnt, cs);
+    at = __builtin_amdgcn_readfirstlane(at);
+    acc.disc += cs;
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const uint32_t len = (uint32_t)(ve[k] - vs[k]);
+    if (ms[k]) {
+      const bool mine = nw[k] && len < (uint32_t)kBurstBig;
+      const uint32_t l = mine ? len : 0u;
+      const uint32_t mx = wave_max_u32(l);
+      acc.deg += wave_sum_u32(l); /* short lists: 64 lengths below 64 */
+      acc.mx = mx > acc.mx ? mx : acc.mx;
+      const uint32_t p = at + lanes_below(ms[k]);
+      if (mine && p < a.seg_cap) {
+        const int64_t i = gb::entry_at(o.rank, p, o.wgs);
+        put_coherent(o.list + i, (uint64_t)y[k] | (uint64_t)len << 32);
+        if (len <= (uint32_t)gb::kInline) {
+          uint64_t* h = o.list + 2 * a.total + 2 * i;
+          put_coherent(h, (uint64_t)id[k][0] | (uint64_t)id[k][1] << 32);
+          put_coherent(h + 1, (uint64_t)id[k][2] | (uint64_t)id[k][3] << 32);
+        } else {
+          put_coherent(o.list + a.total + i, (uint64_t)vs[k]);
+        }
       }
+      at += (uint32_t)__popcll(ms[k]);
+    }
+    if (nw[k]) a.depth[y[k]] = o.level + 1;
+  }
+  if (!any_pieces) return;
+  uint32_t np = 0, npc[K];
+  unsigned long long deg = 0, mx = 0;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int64_t len = ve[k] - vs[k];
+    npc[k] = (nw[k] && len >= kBurstBig) ? (uint32_t)((len + gb::kPiece - 1) / gb::kPiece) : 0u;
+    np += npc[k];
+    if (npc[k]) {
+      deg += (unsigned long long)len;
+      mx = (unsigned long long)len > mx ? (unsigned long long)len : mx;
+    }
+    acc.disc += (uint32_t)__popcll(ballot(npc[k] != 0));
+  }
+  const uint32_t ip = wave_inclusive_scan(np);
+  const uint32_t tp = wave_lane(ip, 63);
+  unsigned long long bp = 0;
+  if (lane_id() == 63) bp = atomic_add(&o.sums->npieces, (unsigned long long)tp);
+  bp = (unsigned long long)shfl_i64((int64_t)bp, 63) + (ip - np);
+  acc.deg += wave_sum_u64(deg);
+  mx = wave_max_u64(mx);
+  acc.mx = (uint32_t)mx > acc.mx ? (uint32_t)mx : acc.mx;
+  acc.npieces = tp > gb::kPiecesClamp || acc.npieces + tp > gb::kPiecesClamp ? gb::kPiecesClamp : acc.npieces + tp;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int64_t len = ve[k] - vs[k];
+    for (uint32_t c = 0; c < npc[k]; ++c, ++bp) {
+      const int64_t at_arc = (int64_t)c * gb::kPiece;
+      const int64_t l = len - at_arc < gb::kPiece ? len - at_arc : gb::kPiece;
+      if ((int64_t)bp < a.cap_pieces)
+        store_entry_coherent(o.pieces + bp, QEntry{vs[k] + at_arc, (int32_t)y[k], (int32_t)l});
     }
   }
 }
 
-/* short lists, 64 entries per wave laid end to end, four arcs per lane per round */
+/* 64 lists of a wave laid end to end (merge path), four arcs per lane per round */
 template<typename OffT>
-__device__ __forceinline__ void gb_visit_small(const GbArgs<OffT>& a, const QEntry* ents, int64_t cnt, int32_t level,
-                                               QEntry* out_small, QEntry* out_pieces, GbSums* sm, BurstAcc& acc,
-                                               int64_t gwave, int64_t nwaves, bool coherent) {
+__device__ __forceinline__ void gb_merge_path(const GbArgs<OffT>& a, int64_t start, uint32_t len,
+                                              const GbOut<OffT>& o, gb::Acc& acc) {
   const int lane = lane_id();
-  for (int64_t base = gwave * 64; base < cnt; base += nwaves * 64) {
-    QEntry qe{0, 0, 0};
-    if (base + lane < cnt) {
-      qe = coherent ? load_entry_coherent(ents + base + lane) : ents[base + lane];
-      /* a list entry of an earlier level of the burst: its vertex joins prev
-       * (fire and forget; nothing in the burst reads prev) */
-      if (coherent) atomic_or(&a.prev[(uint32_t)qe.v >> 6], 1ull << (qe.v & 63));
-    }
-    const uint32_t incl = wave_inclusive_scan((uint32_t)qe.len);
-    const uint32_t total = wave_lane(incl, 63);
-    const uint32_t excl = incl - (uint32_t)qe.len;
-    for (uint32_t t0 = 0; t0 < total; t0 += 4 * 64) {
-      uint32_t y[4];
-      bool ok[4];
+  const uint32_t incl = wave_inclusive_scan(len);
+  const uint32_t total = wave_lane(incl, 63);
+  const uint32_t excl = incl - len;
+  for (uint32_t t0 = 0; t0 < total; t0 += 4 * 64) {
+    uint32_t y[4];
+    bool ok[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t t = t0 + 64 * k + lane;
-        const int owner = scan_owner(incl, t);
-        const uint32_t before = __shfl(excl, owner, 64);
-        const int64_t st = shfl_i64(qe.start, owner);
-        ok[k] = t < total;
-        y[k] = ok[k] ? (uint32_t)a.cols[st + (t - before)] : 0u;
-      }
-      gb_claim4(a, y, ok, level, out_small, out_pieces, sm, acc);
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t t = t0 + 64 * k + lane;
+      const int owner = scan_owner(incl, t);
+      const uint32_t before = __shfl(excl, owner, 64);
+      const int64_t st = shfl_i64(start, owner);
+      ok[k] = t < total;
+      y[k] = ok[k] ? (uint32_t)a.cols[st + (t - before)] : 0u;
     }
+    gb_claim<4>(a, y, ok, o, acc);
+  }
+}
+
+/* The workgroups' segments, gb::kGroup entries per wave and step; s_n[w]:
+ * entries of segment w, most: of the longest.  Where every list's heads are
+ * in its entry, each lane takes one arc: a wave's time is its instructions and
+ * divergent loads, a lookup per lane each, and one arc per lane spreads a
+ * small level's over four times the waves of four.  An entry's vertex joins
+ * prev last, so that nothing waits for that atomic before the level's end
+ * (nothing in the burst reads prev). */
+template<typename OffT>
+__device__ __forceinline__ void gb_visit_list(const GbArgs<OffT>& a, const uint64_t* in, const uint32_t* s_n,
+                                              uint32_t most, const GbOut<OffT>& o, gb::Acc& acc) {
+  const int lane = lane_id();
+  for (uint32_t k = threadIdx.x >> 6; k * gb::kGroup < most; k += gb::kWaves) {
+    const uint32_t w = gb::segment_of(k, o.rank, o.wgs);
+    if (k * gb::kGroup >= s_n[w]) continue;
+    const uint32_t i = k * gb::kGroup + (uint32_t)lane / gb::kInline;
+    const int64_t e = gb::entry_at(w, i, o.wgs);
+    const uint32_t sub = (uint32_t)lane % gb::kInline;
+    const bool has = i < s_n[w];
+    uint64_t e0 = 0;
+    uint32_t y[1] = {0};
+    if (has) {
+      e0 = atomic_load(in + e);
+      y[0] = atomic_load(reinterpret_cast<const uint32_t*>(in + 2 * a.total) + gb::kInline * e + sub);
+    }
+    const uint32_t len = (uint32_t)(e0 >> 32);
+    if (ballot(len > (uint32_t)gb::kInline)) {
+      int64_t start = 0; /* the entry's first lane lays its list */
+      if (has && sub == 0)
+        start = len > (uint32_t)gb::kInline ? (int64_t)atomic_load(in + a.total + e) : (int64_t)a.off[(uint32_t)e0];
+      gb_merge_path(a, start, sub == 0 ? len : 0u, o, acc);
+    } else {
+      const bool ok[1] = {sub < len};
+      gb_claim<1>(a, y, ok, o, acc);
+    }
+    if (has && sub == 0) atomic_or(&a.prev[(uint32_t)e0 >> 6], 1ull << (e0 & 63));
   }
 }
 
 /* long lists: a wave per entry (a piece, or a class 1 / class 2 queue entry),
  * 256 arcs per round */
 template<typename OffT>
-__device__ __forceinline__ void gb_visit_pieces(const GbArgs<OffT>& a, const QEntry* ents, int64_t cnt, int32_t level,
-                                                QEntry* out_small, QEntry* out_pieces, GbSums* sm, BurstAcc& acc,
-                                                int64_t gwave, int64_t nwaves, bool coherent) {
+__device__ __forceinline__ void gb_visit_pieces(const GbArgs<OffT>& a, const QEntry* ents, int64_t cnt,
+                                                const GbOut<OffT>& o, gb::Acc& acc, uint32_t gwave, uint32_t nwaves,
+                                                bool coherent) {
   const int lane = lane_id();
   for (int64_t i = gwave; i < cnt; i += nwaves) {
     const QEntry qe = coherent ? load_entry_coherent(ents + i) : ents[i];
-    if (coherent && lane == 0 && qe.start == (int64_t)a.off[qe.v]) /* the vertex's first piece */
-      atomic_or(&a.prev[(uint32_t)qe.v >> 6], 1ull << (qe.v & 63));
     for (int64_t o0 = 0; o0 < qe.len; o0 += 4 * 64) {
       uint32_t y[4];
       bool ok[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const int64_t o = o0 + 64 * k + lane;
-        ok[k] = o < qe.len;
-        y[k] = ok[k] ? (uint32_t)a.cols[qe.start + o] : 0u;
+        const int64_t j = o0 + 64 * k + lane;
+        ok[k] = j < qe.len;
+        y[k] = ok[k] ? (uint32_t)a.cols[qe.start + j] : 0u;
       }
-      gb_claim4(a, y, ok, level, out_small, out_pieces, sm, acc);
+      gb_claim<4>(a, y, ok, o, acc);
     }
+    if (coherent && lane == 0 && qe.start == (int64_t)a.off[qe.v]) /* the vertex's first piece */
+      atomic_or(&a.prev[(uint32_t)qe.v >> 6], 1ull << (qe.v & 63));
   }
 }
 
 template<typename OffT>
-__global__ void __launch_bounds__(kGbThreads) gburst_kernel(GbArgs<OffT> a, BfsCtl* ctl, DecideParams p, int32_t step,
+__global__ void __launch_bounds__(gb::kThreads) gburst_kernel(GbArgs<OffT> a, BfsCtl* ctl, DecideParams p, int32_t step,
                                                             LevelLog* levlog, StepLog* steplog) {
   __shared__ sg::policy::Staged s_pol;
-  __shared__ unsigned long long s_red[kGbWaves][3];
-  __shared__ unsigned long long s_tot[5];
+  __shared__ uint32_t s_n[kGbMaxWgs], s_most;
+  __shared__ gb::Local s_local;
+  __shared__ int32_t s_next; /* 0: another level, 1: none, 2: a wait ran out */
+  __shared__ int64_t s_pieces;
+  if (blockIdx.x % a.stride) return;
   if (ctl->done || ctl->skip || ctl->dir != 0 || ctl->f_edges > a.gb_arcs) return; /* the same for every workgroup */
+  const uint32_t rank = blockIdx.x / a.stride, wgs = gridDim.x / a.stride;
   stage_policy(p, &s_pol);
   const int lane = lane_id(), wv = threadIdx.x >> 6;
   /* the waves' ranks run across the workgroups first (rank = wave * grid +
    * workgroup): a level of a few thousand entries needs a few dozen waves,
    * and ranked within a workgroup first they all sat on the first few
    * compute units, queueing their memory requests there */
-  const int64_t gwave = (int64_t)(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-  const int64_t nwaves = ((int64_t)gridDim.x * kGbThreads) >> 6;
-  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-  int32_t level = ctl->level, lb = ctl->lb;
+  const uint32_t gwave = (uint32_t)wv * wgs + rank;
+  const uint32_t nwaves = wgs * gb::kWaves;
+  const bool lead = rank == 0 && threadIdx.x == 0;
+  const int32_t first_level = ctl->level, n_pull = ctl->n_pull;
+  /* followed by the first wave only */
+  int32_t lb = ctl->lb;
   int64_t f_vertices = ctl->f_vertices, f_edges = ctl->f_edges;
   unsigned long long vdeg = ctl->visited_deg, reached = ctl->reached;
-  int32_t n_push = ctl->n_push, done = 0, act = 0;
-  const int32_t n_pull = ctl->n_pull;
+  int32_t n_push = ctl->n_push, done = 0, act = 0, level = first_level;
   const QueueHdr h0 = *a.hdr;
-  uint32_t bt = 0;
-  int64_t n_small = 0, n_pieces = 0;
+  if (threadIdx.x == 0) s_local = gb::Local{0, 0, 0, 0, 0};
   __syncthreads();
   for (int it = 0;; ++it) {
     const int cur = it & 1;
-    GbSums* sm = a.sums + (it % 3);
-    if (lead) { /* the copy of the level after next: last read before the previous barrier */
-      unsigned long long* z = reinterpret_cast<unsigned long long*>(a.sums + ((it + 1) % 3));
-      for (int k = 0; k < 2; ++k) atomic_store(z + k, 0ull);
-    }
-    BurstAcc acc{0, 0, 0, 0, 0};
-    QEntry* out_small = a.small[cur ^ 1];
-    QEntry* out_pieces = a.pieces[cur ^ 1];
+    if (lead) /* the copy of the level after next: its pieces were last counted two levels ago */
+      atomic_store(&a.x.sums[(it + 1) % 3].npieces, 0ull);
+    gb::Acc acc{0, 0, 0, 0};
+    const GbOut<OffT> o{a.list[cur ^ 1], rank, wgs, a.pieces[cur ^ 1], a.x.sums + (it % 3), &s_local,
+                        first_level + it};
     if (it == 0) {
-      gb_visit_small(a, a.q[0], h0.count[0], level, out_small, out_pieces, sm, acc, gwave, nwaves, false);
-      gb_visit_pieces(a, a.q[1], h0.count[1], level, out_small, out_pieces, sm, acc, gwave, nwaves, false);
-      gb_visit_pieces(a, a.q[2], h0.count[2], level, out_small, out_pieces, sm, acc, gwave, nwaves, false);
+      for (int64_t base = (int64_t)gwave * 64; base < h0.count[0]; base += (int64_t)nwaves * 64) {
+        QEntry qe{0, 0, 0};
+        if (base + lane < h0.count[0]) qe = a.q[0][base + lane];
+        gb_merge_path(a, qe.start, (uint32_t)qe.len, o, acc);
+      }
+      gb_visit_pieces(a, a.q[1], h0.count[1], o, acc, gwave, nwaves, false);
+      gb_visit_pieces(a, a.q[2], h0.count[2], o, acc, gwave, nwaves, false);
     } else {
-      /* the previous level's discoveries join prev as their entries are read */
-      gb_visit_small(a, a.small[cur], n_small, level, out_small, out_pieces, sm, acc, gwave, nwaves, true);
-      gb_visit_pieces(a, a.pieces[cur], n_pieces, level, out_small, out_pieces, sm, acc, gwave, nwaves, true);
+      gb_visit_list(a, a.list[cur], s_n, s_most, o, acc);
+      gb_visit_pieces(a, a.pieces[cur], s_pieces, o, acc, gwave, nwaves, true);
     }
-    acc.disc = wave_sum_u64(acc.disc);
-    acc.deg = wave_sum_u64(acc.deg);
-    acc.mx = wave_max_u64(acc.mx);
-    if (lane == 0) {
-      s_red[wv][0] = acc.disc;
-      s_red[wv][1] = acc.deg;
-      s_red[wv][2] = acc.mx;
+    gb::add_local(&s_local, acc);
+    wait_stores_complete(); /* the lists: no fences, they are written and read coherently */
+    __syncthreads();
+    if (wv == 0) {
+      gb::Totals t{};
+      int32_t next = 2;
+      if (gb::exchange(a.x, &s_local, it, rank, wgs, s_n, t)) {
+        const unsigned long long unexplored = p.total_degree - (vdeg + t.deg);
+        act = decide_action(p, &s_pol, 0, t.disc, t.deg, unexplored, level + 1, t.mx);
+        done = t.disc == 0 ? 1 : 0;
+        const bool more = !done && act / 3 == 0 && (int64_t)t.deg <= a.gb_arcs && t.most <= a.seg_cap &&
+                          (int64_t)t.npieces <= a.cap_pieces;
+        if (more || done) { /* otherwise the count pass of this step counts and decides this level */
+          if (lead && level < SG_MAX_LEVELS_RECORDED) {
+            /* into device memory: a store to the host's would hold up this
+             * wave's next wait for its stores by a trip over the host link */
+            LevelLog e;
+            e.level = level;
+            e.dir = 0;
+            e.done = done;
+            e.next_dir = act / 3;
+            e.action = lb;
+            e.burst = 2;
+            e.f_vertices = f_vertices;
+            e.f_edges = f_edges;
+            e.disc = (int64_t)t.disc;
+            e.disc_deg = (int64_t)t.deg;
+            e.edges = f_edges;
+            e.scanned = f_vertices;
+            e.misses = 0;
+            e.max_deg = (int64_t)t.mx;
+            e.unexplored = (int64_t)unexplored;
+            a.log[level] = e;
+          }
+          vdeg += t.deg;
+          reached += t.disc;
+          ++n_push;
+          f_vertices = (int64_t)t.disc;
+          f_edges = (int64_t)t.deg;
+          lb = act % 3;
+          ++level;
+        }
+        next = more ? 0 : 1;
+      }
+      if (lane == 0) {
+        s_next = next;
+        s_most = t.most;
+        s_pieces = (int64_t)t.npieces;
+      }
     }
     __syncthreads();
-    GbSlot* slots = a.slots + (int64_t)(it & 1) * kGbMaxWgs;
-    if (threadIdx.x == 0) {
-      unsigned long long d = 0, g = 0, x = 0;
-      for (int w = 0; w < kGbWaves; ++w) {
-        d += s_red[w][0];
-        g += s_red[w][1];
-        x = s_red[w][2] > x ? s_red[w][2] : x;
-      }
-      atomic_store(&slots[blockIdx.x].disc, d);
-      atomic_store(&slots[blockIdx.x].deg, g);
-      atomic_store(&slots[blockIdx.x].mx, x);
-    }
-    /* no fences: the lists, sums and slots are written and read coherently */
-    if (!grid_barrier<false>(a.bar, bt, a.wait_ticks, 0u)) break; /* timed out: reported through the bar flags */
-    if (threadIdx.x < 64) { /* wave 0 totals the slots of every workgroup and reads the list sizes */
-      unsigned long long d = 0, g = 0, x = 0, lists = 0;
-      if (threadIdx.x < 2) lists = atomic_load(threadIdx.x == 0 ? &sm->nsmall : &sm->npieces);
-      for (uint32_t i = threadIdx.x; i < gridDim.x; i += 64) {
-        d += atomic_load(&slots[i].disc);
-        g += atomic_load(&slots[i].deg);
-        const unsigned long long y = atomic_load(&slots[i].mx);
-        x = y > x ? y : x;
-      }
-      d = wave_sum_u64(d);
-      g = wave_sum_u64(g);
-      x = wave_max_u64(x);
-      if (threadIdx.x == 0) {
-        s_tot[0] = d;
-        s_tot[1] = g;
-        s_tot[2] = x;
-        s_tot[3] = lists;
-      }
-      if (threadIdx.x == 1) s_tot[4] = lists;
-    }
-    __syncthreads();
-    const unsigned long long disc = s_tot[0], disc_deg = s_tot[1], max_deg = s_tot[2];
-    const int64_t ns = (int64_t)s_tot[3], np = (int64_t)s_tot[4];
-    const unsigned long long unexplored = p.total_degree - (vdeg + disc_deg);
-    act = decide_action(p, &s_pol, 0, disc, disc_deg, unexplored, level + 1, max_deg);
-    done = disc == 0 ? 1 : 0;
-    const bool more = !done && act / 3 == 0 && (int64_t)disc_deg <= a.gb_arcs && ns <= a.cap_small &&
-                      np <= a.cap_pieces;
-    if (!more && !done) break; /* the count pass of this step counts and decides this level */
-    if (lead && level < SG_MAX_LEVELS_RECORDED) {
-      LevelLog e;
-      e.level = level;
-      e.dir = 0;
-      e.done = done;
-      e.next_dir = act / 3;
-      e.action = lb;
-      e.burst = 2;
-      e.f_vertices = f_vertices;
-      e.f_edges = f_edges;
-      e.disc = (int64_t)disc;
-      e.disc_deg = (int64_t)disc_deg;
-      e.edges = f_edges;
-      e.scanned = f_vertices;
-      e.misses = 0;
-      e.max_deg = (int64_t)max_deg;
-      e.unexplored = (int64_t)unexplored;
-      levlog[level] = e;
-    }
-    vdeg += disc_deg;
-    reached += disc;
-    ++n_push;
-    f_vertices = (int64_t)disc;
-    f_edges = (int64_t)disc_deg;
-    lb = act % 3;
-    ++level;
-    n_small = ns;
-    n_pieces = np;
-    if (!more) break; /* done */
+    if (s_next) break;
   }
-  if (atomic_load(&a.bar->flags) & kBarTimeout) {
-    /* a barrier timed out: stop the traversal and report it in the step record */
+  if (s_next == 2) {
+    /* a wait ran out: stop the traversal and report it in the step record */
     if (threadIdx.x == 0) {
       ctl->done = 1;
       StepLog sl{};
@@ -1257,6 +1297,16 @@ __global__ void __launch_bounds__(kGbThreads) gburst_kernel(GbArgs<OffT> a, BfsC
       publish_step(&steplog[step % kRing], sl);
     }
     return;
+  }
+  if (rank != 0 || wv != 0) return;
+  { /* the level records, the first wave of the first workgroup */
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    const int32_t last = level < SG_MAX_LEVELS_RECORDED ? level : SG_MAX_LEVELS_RECORDED;
+    constexpr int kWords = (int)(sizeof(LevelLog) / 8);
+    const unsigned long long* from = reinterpret_cast<const unsigned long long*>(a.log);
+    unsigned long long* to = reinterpret_cast<unsigned long long*>(levlog);
+    for (int64_t i = (int64_t)first_level * kWords + lane; i < (int64_t)last * kWords; i += 64) to[i] = from[i];
+    __threadfence_system();
   }
   if (!lead) return;
   ctl->level = level;
@@ -1286,13 +1336,6 @@ __global__ void __launch_bounds__(kGbThreads) gburst_kernel(GbArgs<OffT> a, BfsC
   __threadfence_system();
 }
 
-__global__ void gb_reset_kernel(GridBar* bar, GbSums* sums) {
-  uint32_t* b = reinterpret_cast<uint32_t*>(bar);
-  for (int i = threadIdx.x; i < (int)(sizeof(GridBar) / 4); i += blockDim.x) b[i] = 0u;
-  unsigned long long* z = reinterpret_cast<unsigned long long*>(sums);
-  for (int i = threadIdx.x; i < (int)(3 * sizeof(GbSums) / 8); i += blockDim.x) z[i] = 0ull;
-}
-
 /* Per-graph BFS workspace, allocated on first use and reused. */
 struct BfsWorkspace {
   int64_t w0 = 0;
@@ -1306,10 +1349,11 @@ struct BfsWorkspace {
   uint32_t* arrive = nullptr; /* arrival counters of the count and write passes (kArriveWords each), zero between launches */
   /* grid bursts, allocated on first use for gb_arcs arcs */
   int64_t gb_arcs = 0;
-  GridBar* gb_bar = nullptr;
-  GbSums* gb_sums = nullptr;
-  GbSlot* gb_slots = nullptr;
-  QEntry* gb_small[2] = {nullptr, nullptr};
+  void* gb_base = nullptr; /* holds the following */
+  gb::Exchange gb_x{};
+  LevelLog* gb_log = nullptr;
+  int64_t gb_total = 0; /* list entries */
+  uint64_t* gb_list[2] = {nullptr, nullptr};
   QEntry* gb_pieces[2] = {nullptr, nullptr};
   LevelLog* levlog = nullptr; /* SG_MAX_LEVELS_RECORDED entries, pinned coherent host memory */
   StepLog* steplog = nullptr; /* kRing entries, pinned coherent host memory */
@@ -1329,13 +1373,7 @@ void ws_free(BfsWorkspace* w) {
   (void)hipFree(w->ctl);
   for (QEntry* l : w->burst_list) (void)hipFree(l);
   (void)hipFree(w->arrive);
-  (void)hipFree(w->gb_bar);
-  (void)hipFree(w->gb_sums);
-  (void)hipFree(w->gb_slots);
-  for (int k = 0; k < 2; ++k) {
-    (void)hipFree(w->gb_small[k]);
-    (void)hipFree(w->gb_pieces[k]);
-  }
+  (void)hipFree(w->gb_base);
   if (w->levlog) (void)hipHostFree(w->levlog);
   if (w->steplog) (void)hipHostFree(w->steplog);
   for (int r = 0; r < kRing; ++r)
@@ -1346,37 +1384,29 @@ void ws_free(BfsWorkspace* w) {
   delete w;
 }
 
-/* list capacities of a grid burst of at most gb_arcs frontier arcs: a level
- * discovers at most its frontier's arcs, and while the discoveries' arcs stay
- * within gb_arcs their pieces number at most gb_arcs / 256 + gb_arcs / 64
- * (a larger count ends the burst, whose lists are then not needed) */
-inline int64_t gb_cap_small(int64_t arcs) { return arcs + 64; }
-inline int64_t gb_cap_pieces(int64_t arcs) { return arcs / 32 + 64; }
-
-int gb_buffers(sg_graph_t g, BfsWorkspace* w, int64_t arcs) {
-  if (w->gb_arcs >= arcs) return SG_OK;
+int gb_buffers(sg_graph_t g, BfsWorkspace* w, int64_t arcs, int wgs) {
+  const int64_t total = gb::seg_cap(arcs, wgs) * wgs;
+  if (w->gb_arcs >= arcs && w->gb_total >= total) return SG_OK;
+  arcs = std::max(arcs, w->gb_arcs);
+  const int64_t entries = std::max(total, w->gb_total);
   sg_device_t dev = g->dev;
   SG_HIP(hipStreamSynchronize(dev->stream));
-  (void)hipFree(w->gb_bar);
-  (void)hipFree(w->gb_sums);
-  (void)hipFree(w->gb_slots);
-  for (int k = 0; k < 2; ++k) {
-    (void)hipFree(w->gb_small[k]);
-    (void)hipFree(w->gb_pieces[k]);
-    w->gb_small[k] = w->gb_pieces[k] = nullptr;
-  }
-  w->gb_bar = nullptr;
-  w->gb_sums = nullptr;
-  w->gb_slots = nullptr;
-  w->gb_arcs = 0;
-  SG_TRY(sg::alloc_device(dev, (void**)&w->gb_bar, sizeof(GridBar)));
-  SG_TRY(sg::alloc_device(dev, (void**)&w->gb_sums, 3 * sizeof(GbSums)));
-  SG_TRY(sg::alloc_device(dev, (void**)&w->gb_slots, 2 * kGbMaxWgs * sizeof(GbSlot)));
-  for (int k = 0; k < 2; ++k) {
-    SG_TRY(sg::alloc_device(dev, (void**)&w->gb_small[k], sizeof(QEntry) * gb_cap_small(arcs)));
-    SG_TRY(sg::alloc_device(dev, (void**)&w->gb_pieces[k], sizeof(QEntry) * gb_cap_pieces(arcs)));
-  }
+  (void)hipFree(w->gb_base);
+  w->gb_base = nullptr;
+  w->gb_arcs = w->gb_total = 0;
+  const size_t list = 4 * sizeof(uint64_t) * (size_t)entries, pieces = sizeof(QEntry) * (size_t)gb::cap_pieces(arcs);
+  SG_TRY(gb::alloc_parts(dev, &w->gb_base,
+                         {{(void**)&w->gb_x.sums, gb::kSumsBytes},
+                          {(void**)&w->gb_x.slots, gb::kSlotsBytes},
+                          {(void**)&w->gb_x.wide, gb::kWideBytes},
+                          {(void**)&w->gb_x.stop, gb::kStopBytes},
+                          {(void**)&w->gb_log, sizeof(LevelLog) * SG_MAX_LEVELS_RECORDED},
+                          {(void**)&w->gb_list[0], list},
+                          {(void**)&w->gb_list[1], list},
+                          {(void**)&w->gb_pieces[0], pieces},
+                          {(void**)&w->gb_pieces[1], pieces}}));
   w->gb_arcs = arcs;
+  w->gb_total = entries;
   return SG_OK;
 }
 
@@ -1487,18 +1517,18 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
   const int32_t lb_fixed = opt.load_balancer == SG_LB_WORKGROUP ? 1 : (opt.load_balancer == SG_LB_SUBGROUP ? 2 : 0);
   const int64_t burst_arcs = opt.burst_arcs < 0 ? 0 : (opt.burst_arcs == 0 ? kBurstDefaultArcs : opt.burst_arcs);
   const int64_t gb_arcs = opt.grid_burst_arcs < 0 ? 0 : (opt.grid_burst_arcs == 0 ? kGbDefaultArcs : opt.grid_burst_arcs);
-  int gb_grid = 0;
+  int gb_grid = 0, gb_stride = 1;
   if (gb_arcs > 0 && opt.policy != SG_POLICY_PULL) {
-    SG_TRY(gb_buffers(g, ws, gb_arcs));
     static int occ = 0; /* per offset width (one instantiation each) */
     if (occ == 0) {
       int nb = 0;
-      SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, gburst_kernel<OffT>, kGbThreads, 0));
+      SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, gburst_kernel<OffT>, gb::kThreads, 0));
       occ = std::max(1, nb);
     }
-    /* at most what is resident at once (the barrier needs every workgroup) */
-    gb_grid = std::min(opt.grid_burst_workgroups > 0 ? opt.grid_burst_workgroups : kGbDefaultWgs, dev->cus * occ);
-    gb_grid = std::min(gb_grid, kGbMaxWgs);
+    const gb::Plan gp = gb::plan(dev, occ, opt.grid_burst_workgroups);
+    gb_grid = gp.wgs;
+    gb_stride = gp.stride;
+    SG_TRY(gb_buffers(g, ws, gb_arcs, gb_grid));
   }
   bfs_start_kernel<OffT><<<sg::grid_for(dev, n, 256, 4), 256, 0, s>>>(
       a, ws->prev, g->isolated, reinterpret_cast<unsigned long long*>(ws->stats),
@@ -1557,26 +1587,28 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
       GbArgs<OffT> gba;
       gba.off = off;
       gba.cols = g->cols;
+      gba.m = g->m;
       gba.visited = ws->visited;
       gba.prev = ws->prev;
       gba.depth = depth;
       for (int k = 0; k < 3; ++k) gba.q[k] = Q.q[cur][k];
       gba.hdr = Q.hdr + cur;
       for (int k = 0; k < 2; ++k) {
-        gba.small[k] = ws->gb_small[k];
+        gba.list[k] = ws->gb_list[k];
         gba.pieces[k] = ws->gb_pieces[k];
       }
-      gba.cap_small = gb_cap_small(gb_arcs);
-      gba.cap_pieces = gb_cap_pieces(gb_arcs);
-      gba.sums = ws->gb_sums;
-      gba.slots = ws->gb_slots;
-      gba.bar = ws->gb_bar;
+      gba.seg_cap = (uint32_t)gb::seg_cap(gb_arcs, gb_grid);
+      gba.total = (int64_t)gba.seg_cap * gb_grid;
+      gba.log = ws->gb_log;
+      gba.cap_pieces = gb::cap_pieces(gb_arcs);
+      gba.x = ws->gb_x;
+      gba.x.wait_ticks = dev->wait_ticks;
       gba.gb_arcs = gb_arcs;
-      gba.wait_ticks = dev->wait_ticks;
-      gb_reset_kernel<<<1, 256, 0, s>>>(ws->gb_bar, ws->gb_sums);
+      gba.stride = (uint32_t)gb_stride;
+      gb::reset_kernel<<<1, 256, 0, s>>>(gba.x, gb_grid);
       int32_t stp = step;
       void* args[] = {&gba, &ws->ctl, &P, &stp, &ws->levlog, &ws->steplog};
-      SG_HIP(launch_resident(reinterpret_cast<const void*>(gburst_kernel<OffT>), gb_grid, kGbThreads, args, s));
+      SG_HIP(launch_resident(reinterpret_cast<const void*>(gburst_kernel<OffT>), gb_grid * gb_stride, gb::kThreads, args, s));
     }
     level_kernel<OffT><<<grid_level, kBlock, 0, s>>>(la, ws->ctl);
     if (timed) SG_HIP(hipEventRecord(ws->ev_mid[r], s));

@@ -50,6 +50,14 @@ struct alignas(32) TileCount {
  * write through to / read from the point of coherence that every XCD's L2
  * shares, so one workgroup can hand data to another within a launch without
  * an L2 write-back or invalidate. */
+/* The same hand-over through an atomic exchange whose result is dropped: it
+ * completes in the L2, where an agent-coherent store writes through to memory
+ * (88 against 480 ns for one, measured on an idle chip). */
+template<typename T>
+__device__ __forceinline__ void put_coherent(T* p, T v) {
+  (void)__hip_atomic_exchange(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 __device__ __forceinline__ void store_coherent(TileCount* p, const TileCount& t) {
   uint64_t w[4];
   __builtin_memcpy(w, &t, sizeof(w));
@@ -86,7 +94,8 @@ __device__ __forceinline__ void wait_stores_complete() {
  *    agent scope, an L2 write-back, so only threads with data for the last
  *    workgroup should), read with ordinary loads after the last workgroup's
  *    acquire (an L2 invalidate). */
-constexpr int kArriveGroups = 8;  /* workgroups are dealt to the 8 XCDs round robin */
+constexpr int kXcds = 8;           /* dies, each with its own L2; workgroups are dealt to them round robin */
+constexpr int kArriveGroups = kXcds;
 constexpr int kArriveStride = 16; /* counters 64 B apart */
 constexpr int kArriveWords = (kArriveGroups + 1) * kArriveStride;
 
@@ -172,6 +181,32 @@ __device__ __forceinline__ int scan_owner(uint32_t incl, uint32_t t) {
     else lo = mid + 1;
   }
   return (int)lo;
+}
+
+/* The arc range [s, e) of vertex v in one load (its two offsets are adjacent;
+ * global loads need only 4-byte alignment). */
+__device__ __forceinline__ void list_bounds(const int64_t* off, uint32_t v, int64_t& s, int64_t& e) {
+  int64_t x[2];
+  __builtin_memcpy(x, off + v, sizeof(x));
+  s = x[0];
+  e = x[1];
+}
+__device__ __forceinline__ void list_bounds(const uint32_t* off, uint32_t v, int64_t& s, int64_t& e) {
+  uint32_t x[2];
+  __builtin_memcpy(x, off + v, sizeof(x));
+  s = (int64_t)x[0];
+  e = (int64_t)x[1];
+}
+
+/* Four ids from position j in one load (only those below m are defined): a
+ * divergent wave pays per load and lane, not per byte. */
+__device__ __forceinline__ void load_ids4(const int32_t* cols, int64_t j, int64_t m, uint32_t (&y)[4]) {
+  if (j + 4 <= m) {
+    __builtin_memcpy(y, cols + j, sizeof(y));
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) y[k] = j + k < m ? (uint32_t)cols[j + k] : 0u;
+  }
 }
 
 __device__ __forceinline__ void zero_slots(StatSlot* s) {
@@ -264,7 +299,7 @@ __device__ __forceinline__ bool tile_walk_item(TileWalk& w, uint64_t mine, int64
   }
   const int k = __ffsll((unsigned long long)w.words) - 1; /* the step-th non-empty word */
   w.words &= w.words - 1;
-  const uint64_t word = wave_lane(mine, k);
+  const uint64_t word = wave_lane((uint64_t)mine, k);
   v = (tile * 64 + k) * 64 + lane;
   return (word >> lane) & 1ull;
 }
@@ -851,17 +886,6 @@ inline int compact_write_only(hipStream_t s, QueueSet& qs, int dst, const OffT* 
   return SG_OK;
 }
 
-/* ------------------------------------------------- grid barrier --- */
-/* Barrier over all workgroups of a cooperative launch (every workgroup
- * co-resident).  Arrival counters only grow -- barrier t completes at t
- * arrivals per member -- so nothing is reset between barriers; the block is
- * zeroed before each launch.  Workgroups are grouped by blockIdx % 8 (the
- * XCD they are dealt to): a group's last arrival bumps the top counter, whose
- * last arrival publishes generation t.  The wait is bounded: past wait_ticks
- * of the constant-rate clock kBarTimeout is raised and every workgroup
- * leaves.  Returns false when the launch must stop (a flag of stop_mask is
- * set); the caller's stores before the barrier are visible to every
- * workgroup after it (agent-scope release / acquire). */
 /* Launch a kernel whose workgroups meet at grid barriers.  The caller sizes
  * the grid from the kernel's occupancy so that every workgroup is resident at
  * once on the device.  The launch is cooperative where the runtime grants it
@@ -881,77 +905,6 @@ inline hipError_t launch_resident(const void* fn, int grid, int block, void** ar
     coop_refused.store(1, std::memory_order_relaxed);
   }
   return hipLaunchKernel(fn, dim3(grid), dim3(block), args, 0, s);
-}
-
-constexpr int kBarGroups = 8;
-constexpr int kBarStride = 32; /* counters 128 bytes apart */
-constexpr uint32_t kBarTimeout = 1u << 31;
-constexpr int kBarFlat = 64; /* grids up to this size use one arrival counter */
-
-struct GridBar {
-  uint32_t grp[kBarGroups * kBarStride];
-  uint32_t top[kBarStride];
-  uint32_t gen[kBarStride];
-  uint32_t flags;
-  uint32_t pad[31];
-};
-
-__device__ __forceinline__ void bar_raise(GridBar* b, uint32_t f) { atomic_or(&b->flags, f); }
-
-/* kFences: the caller exchanges data through ordinary loads and stores, so
- * the barrier releases (an L2 write-back of every workgroup's XCD) and
- * acquires (an L2 invalidate) at agent scope.  Without: everything the
- * workgroups exchange is written with agent-coherent stores and read with
- * agent-coherent loads (relaxed atomics at agent scope, which go to the
- * point of coherence every XCD shares), and each wave only waits for its own
- * stores to complete before its workgroup arrives -- no L2 is written back or
- * invalidated, which costs tens of microseconds per barrier once hundreds of
- * workgroups each do it. */
-template<bool kFences = true>
-__device__ __noinline__ bool grid_barrier(GridBar* c, uint32_t& t, uint64_t wait_ticks, uint32_t stop_mask) {
-  __shared__ uint32_t s_stop;
-  if (kFences) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-  else wait_stores_complete();
-  __syncthreads();
-  ++t;
-  if (threadIdx.x == 0) {
-    const uint32_t grid = gridDim.x, g = blockIdx.x % kBarGroups;
-    const uint32_t ngroups = grid < (uint32_t)kBarGroups ? grid : (uint32_t)kBarGroups;
-    const uint32_t in_group = (grid - g + kBarGroups - 1) / kBarGroups;
-    /* up to kBarFlat workgroups arrive on the top counter directly: one
-     * atomic round trip fewer, and few enough not to queue long on it */
-    const bool flat = grid <= (uint32_t)kBarFlat;
-    bool released = false;
-    if (flat || atomic_add(&c->grp[g * kBarStride], 1u) == t * in_group - 1) {
-      if (kFences) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      if (atomic_add(&c->top[0], 1u) == t * (flat ? grid : ngroups) - 1) {
-        if (kFences) {
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
-          __hip_atomic_store(&c->gen[0], t, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-          atomic_store(&c->gen[0], t);
-        }
-        released = true;
-      }
-    }
-    if (!released) {
-      const uint64_t t0 = wall_clock64();
-      while ((kFences ? __hip_atomic_load(&c->gen[0], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT)
-                      : atomic_load(&c->gen[0])) < t) {
-        if (atomic_load(&c->flags) & (stop_mask | kBarTimeout)) break;
-        if ((uint64_t)(wall_clock64() - t0) > wait_ticks) {
-          bar_raise(c, kBarTimeout);
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-      }
-    }
-    s_stop = (atomic_load(&c->flags) & (stop_mask | kBarTimeout)) ? 1u : 0u;
-  }
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __syncthreads();
-  if (kFences) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  return s_stop == 0;
 }
 
 /* A queue entry written with agent-coherent stores / read with

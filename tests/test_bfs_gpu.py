@@ -377,3 +377,50 @@ def test_bfs_many_rows_match_oracle(sg, device, oracle_mod, policy):
         with pytest.raises(sg.SygraphError):
             sg.bfs_many(G, [0, G.n], policy=pol)
         G.destroy()
+
+
+def _layers(seed, layers=300, width=50):
+    """A path of layers: every vertex has 0 to 70 arcs into the next layer, most of them at most four
+    (lists carried by their entries, walked from their start, and cut into pieces, side by side)."""
+    rng = np.random.default_rng(seed)
+    u, v = [], []
+    for k in range(layers - 1):
+        deg = np.where(rng.random(width) < 0.8, rng.integers(1, 4, width), rng.integers(0, 71, width))
+        u.append(np.repeat(np.arange(k * width, (k + 1) * width), deg))
+        v.append((k + 1) * width + rng.integers(0, width, int(deg.sum())))
+    return np.concatenate(u), np.concatenate(v), layers * width
+
+
+@pytest.mark.parametrize("workgroups", [1, 3, 32, 1024])
+@pytest.mark.parametrize("offset_bytes", [4, 8])
+@pytest.mark.parametrize("directed", [False, True])
+def test_grid_burst_workgroups_and_list_lengths(sg, device, oracle_mod, workgroups, offset_bytes, directed):
+    """Grid bursts of one workgroup, of a number that is no power of two, the
+    default and the largest, over lists of 0 to 70 (directed: 0 to 70 out-arcs)
+    and of many times that (a hub on a long path): the oracle's depths and the
+    level records of the levels run on their own."""
+    u, v, n = _layers(31 + offset_bytes)
+    hub = np.full(2500, n // 2)
+    u, v = np.concatenate([u, hub]), np.concatenate([v, np.arange(n, n + 2500)])
+    n += 2500
+    if directed:
+        key = np.unique(u * n + v)
+        off = np.zeros(n + 1, dtype=np.int64)
+        np.add.at(off, key // n + 1, 1)
+        g = oracle_mod.CSRGraph(n, np.cumsum(off), (key % n).astype(np.int32))
+    else:
+        g = oracle_mod.csr_from_pairs(n, u, v)
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, directed=directed, offset_bytes=offset_bytes)
+    src = int(np.nonzero(g.degrees()[:50] > 0)[0][0])
+    ref, levels = oracle_mod.bfs(g, src)
+    runs = []
+    for grid in (-1, 0, 2000):
+        b = sg.BFS(G)
+        b.init(src)
+        st = b.run(sg.POLICY_PUSH, tuning={"burst_arcs": -1, "grid_burst_arcs": grid,
+                                           "grid_burst_workgroups": workgroups}, record_levels=False)
+        assert np.array_equal(b.get_distances(), ref), grid
+        runs.append((st.levels, [(x.frontier_vertices, x.frontier_edges, x.discovered, x.unexplored_edges, x.max_degree)
+                                 for x in st.level[:st.levels]]))
+        assert (sum(x.burst == 2 for x in st.level[:st.levels]) > levels // 2) == (grid >= 0)
+    assert runs[0][0] == levels and runs[1] == runs[0] and runs[2] == runs[0]
