@@ -279,7 +279,8 @@ typedef struct sg_bfs_options {
                               one grid barrier per level, once two steps in a row have left such a
                               level (default 262144, at most 2^24; negative: never) */
   int32_t grid_burst_workgroups; /* 512-thread workgroups of that launch (default 32; at most 1024, and
-                                     never more than fit on the device at once) */
+                                     never more than fit on the device at once; rounded down to a
+                                     power of two) */
   int32_t learned_gate;    /* SG_POLICY_LEARNED: a level whose frontier has fewer arcs than the graph's
                               arcs / learned_gate pushes with the bucketing mapping without asking the
                               network (default 1024; negative: the network decides every level) */
@@ -384,7 +385,9 @@ typedef struct sg_sssp_options {
                             weight on a graph of at least 2^25 arcs and 8 arcs per vertex; none
                             otherwise: on smaller graphs an iteration's launches cost more than the
                             relaxations buckets save, on sparse long-diameter ones such as grids
-                            buckets multiply the iterations), negative or infinite =
+                            buckets multiply the iterations.  Below 2^25 arcs, rounds of at most 2^17
+                            arcs run back to back in one launch, where putting off the farther
+                            vertices pays: fewer relaxations, other rounds), negative or infinite =
                             none, i.e. every dirty vertex is relaxed each round (the reference's
                             frontier Bellman-Ford, sssp.hpp:152-210) */
   int32_t heavy_pull;    /* direction of a bucket's heavy round on an undirected graph: 0 = automatic

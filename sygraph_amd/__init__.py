@@ -616,11 +616,13 @@ class SSSP:
             burst_arcs: int = 0, record_relax: bool = False) -> SsspStats:
         """delta: bucket width of the near/far split (0 automatic: half the
         mean arc weight on a graph of at least 2^25 arcs and 8 arcs per
-        vertex, none otherwise; negative or inf for the
+        vertex, none otherwise, with the farther vertices put off where small
+        rounds run back to back, below 2^25 arcs; negative or inf for the
         reference's frontier Bellman-Ford).  heavy_pull: direction of a
         bucket's heavy round (0 automatic, 1 pull, -1 push).  burst_arcs:
         small rounds of the reference's schedule run inside one workgroup (0
-        default 4096, negative never).  record_relax: time each relax launch on its own
+        default 4096), larger ones of at most 2^17 arcs in one launch of
+        resident workgroups (negative: neither).  record_relax: time each relax launch on its own
         (stats.relax_ms, stats.relax_launches)."""
         if self.source is None:
             raise SygraphError(SG_ERR_STATE, "SSSP instance not initialized")

@@ -30,9 +30,11 @@
 #include <limits>
 #include <cstring>
 
+#include "gridburst.hpp"
 #include "traverse.hpp"
 
 using namespace sg::trav;
+namespace gb = sg::gb;
 
 namespace {
 
@@ -89,6 +91,7 @@ struct SsspCtl {
 
 struct alignas(64) RoundLog {
   int32_t iter, done, relax, rounds;
+  int32_t fail; /* a wait of a grid burst ran out */
   int64_t near_v, near_e;
   unsigned long long relaxed;
 };
@@ -502,6 +505,497 @@ __device__ __forceinline__ uint32_t next_threshold(uint32_t fmin_bits, double de
   return DistOps<W>::bits(tn);
 }
 
+/* ------------------------------------------------------- grid bursts --- */
+/* Rounds of the reference's schedule too large for one workgroup but too small
+ * to fill the chip -- a 1201 x 1301 grid has thousands of about ten thousand
+ * arcs, 42 us each as three launches -- run back to back in one launch of
+ * resident workgroups (gridburst.hpp), one exchange per round.  It starts
+ * from the queues the write pass of the same iteration wrote and stops when a
+ * round lowers nothing or the next one has more than grid_arcs arcs (or needs
+ * longer lists): what is left gets its dirty bits back and the next
+ * iteration's selection takes it from the bitmap.
+ *
+ * Every relaxation that lowers dist[v] appends v with the distance it gave, so
+ * nothing has to be deduplicated: a vertex lowered twice in a round is listed
+ * twice, but the entry with the larger distance lowers nothing that the other
+ * does not, so copies do not multiply.  An entry carries vertex and length,
+ * distance, and for lists of at most gb::kInline arcs heads and weights,
+ * loaded while the minimum is in flight: a round's chain is the entry, the
+ * head's distance and list bounds, the minimum with the head's own list, and
+ * the store of the next entry.
+ *
+ * Near and far (the automatic schedule only).  Relaxing every lowered vertex
+ * at once, the reference's order, relaxes an arc dozens of times on a grid.
+ * With a round at a few microseconds it pays to put off what lies beyond a
+ * threshold T (the near-far piles of Davidson, Baxter, Garland and Owens,
+ * IPDPS 2014): a vertex lowered to T or more goes to its workgroup's far list
+ * instead, and when a round leaves nothing near, T moves to the smallest far
+ * distance plus a step and a far pass takes what is below it, dropping what
+ * has been lowered since.  The step follows the rounds' sizes: doubled when a
+ * bucket's rounds had fewer than kNearFew arcs on average, which cost their
+ * latency whatever they hold, halved above kNearMany, where they take several
+ * turns of the waves (2,048 / 8,192: 14.8 ms on the grid below, 4,096 /
+ * 16,384: 14.0, 8,192 / 32,768: 14.7, 16,384 / 49,152: 27.3 with half the
+ * workgroups, where 4,096 / 16,384 took 16.6).
+ *
+ * 1201 x 1301 grid, u32 weights: 66.6 ms by launches and single-workgroup
+ * bursts (364 M relaxations, 42 us a launched round), 14.1 so (24 M, 5.2 us a
+ * round). */
+constexpr int kSsspGridWgs = 64; /* 32: 15.1 ms, 128: 15.2 */
+constexpr int64_t kSsspGridArcs = 1 << 17;
+constexpr int64_t kNearFew = 4096, kNearMany = 16384;
+/* far entries per workgroup: an even share of a quarter of the vertices; what
+ * does not fit waits for the burst's end */
+inline uint32_t far_capacity(int64_t n, int wgs) {
+  return (uint32_t)std::min<int64_t>(std::max<int64_t>(n / (4 * wgs), 1024), 1 << 18);
+}
+
+template<typename OffT, typename W>
+struct SsspGrid {
+  const OffT* off;
+  const int32_t* cols;
+  const W* w;
+  int64_t m;
+  uint32_t* dist;
+  uint64_t* dirty;
+  QEntry* q[3]; /* the round's queues */
+  const QueueHdr* hdr;
+  /* [parity]: `total` entries of two words (vertex | length << 32; first
+   * arc), then `total` distances, kInline heads and kInline weights per entry */
+  uint64_t* list[2];
+  int64_t total;
+  uint32_t seg_cap;
+  QEntry* pieces[2];
+  int64_t cap_pieces, grid_arcs;
+  uint64_t* far[2]; /* [parity]: far_cap entries per workgroup, vertex | distance << 32 */
+  uint32_t far_cap;
+  double step;      /* first step of T; 0: no far list */
+  double w_max;
+  gb::Exchange x;
+  unsigned long long* relax_slots;
+  RoundLog* log;
+  uint32_t stride; /* the burst's workgroups are those with blockIdx.x % stride == 0 */
+};
+constexpr int64_t kSsspGridWords(int64_t total) { return 2 * total + total / 2 + total / 2 * gb::kInline * 2; }
+
+template<typename OffT, typename W>
+struct SsspGridOut {
+  uint64_t* list;
+  uint32_t rank, wgs;
+  QEntry* pieces;
+  gb::Sums* sums;
+  gb::Local* local;
+  uint64_t* far; /* the workgroup's far list and its counter (LDS) */
+  uint32_t* far_n;
+  uint32_t T; /* bits of the threshold (no far list: above every distance) */
+};
+
+/* Append this lane's (v, d) to the workgroup's far list (all lanes call). */
+template<typename OffT, typename W>
+__device__ __forceinline__ void sssp_far_append(const SsspGrid<OffT, W>& a, const SsspGridOut<OffT, W>& o, bool is_far,
+                                                uint32_t v, uint32_t d) {
+  const uint64_t m = ballot(is_far);
+  if (!m) return;
+  uint32_t at = 0;
+  if (lane_id() == 0) at = atomicAdd(o.far_n, (uint32_t)__popcll(m));
+  at = __builtin_amdgcn_readfirstlane(at) + lanes_below(m);
+  if (!is_far) return;
+  if (at < a.far_cap) o.far[at] = (uint64_t)v | (uint64_t)d << 32;
+  else atomic_or(&a.dirty[v >> 6], 1ull << (v & 63)); /* no room: left to the rounds after the burst */
+}
+
+/* Append this lane's vertices with their lists (ms[k]: the lanes of the k-th
+ * whose lists are short; the caller holds the heads and weights of those of at
+ * most kInline arcs). */
+template<int K, typename OffT, typename W>
+__device__ __forceinline__ void sssp_grid_append(const SsspGrid<OffT, W>& a, const SsspGridOut<OffT, W>& o,
+                                                 const uint32_t (&y)[K], const uint32_t (&nb)[K], const bool (&low)[K],
+                                                 const int64_t (&vs)[K], const int64_t (&ve)[K],
+                                                 const uint32_t (&id)[K][gb::kInline],
+                                                 const uint32_t (&wt)[K][gb::kInline], gb::Acc& acc);
+
+/* Relax the (up to) K arcs of each lane: head y[k], distance nb[k] over it. */
+template<int K, typename OffT, typename W>
+__device__ __forceinline__ void sssp_grid_relax(const SsspGrid<OffT, W>& a, const uint32_t (&y)[K],
+                                                const uint32_t (&nb)[K], const bool (&ok)[K],
+                                                const SsspGridOut<OffT, W>& o, gb::Acc& acc) {
+  uint32_t d[K];
+  int64_t vs[K], ve[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    d[k] = 0;
+    vs[k] = ve[k] = 0;
+    if (ok[k]) {
+      d[k] = atomic_load(&a.dist[y[k]]);
+      list_bounds(a.off, y[k], vs[k], ve[k]);
+    }
+  }
+  uint32_t id[K][gb::kInline], wt[K][gb::kInline];
+  bool low[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    low[k] = ok[k] && nb[k] < d[k];
+    if (low[k]) d[k] = atomic_min(&a.dist[y[k]], nb[k]);
+    if (low[k] && nb[k] < o.T && ve[k] - vs[k] <= gb::kInline) {
+      load_ids4(a.cols, vs[k], a.m, id[k]);
+      load_ids4(reinterpret_cast<const int32_t*>(a.w), vs[k], a.m, wt[k]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    low[k] = low[k] && nb[k] < d[k] && ve[k] > vs[k]; /* a vertex without arcs has nothing to relax */
+    const bool is_far = low[k] && nb[k] >= o.T;
+    sssp_far_append(a, o, is_far, y[k], nb[k]);
+    low[k] = low[k] && !is_far;
+  }
+  sssp_grid_append<K>(a, o, y, nb, low, vs, ve, id, wt, acc);
+}
+
+template<int K, typename OffT, typename W>
+__device__ __forceinline__ void sssp_grid_append(const SsspGrid<OffT, W>& a, const SsspGridOut<OffT, W>& o,
+                                                 const uint32_t (&y)[K], const uint32_t (&nb)[K], const bool (&low)[K],
+                                                 const int64_t (&vs)[K], const int64_t (&ve)[K],
+                                                 const uint32_t (&id)[K][gb::kInline],
+                                                 const uint32_t (&wt)[K][gb::kInline], gb::Acc& acc) {
+  uint64_t ms[K];
+  uint32_t cs = 0;
+  bool pieces = false;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const bool big = ve[k] - vs[k] >= gb::kBig;
+    ms[k] = ballot(low[k] && !big);
+    cs += (uint32_t)__popcll(ms[k]);
+    pieces = pieces || (low[k] && big);
+  }
+  const bool any_pieces = ballot(pieces) != 0;
+  if (cs == 0 && !any_pieces) return;
+  uint32_t at = 0;
+  if (cs) {
+    if (lane_id() == 0) at = atomicAdd(&o.local->cnt, cs);
+    at = __builtin_amdgcn_readfirstlane(at);
+    acc.disc += cs;
+  }
+  uint32_t* dists = reinterpret_cast<uint32_t*>(o.list + 2 * a.total);
+  uint64_t* heads = o.list + 2 * a.total + a.total / 2;
+  uint64_t* wts = heads + a.total / 2 * gb::kInline;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    if (!ms[k]) continue;
+    const uint32_t len = (uint32_t)(ve[k] - vs[k]);
+    const bool mine = low[k] && len < (uint32_t)gb::kBig;
+    acc.deg += wave_sum_u32(mine ? len : 0u);
+    const uint32_t p = at + lanes_below(ms[k]);
+    if (mine && p < a.seg_cap) {
+      const int64_t i = gb::entry_at(o.rank, p, o.wgs);
+      put_coherent(o.list + i, (uint64_t)y[k] | (uint64_t)len << 32);
+      put_coherent(dists + i, nb[k]);
+      if (len <= (uint32_t)gb::kInline) {
+        put_coherent(heads + 2 * i, (uint64_t)id[k][0] | (uint64_t)id[k][1] << 32);
+        put_coherent(heads + 2 * i + 1, (uint64_t)id[k][2] | (uint64_t)id[k][3] << 32);
+        put_coherent(wts + 2 * i, (uint64_t)wt[k][0] | (uint64_t)wt[k][1] << 32);
+        put_coherent(wts + 2 * i + 1, (uint64_t)wt[k][2] | (uint64_t)wt[k][3] << 32);
+      } else {
+        put_coherent(o.list + a.total + i, (uint64_t)vs[k]);
+      }
+    } else if (mine) { /* no room: the burst ends with this round */
+      atomic_or(&a.dirty[y[k] >> 6], 1ull << (y[k] & 63));
+    }
+    at += (uint32_t)__popcll(ms[k]);
+  }
+  if (!any_pieces) return;
+  uint32_t np = 0, npc[K];
+  unsigned long long deg = 0;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int64_t len = ve[k] - vs[k];
+    npc[k] = (low[k] && len >= gb::kBig) ? (uint32_t)((len + gb::kPiece - 1) / gb::kPiece) : 0u;
+    np += npc[k];
+    if (npc[k]) deg += (unsigned long long)len;
+    acc.disc += (uint32_t)__popcll(ballot(npc[k] != 0));
+  }
+  const uint32_t ip = wave_inclusive_scan(np);
+  const uint32_t tp = wave_lane(ip, 63);
+  unsigned long long bp = 0;
+  if (lane_id() == 63) bp = atomic_add(&o.sums->npieces, (unsigned long long)tp);
+  bp = wave_lane((uint64_t)bp, 63) + (ip - np);
+  acc.deg += wave_sum_u64(deg);
+  acc.npieces = tp > gb::kPiecesClamp || acc.npieces + tp > gb::kPiecesClamp ? gb::kPiecesClamp : acc.npieces + tp;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int64_t len = ve[k] - vs[k];
+    for (uint32_t c = 0; c < npc[k]; ++c, ++bp) {
+      const int64_t from = (int64_t)c * gb::kPiece;
+      const int64_t l = len - from < gb::kPiece ? len - from : gb::kPiece;
+      if ((int64_t)bp < a.cap_pieces) store_entry_coherent(o.pieces + bp, QEntry{vs[k] + from, (int32_t)y[k], (int32_t)l});
+      else atomic_or(&a.dirty[y[k] >> 6], 1ull << (y[k] & 63));
+    }
+  }
+}
+
+/* 64 lists of a wave laid end to end (merge path), four arcs per lane per
+ * round; du: the distance of each lane's list */
+template<typename OffT, typename W>
+__device__ __forceinline__ void sssp_grid_merge(const SsspGrid<OffT, W>& a, int64_t start, uint32_t len, uint32_t du,
+                                                const SsspGridOut<OffT, W>& o, gb::Acc& acc) {
+  const int lane = lane_id();
+  const uint32_t incl = wave_inclusive_scan(len);
+  const uint32_t total = wave_lane(incl, 63);
+  const uint32_t excl = incl - len;
+  for (uint32_t t0 = 0; t0 < total; t0 += 4 * 64) {
+    uint32_t y[4], nb[4];
+    bool ok[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t t = t0 + 64 * k + lane;
+      const int owner = scan_owner(incl, t);
+      const uint32_t before = __shfl(excl, owner, 64);
+      const int64_t j = shfl_i64(start, owner) + (t - before);
+      const uint32_t d = __shfl(du, owner, 64);
+      ok[k] = t < total;
+      y[k] = ok[k] ? (uint32_t)a.cols[j] : 0u;
+      nb[k] = ok[k] ? DistOps<W>::bits(DistOps<W>::value(d) + a.w[j]) : 0u;
+    }
+    sssp_grid_relax<4>(a, y, nb, ok, o, acc);
+  }
+}
+
+/* pieces of long lists, a wave per entry */
+template<typename OffT, typename W>
+__device__ __forceinline__ void sssp_grid_pieces(const SsspGrid<OffT, W>& a, const QEntry* ents, int64_t cnt,
+                                                 const SsspGridOut<OffT, W>& o, gb::Acc& acc, uint32_t gwave,
+                                                 uint32_t nwaves, bool coherent) {
+  const int lane = lane_id();
+  for (int64_t i = gwave; i < cnt; i += nwaves) {
+    const QEntry qe = coherent ? load_entry_coherent(ents + i) : ents[i];
+    const W du = DistOps<W>::value(atomic_load(&a.dist[qe.v]));
+    for (int64_t o0 = 0; o0 < qe.len; o0 += 4 * 64) {
+      uint32_t y[4], nb[4];
+      bool ok[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int64_t j = o0 + 64 * k + lane;
+        ok[k] = j < qe.len;
+        y[k] = ok[k] ? (uint32_t)a.cols[qe.start + j] : 0u;
+        nb[k] = ok[k] ? DistOps<W>::bits(du + a.w[qe.start + j]) : 0u;
+      }
+      sssp_grid_relax<4>(a, y, nb, ok, o, acc);
+    }
+  }
+}
+
+template<typename OffT, typename W>
+__global__ void __launch_bounds__(gb::kThreads) sssp_grid_kernel(SsspGrid<OffT, W> a, SsspCtl* ctl, int32_t iter) {
+  __shared__ uint32_t s_n[gb::kMaxWgs], s_most;
+  __shared__ gb::Local s_local;
+  __shared__ int32_t s_next; /* 0: another round, 1: none, 2: a wait ran out, 3: a far pass */
+  __shared__ int64_t s_pieces;
+  __shared__ uint32_t s_far_n[2], s_far_top, s_T; /* far entries; complement of the smallest kept one's bits */
+  if (blockIdx.x % a.stride) return;
+  const QueueHdr h0 = *a.hdr;
+  /* the same for every workgroup */
+  if (ctl->done || !ctl->relax || ctl->pull || (int64_t)h0.deg > a.grid_arcs) return;
+  const uint32_t rank = blockIdx.x / a.stride, wgs = gridDim.x / a.stride;
+  const int lane = lane_id(), wv = threadIdx.x >> 6;
+  const uint32_t gwave = (uint32_t)wv * wgs + rank, nwaves = wgs * gb::kWaves; /* across the workgroups first */
+  const bool lead = rank == 0 && threadIdx.x == 0;
+  unsigned long long arcs = h0.deg, relaxed = 0; /* arcs of the round; of the rounds before it (first wave) */
+  int32_t rounds = 0;
+  const bool piles = a.step > 0.0;
+  double step = a.step;                               /* first wave, like what follows */
+  unsigned long long bucket_arcs = 0, bucket_rounds = 0;
+  bool far_pass = piles; /* every thread's; the first sorts the queues into the far lists (T = 0) */
+  int fp = 0;            /* the far list in use */
+  if (threadIdx.x == 0) {
+    s_local = gb::Local{0, 0, 0, 0, 0};
+    s_far_n[0] = s_far_n[1] = s_far_top = 0;
+    s_T = piles ? 0u : 0xFFFFFFFFu;
+  }
+  __syncthreads();
+  for (int it = 0;; ++it) {
+    const int cur = it & 1;
+    if (lead) /* the copy of the round after next: its pieces were last counted two rounds ago */
+      atomic_store(&a.x.sums[(it + 1) % 3].npieces, 0ull);
+    gb::Acc acc{0, 0, 0, 0};
+    const SsspGridOut<OffT, W> o{a.list[cur ^ 1], rank, wgs, a.pieces[cur ^ 1], a.x.sums + (it % 3), &s_local,
+                                   a.far[far_pass ? fp ^ 1 : fp] + (int64_t)rank * a.far_cap,
+                                   &s_far_n[far_pass ? fp ^ 1 : fp], s_T};
+    uint32_t far_top = 0;
+    if (it == 0 && piles) {
+      for (int q = 0; q < 3; ++q)
+        for (int64_t base = (int64_t)gwave * 64; base < h0.count[q]; base += (int64_t)nwaves * 64) {
+          QEntry qe{0, 0, 0};
+          uint32_t d = 0;
+          bool is_far = base + lane < h0.count[q];
+          if (is_far) {
+            qe = a.q[q][base + lane];
+            is_far = q < 2 || qe.start == (int64_t)a.off[qe.v]; /* a long list's first chunk stands for it */
+            d = atomic_load(&a.dist[qe.v]);
+          }
+          sssp_far_append(a, o, is_far, (uint32_t)qe.v, d);
+          if (is_far) far_top = ~d > far_top ? ~d : far_top;
+        }
+    } else if (far_pass) {
+      const uint64_t* mine = a.far[fp] + (int64_t)rank * a.far_cap;
+      const uint32_t cnt = s_far_n[fp] < a.far_cap ? s_far_n[fp] : a.far_cap;
+      for (uint32_t base = (uint32_t)wv * 64; base < cnt; base += gb::kThreads) {
+        uint32_t y[1] = {0}, nb[1] = {0}, id[1][gb::kInline], wt[1][gb::kInline];
+        int64_t vs[1] = {0}, ve[1] = {0};
+        bool low[1] = {base + lane < cnt};
+        bool is_far = false;
+        if (low[0]) {
+          const uint64_t e = mine[base + lane];
+          y[0] = (uint32_t)e;
+          nb[0] = (uint32_t)(e >> 32);
+          const uint32_t d = atomic_load(&a.dist[y[0]]);
+          list_bounds(a.off, y[0], vs[0], ve[0]);
+          is_far = d == nb[0] && nb[0] >= o.T; /* otherwise lowered since: it has another entry */
+          low[0] = d == nb[0] && !is_far;
+        }
+        if (low[0] && ve[0] - vs[0] <= gb::kInline) {
+          load_ids4(a.cols, vs[0], a.m, id[0]);
+          load_ids4(reinterpret_cast<const int32_t*>(a.w), vs[0], a.m, wt[0]);
+        }
+        sssp_far_append(a, o, is_far, y[0], nb[0]);
+        if (is_far) far_top = ~nb[0] > far_top ? ~nb[0] : far_top;
+        sssp_grid_append<1>(a, o, y, nb, low, vs, ve, id, wt, acc);
+      }
+    } else if (it == 0) {
+      for (int64_t base = (int64_t)gwave * 64; base < h0.count[0]; base += (int64_t)nwaves * 64) {
+        QEntry qe{0, 0, 0};
+        uint32_t du = 0;
+        if (base + lane < h0.count[0]) {
+          qe = a.q[0][base + lane];
+          du = atomic_load(&a.dist[qe.v]);
+        }
+        sssp_grid_merge(a, qe.start, (uint32_t)qe.len, du, o, acc);
+      }
+      sssp_grid_pieces(a, a.q[1], h0.count[1], o, acc, gwave, nwaves, false);
+      sssp_grid_pieces(a, a.q[2], h0.count[2], o, acc, gwave, nwaves, false);
+    } else {
+      const uint64_t* in = a.list[cur];
+      const uint32_t* dists = reinterpret_cast<const uint32_t*>(in + 2 * a.total);
+      const uint32_t* heads = reinterpret_cast<const uint32_t*>(in + 2 * a.total + a.total / 2);
+      const uint32_t* wts = heads + a.total * gb::kInline;
+      const uint32_t most = s_most;
+      for (uint32_t k = wv; k * gb::kGroup < most; k += gb::kWaves) {
+        const uint32_t w = gb::segment_of(k, rank, wgs);
+        if (k * gb::kGroup >= s_n[w]) continue;
+        const uint32_t i = k * gb::kGroup + (uint32_t)lane / gb::kInline;
+        const int64_t e = gb::entry_at(w, i, wgs);
+        const uint32_t sub = (uint32_t)lane % gb::kInline;
+        const bool has = i < s_n[w];
+        uint64_t e0 = 0;
+        uint32_t du = 0, wt = 0, y[1] = {0};
+        if (has) {
+          e0 = atomic_load(in + e);
+          du = atomic_load(dists + e);
+          y[0] = atomic_load(heads + gb::kInline * e + sub);
+          wt = atomic_load(wts + gb::kInline * e + sub);
+        }
+        const uint32_t len = (uint32_t)(e0 >> 32);
+        if (ballot(len > (uint32_t)gb::kInline)) {
+          int64_t start = 0; /* the entry's first lane lays its list */
+          if (has && sub == 0)
+            start = len > (uint32_t)gb::kInline ? (int64_t)atomic_load(in + a.total + e) : (int64_t)a.off[(uint32_t)e0];
+          sssp_grid_merge(a, start, sub == 0 ? len : 0u, du, o, acc);
+        } else {
+          const bool ok[1] = {sub < len};
+          const uint32_t nb[1] = {DistOps<W>::bits(DistOps<W>::value(du) + DistOps<W>::value(wt))};
+          sssp_grid_relax<1>(a, y, nb, ok, o, acc);
+        }
+      }
+      sssp_grid_pieces(a, a.pieces[cur], s_pieces, o, acc, gwave, nwaves, true);
+    }
+    gb::add_local(&s_local, acc);
+    if (far_pass) {
+      far_top = wave_max_u32(far_top);
+      if (lane == 0 && far_top) atomicMax(&s_far_top, far_top);
+    }
+    wait_stores_complete(); /* the lists: no fences, they are written and read coherently */
+    __syncthreads();
+    if (wv == 0) {
+      gb::Totals t{};
+      int32_t next = 2;
+      /* whether anything is far, and after a far pass the smallest of it */
+      const uint32_t kept = s_far_n[far_pass ? fp ^ 1 : fp];
+      const unsigned long long extra = !kept ? 0ull : far_pass ? 1ull << 32 | s_far_top : 1ull;
+      if (gb::exchange(a.x, &s_local, it, rank, wgs, s_n, t, extra)) {
+        if (!far_pass) {
+          relaxed += arcs;
+          bucket_arcs += arcs;
+          ++bucket_rounds;
+          ++rounds;
+        }
+        arcs = t.deg;
+        const bool fits = (int64_t)t.deg <= a.grid_arcs && t.most <= a.seg_cap && (int64_t)t.npieces <= a.cap_pieces;
+        next = t.disc > 0 ? (fits ? 0 : 1) : t.mx ? 3 : 1;
+        if (next == 3) { /* the bucket is done: on by a step, or where that found nothing from the smallest left */
+          if (bucket_rounds) {
+            if (bucket_arcs < (unsigned long long)kNearFew * bucket_rounds) step *= 2.0;
+            else if (bucket_arcs > (unsigned long long)kNearMany * bucket_rounds && step > a.step / 64) step *= 0.5;
+          }
+          bucket_arcs = bucket_rounds = 0;
+          const uint32_t T = next_threshold<W>(far_pass ? ~(uint32_t)t.mx : s_T, step, a.w_max);
+          if (lane == 0) s_T = T;
+        }
+      }
+      if (lane == 0) {
+        s_next = next;
+        s_most = t.most;
+        s_pieces = (int64_t)(t.npieces < (unsigned long long)a.cap_pieces ? t.npieces : (unsigned long long)a.cap_pieces);
+        if (far_pass) {
+          s_far_n[fp] = 0; /* read; the next far pass fills it */
+          s_far_top = 0;
+        }
+      }
+    }
+    __syncthreads();
+    if (far_pass) fp ^= 1;
+    far_pass = s_next == 3;
+    if (s_next == 0 || s_next == 3) continue;
+    if (s_next == 1) { /* what the last round lowered goes back to the dirty bitmap */
+      const uint64_t* left = a.list[cur ^ 1];
+      const uint32_t mine = s_n[rank] < a.seg_cap ? s_n[rank] : a.seg_cap;
+      for (uint32_t i = threadIdx.x; i < mine; i += gb::kThreads) {
+        const uint32_t v = (uint32_t)atomic_load(left + gb::entry_at(rank, i, wgs));
+        atomic_or(&a.dirty[v >> 6], 1ull << (v & 63));
+      }
+      const uint64_t* far = a.far[fp] + (int64_t)rank * a.far_cap;
+      const uint32_t nf = piles ? (s_far_n[fp] < a.far_cap ? s_far_n[fp] : a.far_cap) : 0u;
+      for (uint32_t i = threadIdx.x; i < nf; i += gb::kThreads) {
+        const uint32_t v = (uint32_t)far[i];
+        atomic_or(&a.dirty[v >> 6], 1ull << (v & 63));
+      }
+      for (int64_t i = (int64_t)rank * gb::kThreads + threadIdx.x; i < s_pieces; i += (int64_t)wgs * gb::kThreads) {
+        const uint32_t v = (uint32_t)load_entry_coherent(a.pieces[cur ^ 1] + i).v;
+        atomic_or(&a.dirty[v >> 6], 1ull << (v & 63));
+      }
+    }
+    break;
+  }
+  if (s_next == 2) { /* a wait ran out: the next iteration's record says so */
+    if (threadIdx.x == 0) {
+      ctl->done = 1;
+      RoundLog e{};
+      e.iter = -1;
+      e.done = 1;
+      e.fail = 1;
+      RoundLog* slot = &a.log[(iter + 1) % kRing];
+      *slot = e;
+      __threadfence_system();
+      __hip_atomic_store(&slot->iter, iter + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __threadfence_system();
+    }
+    return;
+  }
+  if (!lead) return;
+  /* the selection counted the first round; the relax launch has nothing left */
+  ctl->rounds += rounds > 1 ? rounds - 1 : 0;
+  ctl->relaxed += relaxed - h0.deg;
+  ctl->relax = 0;
+  atomic_add(&a.relax_slots[0], relaxed);
+}
+
 /* Where a selection launch keeps its scratch and writes its decision. */
 struct SelectArgs {
   uint64_t *dirty, *near_bm, *settled, *settled_all;
@@ -669,6 +1163,13 @@ struct SsspWorkspace {
   uint32_t* arrive = nullptr; /* arrival counters of the selection and write launches (kArriveWords each), zero
                                  between launches */
   QEntry* burst_list[2] = {nullptr, nullptr}; /* kSsspBurstMax entries each */
+  /* grid bursts, allocated on the first run of the reference's schedule */
+  void* grid_base = nullptr; /* holds the following */
+  gb::Exchange grid_x{};
+  uint64_t* grid_list[2] = {nullptr, nullptr};
+  QEntry* grid_pieces[2] = {nullptr, nullptr};
+  uint64_t* grid_far[2] = {nullptr, nullptr};
+  int grid_wgs = 0, grid_stride = 1;
   RoundLog* log = nullptr; /* kRing entries, pinned coherent host memory */
   hipEvent_t ev[kRing] = {};
   hipEvent_t ev_pre[kRing] = {}; /* before each iteration's relax launch (record_relax) */
@@ -689,6 +1190,7 @@ void sssp_ws_free(SsspWorkspace* w) {
   (void)hipFree(w->arrive);
   (void)hipFree(w->burst_list[0]);
   (void)hipFree(w->burst_list[1]);
+  (void)hipFree(w->grid_base);
   if (w->log) (void)hipHostFree(w->log);
   for (hipEvent_t e : w->ev)
     if (e) (void)hipEventDestroy(e);
@@ -741,6 +1243,30 @@ int sssp_workspace_for(sg_graph_t g, SsspWorkspace** out) {
   return SG_OK;
 }
 
+int sssp_grid_buffers(sg_graph_t g, SsspWorkspace* ws, int occ) {
+  if (ws->grid_wgs > 0) return SG_OK;
+  sg_device_t dev = g->dev;
+  const gb::Plan p = gb::plan(dev, occ, kSsspGridWgs);
+  const int64_t total = gb::seg_cap(kSsspGridArcs, p.wgs) * p.wgs;
+  const size_t list = sizeof(uint64_t) * (size_t)kSsspGridWords(total);
+  const size_t pieces = sizeof(QEntry) * (size_t)gb::cap_pieces(kSsspGridArcs);
+  const size_t far = sizeof(uint64_t) * (size_t)far_capacity(g->n, p.wgs) * p.wgs;
+  SG_TRY(gb::alloc_parts(dev, &ws->grid_base,
+                         {{(void**)&ws->grid_x.sums, gb::kSumsBytes},
+                          {(void**)&ws->grid_x.slots, gb::kSlotsBytes},
+                          {(void**)&ws->grid_x.wide, gb::kWideBytes},
+                          {(void**)&ws->grid_x.stop, gb::kStopBytes},
+                          {(void**)&ws->grid_list[0], list},
+                          {(void**)&ws->grid_list[1], list},
+                          {(void**)&ws->grid_pieces[0], pieces},
+                          {(void**)&ws->grid_pieces[1], pieces},
+                          {(void**)&ws->grid_far[0], far},
+                          {(void**)&ws->grid_far[1], far}}));
+  ws->grid_stride = p.stride;
+  ws->grid_wgs = p.wgs;
+  return SG_OK;
+}
+
 /* The light-first adjacency for bucket width dlt, built on first use and
  * kept with the graph until a run asks for another width. */
 template<typename OffT, typename W>
@@ -766,8 +1292,8 @@ int ensure_split(sg_graph_t g, W dlt) {
 }
 
 template<typename OffT, typename W>
-int run_sssp(sg_graph_t g, int32_t src, double delta, int32_t heavy_pull, int64_t burst_arcs, bool record_relax,
-             W* dist_out, sg_sssp_stats* stats) {
+int run_sssp(sg_graph_t g, int32_t src, double delta, double grid_step, int32_t heavy_pull, int64_t burst_arcs,
+             bool record_relax, W* dist_out, sg_sssp_stats* stats) {
   sg_device_t dev = g->dev;
   hipStream_t s = dev->stream;
   const int64_t n = g->n;
@@ -852,7 +1378,9 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, int32_t heavy_pull, int64_
   sa.w_max = w_max;
   sa.pull_mode = pull_mode;
   sa.bellman = bellman ? 1 : 0;
-  sa.burst_arcs = burst_arcs;
+  /* the grid bursts' near and far piles take the small rounds from the start */
+  const bool grid = bellman && burst_arcs > 0, piles = grid && grid_step > 0.0;
+  sa.burst_arcs = piles ? 0 : burst_arcs;
   SsspBurst<OffT, W> sb{};
   sb.off = off;
   sb.cols = g->cols;
@@ -870,9 +1398,50 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, int32_t heavy_pull, int64_
   /* one iteration, three launches: split + near-set count + decision (relax /
    * next bucket / stop); queue write; relax.  Everything the host needs is in
    * the iteration's record. */
-  auto enqueue = [&](int32_t it) -> int {
+  SsspGrid<OffT, W> sg_args{};
+  if (grid) {
+    static int occ = 0; /* per instantiation */
+    if (occ == 0) {
+      int nb = 0;
+      SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, sssp_grid_kernel<OffT, W>, gb::kThreads, 0));
+      occ = std::max(1, nb);
+    }
+    SG_TRY(sssp_grid_buffers(g, ws, occ));
+    sg_args.off = off;
+    sg_args.cols = g->cols;
+    sg_args.w = (const W*)g->weights;
+    sg_args.m = g->m;
+    sg_args.dist = dist;
+    sg_args.dirty = dirty;
+    for (int k = 0; k < 3; ++k) sg_args.q[k] = Q.q[0][k];
+    sg_args.hdr = Q.hdr;
+    sg_args.seg_cap = (uint32_t)gb::seg_cap(kSsspGridArcs, ws->grid_wgs);
+    sg_args.total = (int64_t)sg_args.seg_cap * ws->grid_wgs;
+    for (int k = 0; k < 2; ++k) {
+      sg_args.list[k] = ws->grid_list[k];
+      sg_args.pieces[k] = ws->grid_pieces[k];
+      sg_args.far[k] = ws->grid_far[k];
+    }
+    sg_args.cap_pieces = gb::cap_pieces(kSsspGridArcs);
+    sg_args.grid_arcs = kSsspGridArcs;
+    sg_args.step = grid_step;
+    sg_args.far_cap = far_capacity(n, ws->grid_wgs);
+    sg_args.w_max = w_max;
+    sg_args.x = ws->grid_x;
+    sg_args.x.wait_ticks = dev->wait_ticks;
+    sg_args.relax_slots = ws->relax_slots;
+    sg_args.log = ws->log;
+    sg_args.stride = (uint32_t)ws->grid_stride;
+  }
+  auto enqueue = [&](int32_t it, bool burst) -> int {
     sssp_select_kernel<OffT, W><<<Q.grid_tiles(), kBlock, 0, s>>>(ca, sa, ws->ctl, it);
     near_write_kernel<OffT, W><<<Q.grid_tiles(), kBlock, 0, s>>>(ca, sb, ws->ctl);
+    if (burst) { /* a grid burst ahead of the relax launch (returns at once unless the round qualifies) */
+      gb::reset_kernel<<<1, 256, 0, s>>>(sg_args.x, ws->grid_wgs);
+      void* args[] = {&sg_args, &ws->ctl, &it};
+      SG_HIP(launch_resident(reinterpret_cast<const void*>(sssp_grid_kernel<OffT, W>), ws->grid_wgs * ws->grid_stride,
+                             gb::kThreads, args, s));
+    }
     if (record_relax) SG_HIP(hipEventRecord(ws->ev_pre[it % kRing], s));
     relax_kernel<OffT, W><<<grid_main, kBlock, 0, s>>>(a, ws->ctl, ws->relax_slots);
     SG_HIP(hipGetLastError());
@@ -882,9 +1451,12 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, int32_t heavy_pull, int64_
     return SG_OK;
   };
   for (int k = 0; k < kRing; ++k) __atomic_store_n(&ws->log[k].iter, -1, __ATOMIC_RELEASE);
-  SG_TRY(enqueue(0));
-  SG_TRY(enqueue(1));
+  SG_TRY(enqueue(0, piles));
+  SG_TRY(enqueue(1, false));
   int32_t round = 0;
+  /* iterations in a row whose round is small enough for a grid burst; from
+   * two on, the iterations enqueued carry one */
+  int32_t small_rounds = 0;
   int64_t relaxed = 0;
   float relax_ms = 0.f;
   int32_t relax_launches = 0;
@@ -898,6 +1470,11 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, int32_t heavy_pull, int64_
       SG_HIP(hipStreamSynchronize(s));
       sg::set_error("sg_sssp: iteration record %d out of order (found %d)", it, e.iter);
       return SG_ERR_STATE;
+    }
+    if (e.fail) {
+      SG_HIP(hipStreamSynchronize(s));
+      sg::set_error("sg_sssp: a grid burst waited longer than the device's wait limit (iteration %d)", it);
+      return SG_ERR_HIP;
     }
     if (e.relax && stats && e.rounds - 1 < SG_MAX_LEVELS_RECORDED) {
       stats->round_vertices[e.rounds - 1] = e.near_v;
@@ -917,7 +1494,8 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, int32_t heavy_pull, int64_
       sg::set_error("sg_sssp: no termination after %lld iterations", (long long)it);
       return SG_ERR_STATE;
     }
-    SG_TRY(enqueue(it + 2));
+    small_rounds = (grid && e.relax && e.near_e <= kSsspGridArcs) ? small_rounds + 1 : 0;
+    SG_TRY(enqueue(it + 2, small_rounds >= 2));
   }
   if (stats) {
     SG_HIP(hipEventRecord(e1, s));
@@ -993,21 +1571,29 @@ int mean_weight(sg_graph_t g, double* out) {
  * 100 generated graphs (RMAT scale 16-22, grids 512^2-4096^2, ER; weights
  * U[1,255]; four sources each) among arc counts 2^18..2^28 and degrees 0..32:
  * 3.4 % over choosing per run (18 % for the reference's schedule everywhere),
- * total time 1.8 % under the reference's schedule everywhere. */
+ * total time 1.8 % under the reference's schedule everywhere.
+ * Below kAutoBucketArcs the grid bursts keep near and far piles (1201 x 1301
+ * grid: 14 ms with them, 66 without; 300 x 400: 4.1 and 22; 200,000 vertices
+ * of 16 arcs: 1.68 and 2.07).  Sparse graphs above it keep the reference's
+ * order of relaxations: their counts of rounds and relaxations are part of
+ * what the automatic schedule is known to report there. */
 constexpr int64_t kAutoBucketArcs = int64_t(1) << 25;
 constexpr int64_t kAutoBucketDegree = 8;
 
 template<typename OffT, typename W>
 int run_sssp_auto(sg_graph_t g, int32_t source, double delta, int32_t heavy_pull, int64_t burst_arcs,
                   bool record_relax, W* dist, sg_sssp_stats* stats) {
-  if (delta == 0.0 && (g->m < kAutoBucketArcs || g->m < kAutoBucketDegree * (int64_t)g->n)) {
-    delta = -1.0;
-  } else if (delta == 0.0) {
+  double grid_step = 0.0;
+  if (delta == 0.0) {
     double mw = 1.0;
     SG_TRY(mean_weight<W>(g, &mw));
     delta = std::max(kAutoDeltaFactor * mw, DistOps<W>::is_float ? 1e-30 : 1.0);
+    if (g->m < kAutoBucketArcs || g->m < kAutoBucketDegree * (int64_t)g->n) {
+      if (g->m < kAutoBucketArcs) grid_step = 4.0 * delta; /* first step of the grid bursts' threshold */
+      delta = -1.0;
+    }
   }
-  return run_sssp<OffT, W>(g, source, delta, heavy_pull, burst_arcs, record_relax, dist, stats);
+  return run_sssp<OffT, W>(g, source, delta, grid_step, heavy_pull, burst_arcs, record_relax, dist, stats);
 }
 
 extern "C" {

@@ -500,3 +500,47 @@ def test_cc_asymmetric_csr_without_directed_flag(sg, device, oracle_mod):
     c.init()
     c.run()
     assert np.array_equal(c.get_labels(), oracle_mod.cc(g))
+
+
+@pytest.mark.parametrize("offset_bytes", [4, 8])
+@pytest.mark.parametrize("kind", ["grid", "layers", "directed"])
+@pytest.mark.parametrize("weight_float", [False, True])
+def test_sssp_grid_bursts(sg, device, oracle_mod, offset_bytes, kind, weight_float):
+    """Rounds of the reference's schedule between a workgroup's burst and 2^17 arcs run back to back in
+    one launch: lists carried by their entries, walked from their start and cut into pieces give the
+    distances of the launched rounds, bit for bit."""
+    rng = np.random.default_rng(40 + offset_bytes)
+    if kind == "grid":
+        g = oracle_mod.grid(260, 300, 0.05, seed=8)
+    else:
+        layers, width = 60, 900
+        u, v = [], []
+        for k in range(layers - 1):
+            deg = np.where(rng.random(width) < 0.8, rng.integers(1, 4, width), rng.integers(0, 90, width))
+            u.append(np.repeat(np.arange(k * width, (k + 1) * width), deg))
+            v.append((k + 1) * width + rng.integers(0, width, int(deg.sum())))
+        u, v, n = np.concatenate(u), np.concatenate(v), layers * width
+        u, v = np.concatenate([u, np.full(800, n // 2)]), np.concatenate([v, rng.integers(0, n, 800)])
+        if kind == "layers":
+            g = oracle_mod.csr_from_pairs(n, u, v)
+        else:
+            key = np.unique(u.astype(np.int64) * n + v)
+            off = np.zeros(n + 1, dtype=np.int64)
+            np.add.at(off, key // n + 1, 1)
+            g = oracle_mod.CSRGraph(n, np.cumsum(off), (key % n).astype(np.int32))
+    w = rng.integers(1, 256, len(g.cols)).astype(np.uint32)
+    if kind != "directed":
+        w = oracle_mod.fill_weights(g, 3)
+    if weight_float:
+        w = (w / 7.0).astype(np.float32)
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, weights=w, weight_float=weight_float,
+                          directed=kind == "directed", offset_bytes=offset_bytes)
+    src = int(np.nonzero(g.degrees() > 0)[0][0])
+    got = []
+    for burst in (-1, 0, 64):
+        s = sg.SSSP(G)
+        s.init(src)
+        s.run(delta=-1.0, burst_arcs=burst)
+        got.append(s.get_distances())
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    assert np.array_equal(got[0].view(np.uint32), got[2].view(np.uint32))
