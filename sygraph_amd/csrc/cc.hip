@@ -10,8 +10,10 @@
  *    (the largest vertex can never be hooked under a larger root).  Work is
  *    O(m) regardless of the graph's diameter, and most arcs are skipped by
  *    sampling (the Afforest scheme of Sutton, Ben-Nun and Barak, IPDPS 2018):
- *    every vertex first links its first kSampleArcs arcs; after a flatten the
- *    most frequent root among a fixed sample of vertices is taken as the
+ *    every vertex first takes the larger end of its list as its parent if that
+ *    is larger than itself (no atomics: everybody writes their own slot), the
+ *    chains this makes are cut short, and then every vertex links its first
+ *    kSampleArcs arcs; after a flatten the most frequent root among a fixed sample of vertices is taken as the
  *    giant component; then only vertices outside it link their remaining
  *    arcs (an arc into the giant component is seen from its other end, since
  *    both directions are stored), and a last flatten points every vertex at
@@ -68,12 +70,66 @@ __global__ void __launch_bounds__(kBlock) hook_kernel(QEntry* q0, QEntry* q1, QE
 constexpr int kSampleArcs = 2;
 constexpr int kRootSamples = 1024;
 
-/* every vertex links its first kSampleArcs arcs */
+/* parent[u] = the larger of u and the heads at its list's ends.  Lists are
+ * usually sorted, and then that is u's largest neighbour, so most vertices of
+ * a component with hubs end in one tree.  Linking a fresh forest by hooks
+ * instead, every vertex its first arcs, spent 4.5 of RMAT scale 20's 4.7 ms
+ * on threads that chase and hook the same few roots. */
 template<typename OffT>
-__global__ void sample_link_kernel(const OffT* off, const int32_t* cols, int64_t n, uint32_t* parent) {
-  for (int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; u < n; u += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t b = (int64_t)off[u], e = (int64_t)off[u + 1];
-    for (int64_t j = b; j < e && j < b + kSampleArcs; ++j) hook(parent, (uint32_t)u, (uint32_t)cols[j]);
+__global__ void __launch_bounds__(kBlock) first_parent_kernel(const OffT* off, const int32_t* cols, int64_t n,
+                                                              uint32_t* parent) {
+  for (int64_t u = blockIdx.x * (int64_t)kBlock + threadIdx.x; u < n; u += (int64_t)gridDim.x * kBlock) {
+    int64_t b, e;
+    list_bounds(off, (uint32_t)u, b, e);
+    uint32_t p = (uint32_t)u;
+    if (b < e) {
+      const uint32_t x = (uint32_t)cols[b], y = (uint32_t)cols[e - 1];
+      p = x > p ? x : p;
+      p = y > p ? y : p;
+    }
+    parent[u] = p;
+  }
+}
+
+/* Every vertex's parent moves up to kShortenHops ancestors up: a chain's
+ * length divides by more than that each pass (a 4096 x 4096 grid's chains are
+ * its columns, three passes). */
+constexpr int kShortenHops = 16, kShortenPasses = 3;
+__global__ void __launch_bounds__(kBlock) shorten_kernel(uint32_t* parent, int64_t n) {
+  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
+    const uint32_t first = atomic_load(&parent[i]);
+    uint32_t x = first;
+    for (int h = 0; h < kShortenHops; ++h) {
+      const uint32_t p = atomic_load(&parent[x]);
+      if (p == x) break;
+      x = p;
+    }
+    if (x != first) atomic_store(&parent[i], x);
+  }
+}
+
+/* Every stride-th vertex links its first kSampleArcs arcs; equal parents need
+ * no look at the root (an older parent is an ancestor too, so a cached one
+ * will do).  Run over a 64th of the vertices first: the arcs between two large
+ * trees are a good part of the graph's, and while the trees are apart every
+ * one of them chases and tries to hook the same root (2.7 ms on RMAT scale 20
+ * in one go).  Once a sample has joined them the rest finds equal parents. */
+constexpr int kFirstStride = 64;
+template<typename OffT>
+__global__ void __launch_bounds__(kBlock) sample_link_kernel(const OffT* off, const int32_t* cols, int64_t n,
+                                                             uint32_t* parent, int stride) {
+  for (int64_t u = (blockIdx.x * (int64_t)kBlock + threadIdx.x) * stride; u < n; u += (int64_t)gridDim.x * kBlock * stride) {
+    int64_t b, e;
+    list_bounds(off, (uint32_t)u, b, e);
+    const uint32_t pu = parent[u];
+    uint32_t v[kSampleArcs], pv[kSampleArcs];
+#pragma unroll
+    for (int k = 0; k < kSampleArcs; ++k) v[k] = b + k < e ? (uint32_t)cols[b + k] : (uint32_t)u;
+#pragma unroll
+    for (int k = 0; k < kSampleArcs; ++k) pv[k] = parent[v[k]];
+#pragma unroll
+    for (int k = 0; k < kSampleArcs; ++k)
+      if (pv[k] != pu) hook(parent, (uint32_t)u, v[k]);
   }
 }
 
@@ -214,6 +270,18 @@ __global__ void __launch_bounds__(kBlock) maxprop_kernel(QEntry* q0, QEntry* q1,
   });
 }
 
+/* The forest of an undirected graph's sampled arcs (not flattened). */
+template<typename OffT>
+void sample_forest(sg_device_t dev, hipStream_t s, const OffT* off, const int32_t* cols, int64_t n, uint32_t* parent) {
+  const int grid = sg::grid_for(dev, n, kBlock, 8);
+  first_parent_kernel<OffT><<<grid, kBlock, 0, s>>>(off, cols, n, parent);
+  for (int k = 0; k < kShortenPasses; ++k) shorten_kernel<<<grid, kBlock, 0, s>>>(parent, n);
+  sample_link_kernel<OffT><<<sg::grid_for(dev, n / kFirstStride + 1, kBlock, 8), kBlock, 0, s>>>(off, cols, n, parent,
+                                                                                               kFirstStride);
+  shorten_kernel<<<grid, kBlock, 0, s>>>(parent, n);
+  sample_link_kernel<OffT><<<grid, kBlock, 0, s>>>(off, cols, n, parent, 1);
+}
+
 template<typename OffT>
 int run_cc(sg_graph_t g, uint32_t* labels, int32_t* rounds_out) {
   sg_device_t dev = g->dev;
@@ -234,12 +302,10 @@ int run_cc(sg_graph_t g, uint32_t* labels, int32_t* rounds_out) {
   int32_t rounds = 0;
   bool sym = false;
   if (!(g->flags & SG_GRAPH_DIRECTED)) SG_TRY(graph_symmetric<OffT>(g, reinterpret_cast<unsigned long long*>(roots), &sym));
-  iota_kernel<<<sg::grid_for(dev, n, 256, 4), 256, 0, s>>>(labels, n);
-  fill_words_kernel<<<sg::grid_for(dev, w0, 256, 4), 256, 0, s>>>(bm[0], w0, n);
   if (sym) {
-    const int grid_n = sg::grid_for(dev, n, 256, 4);
-    sample_link_kernel<OffT><<<grid_n, 256, 0, s>>>(off, g->cols, n, labels);
-    flatten_kernel<<<grid_n, 256, 0, s>>>(labels, n);
+    const int grid_n = sg::grid_for(dev, n, kBlock, 8);
+    sample_forest<OffT>(dev, s, off, g->cols, n, labels);
+    flatten_kernel<<<grid_n, kBlock, 0, s>>>(labels, n);
     /* the giant component: the most frequent root of a fixed vertex sample */
     std::vector<uint32_t> h(kRootSamples);
     if (n > 0) {
@@ -263,10 +329,12 @@ int run_cc(sg_graph_t g, uint32_t* labels, int32_t* rounds_out) {
     st = compact_to_queues<OffT, kFromBitmap>(s, Q, 0, off, nullptr, nullptr, bm[0], tune, false, kSampleArcs);
     if (st == SG_OK) {
       hook_kernel<OffT><<<grid, kBlock, 0, s>>>(Q.q[0][0], Q.q[0][1], Q.q[0][2], Q.hdr, g->cols, labels);
-      flatten_kernel<<<grid_n, 256, 0, s>>>(labels, n);
+      flatten_kernel<<<grid_n, kBlock, 0, s>>>(labels, n);
       rounds = 1;
     }
   } else {
+    iota_kernel<<<sg::grid_for(dev, n, 256, 4), 256, 0, s>>>(labels, n);
+    fill_words_kernel<<<sg::grid_for(dev, w0, 256, 4), 256, 0, s>>>(bm[0], w0, n);
     /* every vertex starts active (the all-vertex pass of cc.hpp:135-145) */
     QueueHdr* hh = (QueueHdr*)dev->host_scratch;
     int cur = 0, qs = 0;
@@ -451,9 +519,8 @@ int run_cc_noalloc(sg_graph_t g, uint32_t* labels, int32_t* rounds_out) {
   int32_t rounds = 0;
   bool sym = false;
   if (!(g->flags & SG_GRAPH_DIRECTED)) SG_TRY(graph_symmetric<OffT>(g, ctr, &sym));
-  iota_kernel<<<grid_n, 256, 0, s>>>(labels, n);
   if (sym) {
-    sample_link_kernel<OffT><<<grid_n, 256, 0, s>>>(off, g->cols, n, labels);
+    sample_forest<OffT>(dev, s, off, g->cols, n, labels);
     flatten_kernel<<<grid_n, 256, 0, s>>>(labels, n);
     sample_roots_kernel<<<kRootSamples / 256, 256, 0, s>>>(labels, n, roots);
     giant_kernel<<<1, kRootSamples, 0, s>>>(roots, giant);
@@ -465,6 +532,7 @@ int run_cc_noalloc(sg_graph_t g, uint32_t* labels, int32_t* rounds_out) {
   } else {
     /* every vertex starts active (the all-vertex pass of cc.hpp:135-145) */
     auto* host = static_cast<unsigned long long*>(dev->host_scratch);
+    iota_kernel<<<grid_n, 256, 0, s>>>(labels, n);
     fill_words_kernel<<<sg::grid_for(dev, w0, 256, 4), 256, 0, s>>>(bmA, w0, n);
     zero_words_kernel<<<sg::grid_for(dev, w0, 256, 4), 256, 0, s>>>(bmB, w0);
     zero_words_kernel<<<1, 64, 0, s>>>(reinterpret_cast<uint64_t*>(ctr), 2);

@@ -544,3 +544,31 @@ def test_sssp_grid_bursts(sg, device, oracle_mod, offset_bytes, kind, weight_flo
         got.append(s.get_distances())
     assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
     assert np.array_equal(got[0].view(np.uint32), got[2].view(np.uint32))
+
+
+@pytest.mark.parametrize("graph", ["columns", "random", "two_grids"])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_cc_first_parents_and_chains(sg, device, oracle_mod, graph, noalloc):
+    """Forests whose first parents form chains longer than the passes that shorten them reach (one
+    column of 9,000 vertices), none at all, and several components of the same size; unsorted lists."""
+    import ctypes as C
+    if graph == "columns":
+        g = oracle_mod.grid(9000, 3, 0.0)
+    elif graph == "random":
+        g = oracle_mod.erdos_renyi(30000, 25000, seed=9)
+    else:
+        g = oracle_mod.grid(400, 300, 0.35, seed=12)
+    cols = g.cols.copy()
+    rng = np.random.default_rng(5)
+    for v in rng.integers(0, g.n, 2000):  # arcs in any order
+        a, b = int(g.offsets[v]), int(g.offsets[v + 1])
+        cols[a:b] = rng.permutation(cols[a:b])
+    G = sg.Graph.from_csr(device, g.offsets, cols)
+    cc = sg.CC(G)
+    cc.init()
+    if noalloc:
+        r = C.c_int32()
+        sg.check(sg.lib().sg_cc_noalloc(G.h, C.c_void_p(cc.labels.ptr), C.byref(r)))
+    else:
+        cc.run()
+    assert np.array_equal(cc.get_labels(), oracle_mod.cc(g))
