@@ -4,24 +4,29 @@
  *
  * Per source s:
  *  1. depths from the fused BFS (sg_bfs, hybrid push/pull);
- *  2. vertices grouped by level: a radix sort of (level, vertex) with the
- *     level clamped to the number of levels, so only a few key bits are sorted;
- *  3. forward, level by level: sigma(v) = sum of sigma(u) over in-arcs u -> v
- *     with depth(u) = depth(v) - 1, then the level is rescaled by a power of
- *     two so that its largest sigma lies in [0.5, 1) -- path counts overflow
- *     FP64 on long-diameter graphs (a 4096 x 4096 grid has ~1e2464 shortest
- *     paths corner to corner), and power-of-two scaling is exact;
- *  4. backward, deepest level first: delta(u) = sigma(u) * scale(L+1) *
- *     sum over out-arcs u -> w with depth(w) = depth(u) + 1 of
- *     (1 + delta(w)) / sigma(w); bc(u) += delta(u) for u != s (no halving on
- *     undirected graphs, as bc.hpp:186-196).
+ *  2. vertices grouped by level, in no particular order (every vertex's sums
+ *     are its own): a counting sort, or with more than kCountLevels levels a
+ *     radix sort of (level, vertex);
+ *  3. forward, level by level: sigma(v) = sum of scale(L - 1) * sigma(u) over
+ *     in-arcs u -> v with depth(u) = depth(v) - 1 = L - 1, where scale(L) is
+ *     the power of two that brings the level's largest sigma into [0.5, 1) --
+ *     path counts overflow FP64 on long-diameter graphs (a 4096 x 4096 grid
+ *     has ~1e2464 shortest paths corner to corner), and power-of-two scaling
+ *     is exact;
+ *  4. backward, deepest level first: delta(u) = scale(L) * sigma(u) * sum of
+ *     R(w) over out-arcs u -> w with depth(w) = depth(u) + 1 = L + 1, and R(u)
+ *     = (1 + delta(u)) / sigma(u), one division per vertex and one gather per
+ *     arc (the scales of w's level cancel); bc(u) += delta(u) for u != s (no
+ *     halving on undirected graphs, as bc.hpp:186-196).
  * Steps 3 and 4 are pulls: each vertex gathers its own sum, so there are no
- * floating-point atomics and results do not depend on scheduling.  A lane
- * sums a vertex's arcs in CSR order; vertices of degree above kCoop are
- * summed by the whole wave (strided partial sums, fixed butterfly), which
- * changes the rounding order but not the result beyond FP64 rounding.
- * sigma, delta and the per-source accumulation are FP64; the output adds the
- * FP64 total to the caller's float array once at the end.
+ * floating-point atomics and results do not depend on scheduling.  Both read
+ * every arc of the reached vertices once; what bounds them is a vertex's
+ * dependent gathers (id, level bit, value), so eight lanes share a vertex,
+ * four arcs each in flight, and vertices of more than kHub arcs get a
+ * workgroup (a wave for 64 vertices one after another, hubs included, took
+ * 0.7-1.3 ms for RMAT scale 18's largest level).  The partial sums are added
+ * in a fixed order.  sigma, R and the per-source accumulation are FP64; the
+ * output adds the FP64 total to the caller's float array once at the end.
  */
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -31,21 +36,104 @@
 #include <vector>
 
 #include "internal.hpp"
+#include "traverse.hpp"
 
-using namespace sygraph::hipdev;
+using namespace sg::trav;
 
 namespace {
 
-constexpr int kBlock = 256;
-constexpr int kCoop = 16; /* degree above which the wave sums one vertex together */
+constexpr int kHub = 512;          /* degree above which a workgroup sums one vertex */
+constexpr int kTeam = 8;           /* lanes that share a vertex otherwise */
+constexpr int kCountLevels = 1024; /* levels up to which the counting sort's histograms fit in LDS */
 constexpr int kMaxSlots = 64;   /* per-level maximum of sigma: slots, one cache line apart */
 constexpr int kSlotStride = 16; /* unsigned long long per 128-byte line */
 constexpr int64_t kLevelBitmapBytes = 1ll << 30; /* per-level bitmaps up to 1 GiB, else depth[] tests */
 
-__device__ __forceinline__ double wave_sum_f64(double x) {
+/* sum over groups of kLanes lanes, in every lane (fixed butterfly) */
+template<int kLanes>
+__device__ __forceinline__ double lanes_sum(double x) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+  for (int o = kLanes / 2; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
   return x;
+}
+
+/* Counting sort by level: the workgroups' histograms added into count[0..nl)
+ * (cleared before), the level starts, then each workgroup's vertices at the
+ * range it reserves in every level.  The first pass also writes the level
+ * bitmaps of at most 64 levels (lane L keeps the word's bits of level L). */
+__global__ void __launch_bounds__(kBlock) level_count_kernel(const int32_t* depth, int64_t n, int64_t w0, int32_t nl,
+                                                             uint32_t* count, uint64_t* lbm) {
+  __shared__ uint32_t s_n[kCountLevels];
+  for (int l = threadIdx.x; l < nl; l += kBlock) s_n[l] = 0;
+  __syncthreads();
+  const int lane = lane_id();
+  const int64_t gw = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6, nw = ((int64_t)gridDim.x * kBlock) >> 6;
+  for (int64_t w = gw; w < w0; w += nw) {
+    const int64_t v = w * 64 + lane;
+    const int32_t d = v < n ? depth[v] : -1;
+    const bool in = d >= 0 && d < nl;
+    if (lbm) {
+      uint64_t mine = 0;
+      for (int l = 0; l < nl; ++l) {
+        const uint64_t m = ballot(in && d == l);
+        if (l == lane) mine = m;
+      }
+      if (lane < nl) {
+        lbm[(int64_t)lane * w0 + w] = mine;
+        if (mine) atomicAdd(&s_n[lane], (uint32_t)__popcll(mine));
+      }
+    } else if (in) {
+      atomicAdd(&s_n[d], 1u);
+    }
+  }
+  __syncthreads();
+  for (int l = threadIdx.x; l < nl; l += kBlock)
+    if (s_n[l]) atomicAdd(&count[l], s_n[l]);
+}
+
+/* lvl[l] = start of level l, lvl[nl] = the reached vertices; cursor = the starts */
+__global__ void __launch_bounds__(64) level_scan_kernel(const uint32_t* count, int32_t nl, int64_t* lvl,
+                                                        uint32_t* cursor) {
+  uint32_t carry = 0;
+  for (int32_t b = 0; b < nl; b += 64) {
+    const int32_t l = b + lane_id();
+    const uint32_t c = l < nl ? count[l] : 0u;
+    const uint32_t incl = wave_inclusive_scan(c);
+    if (l < nl) {
+      lvl[l] = carry + incl - c;
+      cursor[l] = carry + incl - c;
+    }
+    carry += wave_lane(incl, 63);
+  }
+  if (lane_id() == 0) lvl[nl] = carry;
+}
+
+__global__ void __launch_bounds__(kBlock) level_scatter_kernel(const int32_t* depth, int64_t n, int32_t nl,
+                                                               uint32_t* cursor, int32_t* order) {
+  __shared__ uint32_t s_n[kCountLevels];
+  const int64_t per = (n + gridDim.x - 1) / gridDim.x;
+  const int64_t first = (int64_t)blockIdx.x * per, last = first + per < n ? first + per : n;
+  for (int l = threadIdx.x; l < nl; l += kBlock) s_n[l] = 0;
+  __syncthreads();
+  for (int64_t v = first + threadIdx.x; v < last; v += kBlock) {
+    const int32_t d = depth[v];
+    if (d >= 0 && d < nl) atomicAdd(&s_n[d], 1u);
+  }
+  __syncthreads();
+  for (int l = threadIdx.x; l < nl; l += kBlock)
+    if (s_n[l]) s_n[l] = atomicAdd(&cursor[l], s_n[l]);
+  __syncthreads();
+  for (int64_t v = first + threadIdx.x; v < last; v += kBlock) {
+    const int32_t d = depth[v];
+    if (d >= 0 && d < nl) order[atomicAdd(&s_n[d], 1u)] = (int32_t)v;
+  }
+}
+
+/* vertices of more than kHub arcs (hub[0] counts them, cleared before) */
+template<typename OffT>
+__global__ void __launch_bounds__(kBlock) hub_list_kernel(const OffT* off, int64_t n, uint32_t* hub) {
+  for (int64_t v = blockIdx.x * (int64_t)kBlock + threadIdx.x; v < n; v += (int64_t)gridDim.x * kBlock)
+    if ((int64_t)(off[v + 1] - off[v]) > kHub) hub[1 + atomicAdd(&hub[0], 1u)] = (uint32_t)v;
 }
 
 __global__ void level_keys_kernel(const int32_t* depth, int64_t n, int32_t nlevels, uint32_t* keys, int32_t* ids) {
@@ -87,67 +175,111 @@ __global__ void level_bits_kernel(const int32_t* depth, int64_t n, int64_t w0, i
 
 __device__ __forceinline__ bool bit_of(const uint64_t* bm, int32_t v) { return (bm[v >> 6] >> (v & 63)) & 1ull; }
 
-__global__ void bc_source_init_kernel(double* sigma, double* scale, int32_t s) {
-  sigma[s] = 1.0;
-  scale[0] = 1.0;
+__global__ void bc_source_init_kernel(double* sigma, int32_t s) { sigma[s] = 1.0; }
+
+/* 2^-e for the exponent e of a level's largest sigma (1 where none was
+ * recorded: the source's level).  All threads call; one barrier. */
+__device__ __forceinline__ double level_scale(const unsigned long long* level_max) {
+  __shared__ double s_scale;
+  if (threadIdx.x < 64) {
+    static_assert(kMaxSlots == 64, "a slot per lane");
+    const double mx =
+        __longlong_as_double((long long)wave_max_u64(level_max[(int)threadIdx.x * kSlotStride]));
+    int ex = 0;
+    (void)frexp(mx, &ex);
+    if (threadIdx.x == 0) s_scale = ldexp(1.0, -ex);
+  }
+  __syncthreads();
+  return s_scale;
 }
 
-/* Sum of f(arc) over the arcs of each vertex in [begin, end) of `order`; the
- * wave takes 64 consecutive entries, lanes with long lists are summed
- * cooperatively.  `store(v, sum)` runs once per vertex. */
-template<typename OffT, typename ArcF, typename StoreF>
-__device__ __forceinline__ void gather_level(const int32_t* order, int64_t begin, int64_t end, const OffT* off,
-                                             ArcF arc, StoreF store) {
-  const int lane = lane_id();
-  const int64_t gwave = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
-  const int64_t nwaves = ((int64_t)gridDim.x * kBlock) >> 6;
-  for (int64_t base = begin + gwave * 64; base < end; base += nwaves * 64) {
-    const int64_t i = base + lane;
+/* Sum of value(x) over the neighbours x of each vertex of level L that are in
+ * `bm` (or, where it is null, at depth `want`); store(v, sum) runs once per
+ * vertex.  The first hub_blocks workgroups take the hubs of the level (hub[0]
+ * of them in all, whatever their level), a workgroup each; the others the
+ * level's vertices in `order`, kTeam lanes each. */
+template<typename OffT, typename ValueF, typename StoreF>
+__device__ __forceinline__ void gather_level(const int32_t* order, const int64_t* lvl, int32_t L, const uint32_t* hub,
+                                             int hub_blocks, const OffT* off, const int32_t* cols,
+                                             const int32_t* depth, const uint64_t* bm, int32_t want, ValueF value,
+                                             StoreF store) {
+  constexpr int kArcs = 4; /* per lane in flight */
+  auto part_sum = [&](int64_t a, int64_t b, int me, int width) {
+    double acc = 0.0;
+    for (int64_t e = a + me; e < b; e += (int64_t)kArcs * width) {
+      int32_t x[kArcs];
+      bool in[kArcs];
+      double y[kArcs];
+#pragma unroll
+      for (int k = 0; k < kArcs; ++k) x[k] = e + k * width < b ? cols[e + k * width] : -1;
+#pragma unroll
+      for (int k = 0; k < kArcs; ++k) in[k] = x[k] >= 0 && (bm ? bit_of(bm, x[k]) : depth[x[k]] == want);
+#pragma unroll
+      for (int k = 0; k < kArcs; ++k) y[k] = in[k] ? value(x[k]) : 0.0;
+#pragma unroll
+      for (int k = 0; k < kArcs; ++k) acc += y[k];
+    }
+    return acc;
+  };
+  const int lane = lane_id(), wv = threadIdx.x >> 6;
+  if ((int)blockIdx.x < hub_blocks) {
+    __shared__ double s_part[kBlock / 64];
+    const uint32_t nh = hub[0];
+    for (uint32_t h = blockIdx.x; h < nh; h += (uint32_t)hub_blocks) {
+      const int32_t v = (int32_t)hub[1 + h];
+      if (depth[v] != L) continue;
+      const double acc = lanes_sum<64>(part_sum((int64_t)off[v], (int64_t)off[v + 1], (int)threadIdx.x, kBlock));
+      if (lane == 0) s_part[wv] = acc;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        double total = 0.0;
+        for (int w = 0; w < kBlock / 64; ++w) total += s_part[w];
+        store(v, total);
+      }
+      __syncthreads();
+    }
+    return;
+  }
+  const int64_t begin = lvl[L], end = lvl[L + 1];
+  constexpr int kPerWave = 64 / kTeam;
+  const int64_t gwave = ((int64_t)(blockIdx.x - hub_blocks) * kBlock + threadIdx.x) >> 6;
+  const int64_t nwaves = ((int64_t)(gridDim.x - hub_blocks) * kBlock) >> 6;
+  for (int64_t base = begin + gwave * kPerWave; base < end; base += nwaves * kPerWave) {
+    const int64_t i = base + lane / kTeam;
     int32_t v = -1;
     int64_t a = 0, b = 0;
     if (i < end) {
       v = order[i];
-      a = (int64_t)off[v];
-      b = (int64_t)off[v + 1];
+      list_bounds(off, (uint32_t)v, a, b);
+      if (b - a > kHub) { /* a hub's workgroup has it */
+        v = -1;
+        b = a;
+      }
     }
-    const bool coop = (b - a) > kCoop;
-    double acc = 0.0;
-    if (v >= 0 && !coop)
-      for (int64_t e = a; e < b; ++e) acc += arc(e);
-    uint64_t heavy = ballot(coop);
-    while (heavy) {
-      const int k = __ffsll((unsigned long long)heavy) - 1;
-      heavy &= heavy - 1;
-      const int64_t ka = (int64_t)wave_lane((uint64_t)a, k), kb = (int64_t)wave_lane((uint64_t)b, k);
-      double part = 0.0;
-      for (int64_t e = ka + lane; e < kb; e += 64) part += arc(e);
-      part = wave_sum_f64(part);
-      if (lane == k) acc = part;
-    }
-    if (v >= 0) store(v, acc);
+    const double sum = lanes_sum<kTeam>(part_sum(a, b, lane % kTeam, kTeam));
+    if (v >= 0 && lane % kTeam == 0) store(v, sum);
   }
 }
 
 /* prev_bm: bitmap of level L-1 (L2-resident), or nullptr to test depth[]:
- * sigma is only loaded for real parents */
+ * sigma is only loaded for real parents.  level_max: the slots of level L,
+ * the level before's right ahead of them.  The deepest level's R is final
+ * here. */
 template<typename OffT>
 __global__ void __launch_bounds__(kBlock) sigma_level_kernel(const int32_t* order, const int64_t* lvl, int32_t L,
+                                                             int32_t nl, const uint32_t* hub, int hub_blocks,
                                                              const OffT* in_off, const int32_t* in_cols,
                                                              const int32_t* depth, const uint64_t* prev_bm,
-                                                             double* sigma, unsigned long long* level_max) {
-  const int64_t begin = lvl[L], end = lvl[L + 1];
+                                                             double* sigma, double* r, unsigned long long* level_max) {
+  const double sc = level_scale(level_max - kMaxSlots * kSlotStride);
   double mx = 0.0;
   gather_level<OffT>(
-      order, begin, end, in_off,
-      [&](int64_t e) {
-        const int32_t u = in_cols[e];
-        const bool parent = prev_bm ? bit_of(prev_bm, u) : depth[u] == L - 1;
-        double x = 0.0;
-        if (parent) x = sigma[u];
-        return x;
-      },
+      order, lvl, L, hub, hub_blocks, in_off, in_cols, depth, prev_bm, L - 1,
+      [&](int32_t u) { return sigma[u]; },
       [&](int32_t v, double s) {
+        s *= sc;
         sigma[v] = s;
+        if (L == nl - 1) r[v] = 1.0 / s;
         mx = s > mx ? s : mx;
       });
   /* positive doubles order like their bit patterns; one atomic per workgroup,
@@ -165,48 +297,21 @@ __global__ void __launch_bounds__(kBlock) sigma_level_kernel(const int32_t* orde
   }
 }
 
-__global__ void __launch_bounds__(kBlock) sigma_scale_kernel(const int32_t* order, const int64_t* lvl, int32_t L,
-                                                             double* sigma, const unsigned long long* level_max,
-                                                             double* scale) {
-  __shared__ unsigned long long s_max;
-  if (threadIdx.x == 0) {
-    unsigned long long m = 0;
-    for (int k = 0; k < kMaxSlots; ++k) m = level_max[k * kSlotStride] > m ? level_max[k * kSlotStride] : m;
-    s_max = m;
-  }
-  __syncthreads();
-  const double mx = __longlong_as_double((long long)s_max);
-  int ex = 0;
-  (void)frexp(mx, &ex);
-  const double sc = ldexp(1.0, -ex);
-  if (blockIdx.x == 0 && threadIdx.x == 0) scale[L] = sc;
-  const int64_t begin = lvl[L], end = lvl[L + 1];
-  for (int64_t i = begin + blockIdx.x * (int64_t)kBlock + threadIdx.x; i < end; i += (int64_t)gridDim.x * kBlock)
-    sigma[order[i]] *= sc;
-}
-
-/* next_bm: bitmap of level L+1, or nullptr to test depth[] */
+/* next_bm: bitmap of level L+1, or nullptr to test depth[]; level_max: the
+ * slots of level L */
 template<typename OffT>
 __global__ void __launch_bounds__(kBlock) delta_level_kernel(const int32_t* order, const int64_t* lvl, int32_t L,
-                                                             const OffT* off, const int32_t* cols, const int32_t* depth,
-                                                             const uint64_t* next_bm, const double* sigma,
-                                                             double* delta, const double* scale, double* acc_bc,
-                                                             int32_t s) {
-  const int64_t begin = lvl[L], end = lvl[L + 1];
-  const double sc = scale[L + 1];
+                                                             const uint32_t* hub, int hub_blocks, const OffT* off,
+                                                             const int32_t* cols, const int32_t* depth,
+                                                             const uint64_t* next_bm, const double* sigma, double* r,
+                                                             const unsigned long long* level_max, double* acc_bc) {
+  const double sc = level_scale(level_max);
   gather_level<OffT>(
-      order, begin, end, off,
-      [&](int64_t e) {
-        const int32_t w = cols[e];
-        const bool child = next_bm ? bit_of(next_bm, w) : depth[w] == L + 1;
-        double x = 0.0;
-        if (child) x = (1.0 + delta[w]) / sigma[w];
-        return x;
-      },
+      order, lvl, L, hub, hub_blocks, off, cols, depth, next_bm, L + 1, [&](int32_t w) { return r[w]; },
       [&](int32_t v, double sum) {
-        const double d = sigma[v] * sum * sc;
-        delta[v] = d;
-        if (v != s) acc_bc[v] += d;
+        const double s = sigma[v], d = s * sum * sc;
+        r[v] = (1.0 + d) / s;
+        acc_bc[v] += d;
       });
 }
 
@@ -222,53 +327,44 @@ __global__ void fill_i64_kernel(int64_t* p, int64_t v, int64_t n) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = v;
 }
 
-struct BcBuffers {
-  int32_t* depth = nullptr;
-  uint32_t* keys[2] = {nullptr, nullptr};
-  int32_t* ids[2] = {nullptr, nullptr};
-  int64_t* lvl = nullptr;
-  double* sigma = nullptr;
-  double* delta = nullptr;
-  double* acc = nullptr;
-  double* scale = nullptr;
-  unsigned long long* level_max = nullptr;
-  int64_t level_max_cap = 0; /* levels the slot array holds */
-  uint64_t* lbm = nullptr;   /* per-level vertex bitmaps */
-  int64_t lbm_cap = 0;       /* levels lbm holds */
-  void* sort_tmp = nullptr;
-  size_t sort_bytes = 0;
-  ~BcBuffers() {
-    void* ps[] = {depth, keys[0], keys[1], ids[0], ids[1], lvl, sigma, delta, acc, scale, level_max, lbm, sort_tmp};
-    for (void* p : ps) (void)hipFree(p);
-  }
-};
-
 template<typename OffT>
 int run_bc(sg_graph_t g, int32_t nsrc, const int32_t* sources, float* out) {
   sg_device_t dev = g->dev;
   hipStream_t st = dev->stream;
-  const int64_t n = g->n;
-  BcBuffers B;
-  SG_TRY(sg::alloc_device(dev, (void**)&B.depth, 4 * (n + 1)));
-  for (int k = 0; k < 2; ++k) {
-    SG_TRY(sg::alloc_device(dev, (void**)&B.keys[k], 4 * (n + 1)));
-    SG_TRY(sg::alloc_device(dev, (void**)&B.ids[k], 4 * (n + 1)));
-  }
-  SG_TRY(sg::alloc_device(dev, (void**)&B.lvl, 8 * (n + 2)));
-  SG_TRY(sg::alloc_device(dev, (void**)&B.sigma, 8 * (n + 1)));
-  SG_TRY(sg::alloc_device(dev, (void**)&B.delta, 8 * (n + 1)));
-  SG_TRY(sg::alloc_device(dev, (void**)&B.acc, 8 * (n + 1)));
-  SG_TRY(sg::alloc_device(dev, (void**)&B.scale, 8 * (n + 2)));
-  B.level_max_cap = 0; /* grown per source to the number of levels */
-  SG_HIP(rocprim::radix_sort_pairs(nullptr, B.sort_bytes, B.keys[0], B.keys[1], B.ids[0], B.ids[1], (size_t)n, 0, 32, st));
-  SG_TRY(sg::alloc_device(dev, &B.sort_tmp, B.sort_bytes + 16));
-
+  const int64_t n = g->n, w0 = (n + 63) / 64;
+  for (int32_t i = 0; i < nsrc; ++i)
+    SG_CHECK(sources[i] >= 0 && sources[i] < n, SG_ERR_INVALID, "sg_bc: source %d out of range [0,%lld)", sources[i],
+             (long long)n);
   const OffT* off = (const OffT*)g->offsets;
   const OffT* in_off = (const OffT*)(g->inv_offsets ? g->inv_offsets : g->offsets);
   const int32_t* in_cols = g->inv_cols ? g->inv_cols : g->cols;
+  const bool directed = in_off != off;
+  /* kept with the graph: repeated calls allocate nothing */
+  int32_t *depth = nullptr, *order = nullptr;
+  int64_t* lvl = nullptr;
+  double *sigma = nullptr, *r = nullptr, *acc = nullptr;
+  uint32_t *count = nullptr, *hubs = nullptr, *in_hubs = nullptr;
+  const size_t hub_cap = (size_t)(g->m / kHub) + 2;
+  SG_TRY(sg::graph_buffer(g, "bc_depth", 4 * (size_t)(n + 1), &depth));
+  SG_TRY(sg::graph_buffer(g, "bc_order", 4 * (size_t)(n + 1), &order));
+  SG_TRY(sg::graph_buffer(g, "bc_lvl", 8 * (size_t)(n + 2), &lvl));
+  SG_TRY(sg::graph_buffer(g, "bc_sigma", 8 * (size_t)(n + 1), &sigma));
+  SG_TRY(sg::graph_buffer(g, "bc_r", 8 * (size_t)(n + 1), &r));
+  SG_TRY(sg::graph_buffer(g, "bc_acc", 8 * (size_t)(n + 1), &acc));
+  SG_TRY(sg::graph_buffer(g, "bc_count", 4 * 2 * kCountLevels, &count));
+  SG_TRY(sg::graph_buffer(g, "bc_hubs", 4 * hub_cap, &hubs));
+  if (directed) SG_TRY(sg::graph_buffer(g, "bc_in_hubs", 4 * hub_cap, &in_hubs));
+  else in_hubs = hubs;
   const int grid_n = sg::grid_for(dev, n, kBlock, 4);
-  const int grid_lvl = dev->cus * 4;
-  fill_f64_kernel<<<grid_n, kBlock, 0, st>>>(B.acc, 0.0, n);
+  const int grid_lvl = dev->cus * 8, hub_blocks = dev->cus * 2;
+  fill_f64_kernel<<<grid_n, kBlock, 0, st>>>(acc, 0.0, n);
+  SG_TRY(sg::zero_async(dev, hubs, 4));
+  hub_list_kernel<OffT><<<grid_n, kBlock, 0, st>>>(off, n, hubs);
+  if (directed) {
+    SG_TRY(sg::zero_async(dev, in_hubs, 4));
+    hub_list_kernel<OffT><<<grid_n, kBlock, 0, st>>>(in_off, n, in_hubs);
+  }
+  SG_HIP(hipGetLastError());
 
   sg_bfs_options opt;
   sg_bfs_options_default(&opt);
@@ -277,58 +373,58 @@ int run_bc(sg_graph_t g, int32_t nsrc, const int32_t* sources, float* out) {
   auto stats = std::make_unique<sg_bfs_stats>();
   for (int32_t si = 0; si < nsrc; ++si) {
     const int32_t s = sources[si];
-    SG_CHECK(s >= 0 && s < n, SG_ERR_INVALID, "sg_bc: source %d out of range [0,%lld)", s, (long long)n);
-    SG_TRY(sg_bfs(g, s, &opt, B.depth, stats.get()));
+    SG_TRY(sg_bfs(g, s, &opt, depth, stats.get()));
     const int32_t nl = stats->levels; /* depths 0 .. nl-1 */
     if (nl < 2) continue;             /* nothing reached: no dependencies */
-    int bits = 1;
-    while ((1u << bits) <= (uint32_t)nl) ++bits;
-    level_keys_kernel<<<grid_n, kBlock, 0, st>>>(B.depth, n, nl, B.keys[0], B.ids[0]);
-    size_t tb = B.sort_bytes;
-    SG_HIP(rocprim::radix_sort_pairs(B.sort_tmp, tb, B.keys[0], B.keys[1], B.ids[0], B.ids[1], (size_t)n, 0, bits, st));
-    fill_i64_kernel<<<sg::grid_for(dev, nl + 2, kBlock, 1), kBlock, 0, st>>>(B.lvl, n, nl + 2);
-    level_starts_kernel<<<grid_n, kBlock, 0, st>>>(B.keys[1], n, B.lvl);
-    if (B.level_max_cap < nl + 1) {
-      SG_HIP(hipStreamSynchronize(st));
-      (void)hipFree(B.level_max);
-      B.level_max = nullptr;
-      SG_TRY(sg::alloc_device(dev, (void**)&B.level_max, 8 * (size_t)(nl + 1) * kMaxSlots * kSlotStride));
-      B.level_max_cap = nl + 1;
-    }
-    fill_i64_kernel<<<sg::grid_for(dev, (int64_t)(nl + 1) * kMaxSlots * kSlotStride, kBlock, 4), kBlock, 0, st>>>(
-        (int64_t*)B.level_max, 0, (int64_t)(nl + 1) * kMaxSlots * kSlotStride);
-    fill_f64_kernel<<<grid_n, kBlock, 0, st>>>(B.delta, 0.0, n);
-    bc_source_init_kernel<<<1, 1, 0, st>>>(B.sigma, B.scale, s);
     /* level bitmaps when they take at most kLevelBitmapBytes (long-diameter
      * graphs fall back to testing depth[]) */
-    const int64_t w0 = (n + 63) / 64;
     const bool use_lbm = (int64_t)nl * w0 * 8 <= kLevelBitmapBytes;
-    if (use_lbm) {
-      if (B.lbm_cap < nl) {
-        SG_HIP(hipStreamSynchronize(st));
-        (void)hipFree(B.lbm);
-        B.lbm = nullptr;
-        SG_TRY(sg::alloc_device(dev, (void**)&B.lbm, 8 * (size_t)nl * w0));
-        B.lbm_cap = nl;
-      }
-      fill_i64_kernel<<<sg::grid_for(dev, (int64_t)nl * w0, kBlock, 4), kBlock, 0, st>>>((int64_t*)B.lbm, 0,
+    uint64_t* lbm = nullptr;
+    if (use_lbm) SG_TRY(sg::graph_buffer(g, "bc_lbm", 8 * (size_t)nl * w0, &lbm));
+    const size_t slot_words = (size_t)kMaxSlots * kSlotStride;
+    unsigned long long* level_max = nullptr;
+    SG_TRY(sg::graph_buffer(g, "bc_level_max", 8 * slot_words * (nl + 1), &level_max));
+    fill_i64_kernel<<<sg::grid_for(dev, (int64_t)((nl + 1) * slot_words), kBlock, 4), kBlock, 0, st>>>(
+        (int64_t*)level_max, 0, (int64_t)((nl + 1) * slot_words));
+    if (nl <= kCountLevels) {
+      uint32_t* cursor = count + kCountLevels;
+      fill_i64_kernel<<<1, kBlock, 0, st>>>((int64_t*)count, 0, kCountLevels / 2);
+      level_count_kernel<<<grid_n, kBlock, 0, st>>>(depth, n, w0, nl, count, use_lbm && nl <= 64 ? lbm : nullptr);
+      level_scan_kernel<<<1, 64, 0, st>>>(count, nl, lvl, cursor);
+      level_scatter_kernel<<<grid_n, kBlock, 0, st>>>(depth, n, nl, cursor, order);
+    } else {
+      uint32_t* keys = nullptr; /* both sides of the sort */
+      int32_t* ids = nullptr;
+      void* tmp = nullptr;
+      size_t tmp_bytes = 0;
+      int bits = 1;
+      while ((1u << bits) <= (uint32_t)nl) ++bits;
+      SG_TRY(sg::graph_buffer(g, "bc_keys", 4 * (size_t)(2 * n + 2), &keys));
+      SG_TRY(sg::graph_buffer(g, "bc_ids", 4 * (size_t)(n + 1), &ids));
+      SG_HIP(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys, keys + n + 1, ids, order, (size_t)n, 0, bits, st));
+      SG_TRY(sg::graph_buffer(g, "bc_sort_tmp", tmp_bytes + 16, &tmp));
+      level_keys_kernel<<<grid_n, kBlock, 0, st>>>(depth, n, nl, keys, ids);
+      SG_HIP(rocprim::radix_sort_pairs(tmp, tmp_bytes, keys, keys + n + 1, ids, order, (size_t)n, 0, bits, st));
+      fill_i64_kernel<<<sg::grid_for(dev, nl + 2, kBlock, 1), kBlock, 0, st>>>(lvl, n, nl + 2);
+      level_starts_kernel<<<grid_n, kBlock, 0, st>>>(keys + n + 1, n, lvl);
+    }
+    if (use_lbm && nl > 64) {
+      fill_i64_kernel<<<sg::grid_for(dev, (int64_t)nl * w0, kBlock, 4), kBlock, 0, st>>>((int64_t*)lbm, 0,
                                                                                       (int64_t)nl * w0);
-      level_bits_kernel<<<sg::grid_for(dev, n, kBlock, 4), kBlock, 0, st>>>(B.depth, n, w0, nl, B.lbm);
+      level_bits_kernel<<<sg::grid_for(dev, n, kBlock, 4), kBlock, 0, st>>>(depth, n, w0, nl, lbm);
     }
-    auto lbm_of = [&](int32_t L) -> const uint64_t* { return use_lbm ? B.lbm + (int64_t)L * w0 : nullptr; };
-    const int32_t* order = B.ids[1];
-    for (int32_t L = 1; L < nl; ++L) {
-      unsigned long long* lm = B.level_max + (size_t)L * kMaxSlots * kSlotStride;
-      sigma_level_kernel<OffT><<<grid_lvl, kBlock, 0, st>>>(order, B.lvl, L, in_off, in_cols, B.depth, lbm_of(L - 1),
-                                                            B.sigma, lm);
-      sigma_scale_kernel<<<grid_lvl, kBlock, 0, st>>>(order, B.lvl, L, B.sigma, lm, B.scale);
-    }
-    for (int32_t L = nl - 2; L >= 0; --L)
-      delta_level_kernel<OffT><<<grid_lvl, kBlock, 0, st>>>(order, B.lvl, L, off, g->cols, B.depth, lbm_of(L + 1),
-                                                            B.sigma, B.delta, B.scale, B.acc, s);
+    bc_source_init_kernel<<<1, 1, 0, st>>>(sigma, s);
+    auto lbm_of = [&](int32_t L) -> const uint64_t* { return use_lbm ? lbm + (int64_t)L * w0 : nullptr; };
+    for (int32_t L = 1; L < nl; ++L)
+      sigma_level_kernel<OffT><<<grid_lvl, kBlock, 0, st>>>(order, lvl, L, nl, in_hubs, hub_blocks, in_off, in_cols,
+                                                            depth, lbm_of(L - 1), sigma, r, level_max + L * slot_words);
+    /* the source's own dependency is not counted */
+    for (int32_t L = nl - 2; L >= 1; --L)
+      delta_level_kernel<OffT><<<grid_lvl, kBlock, 0, st>>>(order, lvl, L, hubs, hub_blocks, off, g->cols, depth,
+                                                            lbm_of(L + 1), sigma, r, level_max + L * slot_words, acc);
     SG_HIP(hipGetLastError());
   }
-  add_to_float_kernel<<<grid_n, kBlock, 0, st>>>(B.acc, out, n);
+  add_to_float_kernel<<<grid_n, kBlock, 0, st>>>(acc, out, n);
   SG_HIP(hipGetLastError());
   SG_HIP(hipStreamSynchronize(st));
   return SG_OK;

@@ -153,3 +153,26 @@ def test_bfs_multi_matches_oracle(sg, device, oracle_mod):
     d = sg.bfs_multi(G, srcs)
     for i, s in enumerate(srcs):
         assert np.array_equal(d[i], oracle_mod.bfs(g, s)[0])
+
+
+@pytest.mark.parametrize("levels", [30, 200, 1500])
+@pytest.mark.parametrize("directed", [False, True])
+def test_bc_level_grouping_and_hubs(sg, device, oracle_mod, levels, directed):
+    """Level counts on each side of the level grouping's limits (64 levels with bitmaps written by the
+    counting pass, 1,024 counted, more sorted), rungs of several shortest paths, and hubs of 700 arcs
+    (a workgroup's share) in the middle and at the end."""
+    a = np.arange(levels - 1)
+    u = np.concatenate([2 * a, 2 * a, 2 * a + 1, np.full(700, levels), np.full(700, 2 * levels - 1)])
+    v = np.concatenate([2 * a + 2, 2 * a + 3, 2 * a + 2, 2 * levels + np.arange(700), 2 * levels + np.arange(700)])
+    n = 2 * levels + 700
+    if directed:
+        key = np.unique(u.astype(np.int64) * n + v)
+        off = np.zeros(n + 1, dtype=np.int64)
+        np.add.at(off, key // n + 1, 1)
+        g = oracle_mod.CSRGraph(n, np.cumsum(off), (key % n).astype(np.int32))
+        ref = oracle_mod.bc(g, [0, 4], inverse=oracle_mod.transpose(g))
+    else:
+        g = oracle_mod.csr_from_pairs(n, u, v)
+        ref = oracle_mod.bc(g, [0, 4])
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, directed=directed)
+    assert _close(_bc(sg, G, [0, 4]), ref)
