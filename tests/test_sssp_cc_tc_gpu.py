@@ -572,3 +572,34 @@ def test_cc_first_parents_and_chains(sg, device, oracle_mod, graph, noalloc):
     else:
         cc.run()
     assert np.array_equal(cc.get_labels(), oracle_mod.cc(g))
+
+
+@pytest.mark.parametrize("offset_bytes", [4, 8])
+@pytest.mark.parametrize("n", [3, 16, 17, 97, 98, 257, 4200])
+def test_tc_complete_graphs_per_vertex(sg, device, n, offset_bytes):
+    """K_n: equal degrees, so vertex u keeps the n - 1 - u larger ids and gets the pairs among them.
+    The sizes put lists on both sides of each of the kernel's limits: a wave or a workgroup per vertex
+    (96 ids), lists walked together, by a quarter wave or a wave (16 and 256), lists too long for the
+    table (4,096)."""
+    cols = (np.arange(n * (n - 1), dtype=np.int64) % (n - 1))
+    row = np.repeat(np.arange(n), n - 1)
+    cols = (cols + (cols >= row)).astype(np.int32)
+    G = sg.Graph.from_csr(device, np.arange(n + 1, dtype=np.int64) * (n - 1), cols, offset_bytes=offset_bytes)
+    t = sg.TC(G)
+    assert t.run(per_vertex=True) == n * (n - 1) * (n - 2) // 6
+    left = np.arange(n, 0, -1, dtype=np.uint64) - np.uint64(1)
+    pairs = left * (left - np.minimum(left, np.uint64(1))) // np.uint64(2)
+    assert np.array_equal(t.per_vertex.download(np.uint64, n), pairs)
+
+
+@pytest.mark.parametrize("seed,n,hubs,arcs", [(1, 5000, 0, 20000), (2, 3000, 3, 30000), (3, 700, 40, 5000)])
+def test_tc_matches_oracle_on_uneven_degrees(sg, device, oracle_mod, seed, n, hubs, arcs):
+    """Random graphs with a few vertices joined to most others: orientation of long lists by the whole
+    wave and of short ones by teams, with vertices of no arcs between them."""
+    rng = np.random.default_rng(seed)
+    u, v = rng.integers(0, n, arcs), rng.integers(0, n, arcs)
+    for h in range(hubs):
+        pick = rng.choice(n, n // 2, replace=False)
+        u, v = np.concatenate([u, np.full(len(pick), h)]), np.concatenate([v, pick])
+    g = oracle_mod.csr_from_pairs(n + 70, u, v)
+    assert sg.TC(sg.Graph.from_csr(device, g.offsets, g.cols)).run() == oracle_mod.tc(g)
