@@ -35,6 +35,10 @@
  * sums align exponents as they go.  The backward pass overwrites sigma with
  * R = (1 + delta) / sigma in the same form, so an arc's term is one product
  * and one ldexp; delta itself is at most the vertex count and stays FP32.
+ * Short-diameter graphs never leave FP32's range, so a batch runs without the
+ * exponents (256 bytes a row instead of 384, and the rows are most of what a
+ * batch reads) until a path count reaches 2^100; it then runs again with
+ * them, and so do the graph's later batches.
  * The backward pass walks the levels deepest first; membership of level d+1
  * is rebuilt from its list into one of two mask arrays (the OR of L_d's masks
  * and the AND-NOT of L_{d+2}'s act on disjoint lanes, so they commute).
@@ -97,8 +101,10 @@ constexpr int kLiRing = 8;    /* level records of the MS-BFS ring */
 constexpr int kBarGroups = 8; /* arrival counters, one per XCD */
 constexpr int kBarStride = 32; /* 128 bytes apart */
 constexpr uint32_t kOvList = 1, kOvHubV = 2, kOvHubC = 4, kOvPart = 8, kOvLevels = 16;
-constexpr uint32_t kTimeout = 32, kRange = 64;
-constexpr uint32_t kStop = kOvList | kOvHubV | kOvHubC | kOvPart | kOvLevels | kTimeout | kRange;
+constexpr uint32_t kTimeout = 32, kRange = 64, kOvPlain = 128;
+constexpr uint32_t kStop = kOvList | kOvHubV | kOvHubC | kOvPart | kOvLevels | kTimeout | kRange | kOvPlain;
+constexpr float kPlainMax = 0x1p100f; /* sigma below this needs no exponent: R = (1 + delta) / sigma and the products
+                                         of the two then stay within FP32's normal range */
 constexpr int kExpMax = 32000; /* |exponent| of sigma and R kept in int16 */
 
 /* One level: its vertices and the chunks of its long lists (out-arcs; in-arcs
@@ -149,6 +155,8 @@ struct MsArgs {
   int32_t bc;       /* 1: batched BC, 0: MS-BFS */
   int32_t ring;     /* 1: level lists in a ring of four slots (MS-BFS) */
   int32_t directed; /* in-arcs are not the out-arcs */
+  int32_t plain;    /* BC: sigma and R as plain FP32 (no exponents) */
+  int64_t mean;     /* arcs per vertex */
   const OffT* off;
   const int32_t* cols;
   const OffT* ioff;
@@ -514,9 +522,13 @@ __device__ __forceinline__ bool pair_item(PairWalk& w, uint64_t mine, uint32_t s
   return (word >> lane) & 1ull;
 }
 
-/* running sum S * 2^E of terms a * 2^e (exponents aligned as they come) */
+/* running sum S * 2^E of terms a * 2^e (exponents aligned as they come);
+ * kPlain: all exponents are zero */
+template<bool kPlain>
 __device__ __forceinline__ void xadd(float& S, int& E, float a, int e) {
-  if (e > E) {
+  if (kPlain) {
+    S += a;
+  } else if (e > E) {
     const int sh = E - e;
     S = __builtin_amdgcn_ldexpf(S, sh < -200 ? -200 : sh) + a;
     E = e;
@@ -527,9 +539,20 @@ __device__ __forceinline__ void xadd(float& S, int& E, float a, int e) {
 }
 constexpr int kNoExp = -(1 << 30);
 
-/* store S * 2^E as mantissa in [0.5, 1) and int16 exponent */
-template<typename OffT>
+template<bool kPlain, typename OffT>
+__device__ __forceinline__ int load_exp(const MsArgs<OffT>& a, int64_t at) {
+  return kPlain ? 0 : (int)cld(&a.se[at]);
+}
+
+/* store S * 2^E as mantissa in [0.5, 1) and int16 exponent; kPlain: S as it
+ * is, which must stay below kPlainMax */
+template<bool kPlain, typename OffT>
 __device__ __forceinline__ void store_norm(const MsArgs<OffT>& a, int64_t at, float S, int E) {
+  if (kPlain) {
+    if (!(S < kPlainMax)) raise_flag(a.ctl, kOvPlain);
+    cst(&a.sm[at], S);
+    return;
+  }
   int k = 0;
   float m = 0.f;
   if (S > 0.f) {
@@ -548,10 +571,11 @@ __device__ __forceinline__ void store_norm(const MsArgs<OffT>& a, int64_t at, fl
 template<typename OffT>
 __device__ __forceinline__ void expand_push(const MsArgs<OffT>& a, int32_t d, int64_t base, int64_t cnt,
                                             const uint64_t* Mc, uint64_t* Mn, LevelInfo* nx, const Bases& nb,
-                                            Stage& stg, int64_t gwave, int64_t nwaves) {
+                                            Stage& stg, int64_t gwave, int64_t nwaves, int64_t mean) {
   const int lane = lane_id();
-  for (int64_t g = gwave; g * 64 < cnt; g += nwaves) {
-    const int64_t i = g * 64 + lane;
+  const int group = group_entries(cnt, nwaves, mean);
+  for (int64_t g = gwave; g * group < cnt; g += nwaves) {
+    const int64_t i = lane < group ? g * group + lane : cnt;
     uint64_t fm = 0;
     int64_t st = 0;
     uint32_t len = 0;
@@ -615,8 +639,11 @@ __device__ __forceinline__ void expand_chunks(const MsArgs<OffT>& a, const HubC*
 }
 
 /* Pull expansion: every vertex still missing lanes ORs the level masks of its
- * in-neighbours, stopping once the missing lanes are covered; lists longer
- * than 64 arcs are ORed by the whole wave. */
+ * in-neighbours, stopping once the missing lanes are covered.  A lane takes
+ * eight arcs at a time, so that eight masks are on their way instead of one;
+ * what is left of a list after kPullSerial arcs, the whole wave ORs, four arcs
+ * per lane and step. */
+constexpr int kPullSerial = 32;
 template<typename OffT>
 __device__ __forceinline__ void expand_pull(const MsArgs<OffT>& a, const uint64_t* Mc, uint64_t* Mn, LevelInfo* nx,
                                             const Bases& nb, Stage& st, int64_t gwave, int64_t nwaves) {
@@ -632,26 +659,40 @@ __device__ __forceinline__ void expand_pull(const MsArgs<OffT>& a, const uint64_
         e = (int64_t)a.ioff[v + 1];
       }
     }
-    const bool coop = e - b > 64;
-    if (!coop)
-      for (int64_t j = b; j < e; ++j) {
-        acc |= cld(&Mc[a.icols[j]]);
-        if ((acc & want) == want) break;
-      }
-    uint64_t heavy = ballot(coop);
-    while (heavy) {
-      const int k = __ffsll((unsigned long long)heavy) - 1;
-      heavy &= heavy - 1;
-      const int64_t kb = (int64_t)wave_lane((uint64_t)b, k), ke = (int64_t)wave_lane((uint64_t)e, k);
-      const uint64_t kwant = wave_lane(want, k);
-      uint64_t part = 0;
-      for (int64_t j0 = kb; j0 < ke; j0 += 64) {
-        if (j0 + lane < ke) part |= cld(&Mc[a.icols[j0 + lane]]);
+    const int64_t head = e - b > kPullSerial ? b + kPullSerial : e;
+    int64_t j = b;
+    for (; j < head; j += 8) {
+      int32_t x[8];
+      uint64_t m[8];
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) part |= shfl_u64(part, lane ^ o);
-        if ((part & kwant) == kwant) break;
+      for (int k = 0; k < 8; ++k) x[k] = j + k < head ? a.icols[j + k] : -1;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) m[k] = x[k] >= 0 ? cld(&Mc[x[k]]) : 0ull;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) acc |= m[k];
+      if ((acc & want) == want) break;
+    }
+    uint64_t heavy = ballot(head < e && (acc & want) != want);
+    while (heavy) {
+      const int k2 = __ffsll((unsigned long long)heavy) - 1;
+      heavy &= heavy - 1;
+      const int64_t kb = (int64_t)wave_lane((uint64_t)head, k2), ke = (int64_t)wave_lane((uint64_t)e, k2);
+      const uint64_t kwant = wave_lane(want, k2);
+      uint64_t part = lane == 0 ? wave_lane(acc, k2) : 0ull;
+      uint64_t all = 0;
+      for (int64_t j0 = kb; j0 < ke; j0 += 4 * 64) {
+        int32_t x[4];
+        uint64_t m[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = j0 + 64 * k + lane < ke ? a.icols[j0 + 64 * k + lane] : -1;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) m[k] = x[k] >= 0 ? cld(&Mc[x[k]]) : 0ull;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) part |= m[k];
+        all = wave_lane(wave_prefix(part, [](uint64_t p, uint64_t q) { return p | q; }), 63);
+        if ((all & kwant) == kwant) break;
       }
-      if (lane == k) acc = part;
+      if (lane == k2) acc = all;
     }
     const uint64_t add = acc & want;
     const bool first = add != 0;
@@ -661,7 +702,7 @@ __device__ __forceinline__ void expand_pull(const MsArgs<OffT>& a, const uint64_
 }
 
 /* Visit L_d: vis |= M_d, depth rows (MS-BFS) or the kept masks (BC). */
-template<typename OffT>
+template<bool kBc, typename OffT>
 __device__ __forceinline__ void visit_level(const MsArgs<OffT>& a, int32_t d, int64_t base, int64_t cnt,
                                             const uint64_t* Mc, int64_t gwave, int64_t nwaves) {
   const int lane = lane_id();
@@ -673,7 +714,7 @@ __device__ __forceinline__ void visit_level(const MsArgs<OffT>& a, int32_t d, in
     const uint64_t m = cld(&Mc[u]);
     const uint64_t old = cld(&a.vis[u]);
     cst(&a.vis[u], old | m);
-    if (a.bc) {
+    if (kBc) {
       cst(&a.lm[base + i], m);
     } else {
       /* one store per source that reached u at this depth (a sparse mask
@@ -737,12 +778,13 @@ __device__ __forceinline__ void wave_list_walk(const int32_t* ids, int64_t vb, i
 
 /* Path counts of the pairs of L_d whose in-lists are short: each pair sums
  * sigma over its in-arcs from depth d-1 (M_{d-1}). */
-template<typename OffT>
+template<bool kPlain, typename OffT>
 __device__ __forceinline__ void sigma_pairs(const MsArgs<OffT>& a, int64_t base, int64_t cnt, const uint64_t* Mc,
-                                            const uint64_t* Mp, int64_t gwave, int64_t nwaves) {
+                                            const uint64_t* Mp, int64_t gwave, int64_t nwaves, int64_t mean) {
   const int lane = lane_id();
-  for (int64_t g = gwave; g * 64 < cnt; g += nwaves) {
-    const int64_t i = g * 64 + lane;
+  const int group = group_entries(cnt, nwaves, mean);
+  for (int64_t g = gwave; g * group < cnt; g += nwaves) {
+    const int64_t i = lane < group ? g * group + lane : cnt;
     int32_t u = 0;
     uint64_t own = 0;
     int64_t b = 0, e = 0;
@@ -767,13 +809,13 @@ __device__ __forceinline__ void sigma_pairs(const MsArgs<OffT>& a, int64_t base,
 #pragma unroll
           for (int k = 0; k < 8; ++k) {
             sv[k] = hit[k] ? cld(&a.sm[(int64_t)x[k] * 64 + l]) : 0.f;
-            ev[k] = hit[k] ? (int)cld(&a.se[(int64_t)x[k] * 64 + l]) : 0;
+            ev[k] = hit[k] ? load_exp<kPlain>(a, (int64_t)x[k] * 64 + l) : 0;
           }
 #pragma unroll
           for (int k = 0; k < 8; ++k)
-            if (hit[k]) xadd(S, E, sv[k], ev[k]);
+            if (hit[k]) xadd<kPlain>(S, E, sv[k], ev[k]);
         });
-        if (ok) store_norm(a, (int64_t)v * 64 + l, S, E);
+        if (ok) store_norm<kPlain>(a, (int64_t)v * 64 + l, S, E);
         continue;
       }
       if (!ok) continue;
@@ -789,20 +831,20 @@ __device__ __forceinline__ void sigma_pairs(const MsArgs<OffT>& a, int64_t base,
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           sv[k] = hit[k] ? cld(&a.sm[(int64_t)x[k] * 64 + l]) : 0.f;
-          ev[k] = hit[k] ? (int)cld(&a.se[(int64_t)x[k] * 64 + l]) : 0;
+          ev[k] = hit[k] ? load_exp<kPlain>(a, (int64_t)x[k] * 64 + l) : 0;
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-          if (hit[k]) xadd(S, E, sv[k], ev[k]);
+          if (hit[k]) xadd<kPlain>(S, E, sv[k], ev[k]);
       }
-      store_norm(a, (int64_t)v * 64 + l, S, E);
+      store_norm<kPlain>(a, (int64_t)v * 64 + l, S, E);
     }
   }
 }
 
 /* Partial path counts over one chunk of a long in-list: a wave per chunk,
  * lane = source. */
-template<typename OffT>
+template<bool kPlain, typename OffT>
 __device__ __forceinline__ void sigma_chunks(const MsArgs<OffT>& a, const HubC* hc, int64_t nc, const uint64_t* Mc,
                                              const uint64_t* Mp, int64_t gwave, int64_t nwaves) {
   const int lane = lane_id();
@@ -820,15 +862,15 @@ __device__ __forceinline__ void sigma_chunks(const MsArgs<OffT>& a, const HubC* 
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         sv[k] = hit[k] ? cld(&a.sm[(int64_t)x[k] * 64 + lane]) : 0.f;
-        ev[k] = hit[k] ? (int)cld(&a.se[(int64_t)x[k] * 64 + lane]) : 0;
+        ev[k] = hit[k] ? load_exp<kPlain>(a, (int64_t)x[k] * 64 + lane) : 0;
       }
 #pragma unroll
       for (int k = 0; k < 8; ++k)
-        if (hit[k]) xadd(S, E, sv[k], ev[k]);
+        if (hit[k]) xadd<kPlain>(S, E, sv[k], ev[k]);
     });
     if (c < a.p_cap) {
       cst(&a.pS[c * 64 + lane], S);
-      cst(&a.pE[c * 64 + lane], E);
+      if (!kPlain) cst(&a.pE[c * 64 + lane], E);
     } else if (lane == 0) {
       raise_flag(a.ctl, kOvPart);
     }
@@ -836,7 +878,7 @@ __device__ __forceinline__ void sigma_chunks(const MsArgs<OffT>& a, const HubC* 
 }
 
 /* Chunked vertices: add the partial rows in chunk order. */
-template<typename OffT>
+template<bool kPlain, typename OffT>
 __device__ __forceinline__ void sigma_combine(const MsArgs<OffT>& a, const HubV* hv, int64_t nv, const uint64_t* Mc,
                                               int64_t gwave, int64_t nwaves) {
   const int lane = lane_id();
@@ -848,35 +890,38 @@ __device__ __forceinline__ void sigma_combine(const MsArgs<OffT>& a, const HubV*
     for (int32_t c = 0; c < h.nch; ++c) {
       const int64_t slot = (int64_t)h.first + c;
       const float s = cld(&a.pS[slot * 64 + lane]);
-      if (s > 0.f) xadd(S, E, s, cld(&a.pE[slot * 64 + lane]));
+      if (s > 0.f) xadd<kPlain>(S, E, s, kPlain ? 0 : cld(&a.pE[slot * 64 + lane]));
     }
-    store_norm(a, (int64_t)h.v * 64 + lane, S, E);
+    store_norm<kPlain>(a, (int64_t)h.v * 64 + lane, S, E);
   }
 }
 
 /* ------------------------------------------------------- backward phase --- */
 /* delta of a pair from its arc sum: R = (1 + delta) / sigma replaces sigma */
-template<typename OffT>
+template<bool kPlain, typename OffT>
 __device__ __forceinline__ void finish_delta(const MsArgs<OffT>& a, int64_t at, float delta) {
   const float m = cld(&a.sm[at]);
-  const int e = (int)cld(&a.se[at]);
+  const int e = load_exp<kPlain>(a, at);
   cst(&a.dl[at], delta);
   const float r = (1.0f + delta) / m;
-  store_norm(a, at, r, -e);
+  store_norm<kPlain>(a, at, r, -e);
 }
 
 /* One arc's term sigma_l(v) / sigma_l(w) * (1 + delta_l(w)) = m_v 2^e_v R_l(w). */
+template<bool kPlain>
 __device__ __forceinline__ float delta_term(float mv, int ev, float mr, int er) {
+  if (kPlain) return mv * mr;
   const int sh = ev + er;
   return __builtin_amdgcn_ldexpf(mv * mr, sh < -200 ? -200 : (sh > 100 ? 100 : sh));
 }
 
-template<typename OffT>
+template<bool kPlain, typename OffT>
 __device__ __forceinline__ void delta_pairs(const MsArgs<OffT>& a, int64_t base, int64_t cnt, const uint64_t* Xa,
-                                            int64_t gwave, int64_t nwaves) {
+                                            int64_t gwave, int64_t nwaves, int64_t mean) {
   const int lane = lane_id();
-  for (int64_t g = gwave; g * 64 < cnt; g += nwaves) {
-    const int64_t i = g * 64 + lane;
+  const int group = group_entries(cnt, nwaves, mean);
+  for (int64_t g = gwave; g * group < cnt; g += nwaves) {
+    const int64_t i = lane < group ? g * group + lane : cnt;
     int32_t u = 0;
     uint64_t own = 0;
     int64_t b = 0, e = 0;
@@ -895,7 +940,7 @@ __device__ __forceinline__ void delta_pairs(const MsArgs<OffT>& a, int64_t base,
       const int64_t at = (int64_t)v * 64 + l;
       if (!w.flat) { /* one vertex, every lane a source */
         const float mv = ok ? cld(&a.sm[at]) : 0.f;
-        const int ev = ok ? (int)cld(&a.se[at]) : 0;
+        const int ev = ok ? load_exp<kPlain>(a, at) : 0;
         float acc = 0.f;
         wave_list_walk(a.cols, vb, ve, Xa, l, ok, [&](const int32_t (&x)[8], const bool (&hit)[8]) {
           float r[8];
@@ -903,18 +948,18 @@ __device__ __forceinline__ void delta_pairs(const MsArgs<OffT>& a, int64_t base,
 #pragma unroll
           for (int k = 0; k < 8; ++k) {
             r[k] = hit[k] ? cld(&a.sm[(int64_t)x[k] * 64 + l]) : 0.f;
-            er[k] = hit[k] ? (int)cld(&a.se[(int64_t)x[k] * 64 + l]) : 0;
+            er[k] = hit[k] ? load_exp<kPlain>(a, (int64_t)x[k] * 64 + l) : 0;
           }
 #pragma unroll
           for (int k = 0; k < 8; ++k)
-            if (hit[k]) acc += delta_term(mv, ev, r[k], er[k]);
+            if (hit[k]) acc += delta_term<kPlain>(mv, ev, r[k], er[k]);
         });
-        if (ok) finish_delta(a, at, acc);
+        if (ok) finish_delta<kPlain>(a, at, acc);
         continue;
       }
       if (!ok) continue;
       const float mv = cld(&a.sm[at]);
-      const int ev = (int)cld(&a.se[at]);
+      const int ev = load_exp<kPlain>(a, at);
       float acc = 0.f;
       for (int64_t j = vb; j < ve; j += 4) {
         int32_t x[4];
@@ -928,18 +973,18 @@ __device__ __forceinline__ void delta_pairs(const MsArgs<OffT>& a, int64_t base,
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           r[k] = hit[k] ? cld(&a.sm[(int64_t)x[k] * 64 + l]) : 0.f;
-          er[k] = hit[k] ? (int)cld(&a.se[(int64_t)x[k] * 64 + l]) : 0;
+          er[k] = hit[k] ? load_exp<kPlain>(a, (int64_t)x[k] * 64 + l) : 0;
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-          if (hit[k]) acc += delta_term(mv, ev, r[k], er[k]);
+          if (hit[k]) acc += delta_term<kPlain>(mv, ev, r[k], er[k]);
       }
-      finish_delta(a, at, acc);
+      finish_delta<kPlain>(a, at, acc);
     }
   }
 }
 
-template<typename OffT>
+template<bool kPlain, typename OffT>
 __device__ __forceinline__ void delta_chunks(const MsArgs<OffT>& a, const HubC* hc, int64_t nc, int64_t lbase,
                                              const uint64_t* Xa, int64_t gwave, int64_t nwaves) {
   const int lane = lane_id();
@@ -949,7 +994,7 @@ __device__ __forceinline__ void delta_chunks(const MsArgs<OffT>& a, const HubC* 
     const bool mine = (own >> lane) & 1ull;
     const int64_t at = (int64_t)h.v * 64 + lane;
     const float mv = mine ? cld(&a.sm[at]) : 0.f;
-    const int ev = mine ? (int)cld(&a.se[at]) : 0;
+    const int ev = mine ? load_exp<kPlain>(a, at) : 0;
     const int64_t s = (int64_t)a.off[h.v] + (int64_t)h.c * kHub;
     const int64_t e = std::min<int64_t>(s + kHub, (int64_t)a.off[h.v + 1]);
     float acc = 0.f;
@@ -959,18 +1004,18 @@ __device__ __forceinline__ void delta_chunks(const MsArgs<OffT>& a, const HubC* 
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         r[k] = hit[k] ? cld(&a.sm[(int64_t)x[k] * 64 + lane]) : 0.f;
-        er[k] = hit[k] ? (int)cld(&a.se[(int64_t)x[k] * 64 + lane]) : 0;
+        er[k] = hit[k] ? load_exp<kPlain>(a, (int64_t)x[k] * 64 + lane) : 0;
       }
 #pragma unroll
       for (int k = 0; k < 8; ++k)
-        if (hit[k]) acc += delta_term(mv, ev, r[k], er[k]);
+        if (hit[k]) acc += delta_term<kPlain>(mv, ev, r[k], er[k]);
     });
     if (c < a.p_cap) cst(&a.pS[c * 64 + lane], acc);
     else if (lane == 0) raise_flag(a.ctl, kOvPart);
   }
 }
 
-template<typename OffT>
+template<bool kPlain, typename OffT>
 __device__ __forceinline__ void delta_combine(const MsArgs<OffT>& a, const HubV* hv, int64_t nv, int64_t lbase,
                                               int64_t gwave, int64_t nwaves) {
   const int lane = lane_id();
@@ -979,7 +1024,7 @@ __device__ __forceinline__ void delta_combine(const MsArgs<OffT>& a, const HubV*
     if (!((cld(&a.lm[lbase + h.pos]) >> lane) & 1ull)) continue;
     float acc = 0.f;
     for (int32_t c = 0; c < h.nch; ++c) acc += cld(&a.pS[((int64_t)h.first + c) * 64 + lane]);
-    finish_delta(a, (int64_t)h.v * 64 + lane, acc);
+    finish_delta<kPlain>(a, (int64_t)h.v * 64 + lane, acc);
   }
 }
 
@@ -1052,11 +1097,15 @@ __device__ __forceinline__ void load_head(unsigned long long* dst, const LevelIn
   if (k >= 0 && k < kLevelInfoZero) dst[k] = atomic_load(reinterpret_cast<const unsigned long long*>(L) + k);
 }
 
-/* three waves per SIMD: the kernel holds a level loop's state, the pair
- * walks and four arcs' loads in flight; left alone the compiler takes 176
- * registers (two waves), which costs the power-law graphs' big levels 7 % */
-template<typename OffT>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) ms_kernel(MsArgs<OffT> a) {
+/* Waves per SIMD: the kernel holds a level loop's state, the pair walks and
+ * four arcs' loads in flight; left alone the compiler takes 176 registers (two
+ * waves), which costs the power-law graphs' big levels 7 %.  MS-BFS and the
+ * batches with exponents fit in three; the plain batches, whose time is row
+ * reads, take five (RMAT scale 20, 64 sources: 12.7 ms with three, 11.1 with
+ * four, 9.8 with five). */
+constexpr int ms_waves(bool bc, bool plain) { return bc && plain ? 5 : 3; }
+template<bool kBc, bool kPlain, typename OffT>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(ms_waves(kBc, kPlain)))) ms_kernel(MsArgs<OffT> a) {
   __shared__ sg::policy::Staged s_pol;
   __shared__ int32_t s_stage[kBlock / 64][kStage];
   __shared__ unsigned long long s_red[2 * (kBlock / 64)];
@@ -1142,7 +1191,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
     int64_t hiv = 0, hic = 0;
     const HubV* hivp = nullptr;
     const HubC* hicp = nullptr;
-    if (a.bc && d >= 1) {
+    if (kBc && d >= 1) {
       hicp = a.directed ? a.hic + (int64_t)h[kHHicBase] : hocp;
       hic = a.directed ? (int64_t)h[kHHic] : hoc;
       hiv = a.directed ? (int64_t)h[kHHiv] : (int64_t)h[kHHov];
@@ -1151,19 +1200,19 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
     if (dir) {
       expand_pull(a, Mc, Mn, nx, nb, st, gwave, nwaves);
     } else {
-      expand_push(a, d, base, cnt, Mc, Mn, nx, nb, st, gwave, nwaves);
+      expand_push(a, d, base, cnt, Mc, Mn, nx, nb, st, gwave, nwaves, (int64_t)(lv_arcs / (unsigned long long)cnt));
       expand_chunks(a, hocp, hoc, Mc, Mn, nx, nb, st, gwave, nwaves);
     }
     stage_finish(a, nx, nb, st, s_red, a.ctl->acc[(d + 1) % 3]);
-    visit_level(a, d, base, cnt, Mc, gwave, nwaves);
+    visit_level<kBc>(a, d, base, cnt, Mc, gwave, nwaves);
     if (d >= 2) clear_level(a, o_base, o_cnt, a.M + (int64_t)((d + 2) & 3) * n, gwave, nwaves);
-    if (a.bc && d >= 1) {
-      sigma_pairs(a, base, cnt, Mc, Mp, gwave, nwaves);
-      sigma_chunks(a, hicp, hic, Mc, Mp, gwave, nwaves);
+    if (kBc && d >= 1) {
+      sigma_pairs<kPlain>(a, base, cnt, Mc, Mp, gwave, nwaves, a.mean);
+      sigma_chunks<kPlain>(a, hicp, hic, Mc, Mp, gwave, nwaves);
     }
     if (!grid_sync(a.ctl, t, a.wait_ticks)) return;
     if (hiv > 0) {
-      sigma_combine(a, hivp, hiv, Mc, gwave, nwaves);
+      sigma_combine<kPlain>(a, hivp, hiv, Mc, gwave, nwaves);
       if (!grid_sync(a.ctl, t, a.wait_ticks)) return;
     }
   }
@@ -1171,7 +1220,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
     a.ctl->levels = d;
     a.ctl->n_pull = n_pull;
   }
-  if (!a.bc) return;
+  if constexpr (!kBc) return;
   /* the partial rows must hold every level's chunks before anything is added
    * to bc (a batch that stops here runs again with more rows) */
   if (max_chunks > a.p_cap) {
@@ -1200,14 +1249,14 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))
     const HubC* hocp = a.hoc + (int64_t)h[kHHocBase];
     const int64_t b1 = (int64_t)s_h[1][kHBase], c1 = (int64_t)s_h[1][kHCount];
     const int64_t b2 = (int64_t)s_h[2][kHBase], c2 = (int64_t)s_h[2][kHCount];
-    delta_pairs(a, base, cnt, Xa, gwave, nwaves);
-    delta_chunks(a, hocp, hoc, base, Xa, gwave, nwaves);
+    delta_pairs<kPlain>(a, base, cnt, Xa, gwave, nwaves, a.mean);
+    delta_chunks<kPlain>(a, hocp, hoc, base, Xa, gwave, nwaves);
     scatter_masks(a, base, cnt, Xb, true, gwave, nwaves);
     if (dd + 2 <= deepest) scatter_masks(a, b2, c2, Xb, false, gwave, nwaves);
     if (dd + 1 <= deepest) accumulate(a, b1, c1, gwave, nwaves);
     if (!grid_sync(a.ctl, t, a.wait_ticks)) return;
     if (hov > 0) {
-      delta_combine(a, hovp, hov, base, gwave, nwaves);
+      delta_combine<kPlain>(a, hovp, hov, base, gwave, nwaves);
       if (!grid_sync(a.ctl, t, a.wait_ticks)) return;
     }
   }
@@ -1244,8 +1293,8 @@ __global__ void __launch_bounds__(64) ms_seed_kernel(MsArgs<OffT> a) {
     atomic_or(&a.vis[s], 1ull << i);
     first = atomic_or(&a.M[s], 1ull << i) == 0ull;
     if (a.bc) {
-      a.sm[(int64_t)s * 64 + i] = 0.5f; /* sigma = 1 = 0.5 * 2^1 */
-      a.se[(int64_t)s * 64 + i] = 1;
+      a.sm[(int64_t)s * 64 + i] = a.plain ? 1.0f : 0.5f; /* sigma = 1 = 0.5 * 2^1 */
+      if (!a.plain) a.se[(int64_t)s * 64 + i] = 1;
     }
   }
   Bases b{0, 0, 0, 0, 0};
@@ -1300,13 +1349,17 @@ int launch_batches(sg_graph_t g, bool bc, int32_t nsrc, const int32_t* sources, 
     caps.hc_cap = chunks_bound;
     caps.li_cap = kLiRing;
   }
-  static int occ = 0; /* per offset width (one instantiation each) */
-  if (occ == 0) {
-    int nb = 0;
-    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, ms_kernel<OffT>, kBlock, 0));
-    occ = std::max(1, std::min(nb, 4));
-  }
-  const int grid = occ * dev->cus;
+  /* MS-BFS; BC with exponents; BC without (per offset width) */
+  const void* const kernels[3] = {reinterpret_cast<const void*>(ms_kernel<false, true, OffT>),
+                                  reinterpret_cast<const void*>(ms_kernel<true, false, OffT>),
+                                  reinterpret_cast<const void*>(ms_kernel<true, true, OffT>)};
+  static int occs[3] = {0, 0, 0};
+  for (int k = 0; k < 3; ++k)
+    if (occs[k] == 0) {
+      int nb = 0;
+      SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernels[k], kBlock, 0));
+      occs[k] = std::max(1, std::min(nb, k == 2 ? 5 : 4));
+    }
   const int grid_n = sg::grid_for(dev, n, kBlock, 8);
 
   if (!bc) {
@@ -1327,6 +1380,8 @@ int launch_batches(sg_graph_t g, bool bc, int32_t nsrc, const int32_t* sources, 
     a.full = k == 64 ? ~0ull : ((1ull << k) - 1ull);
     a.k = k;
     a.bc = bc ? 1 : 0;
+    a.plain = g->msbc_exponents ? 0 : 1;
+    a.mean = n > 0 ? m / n : 0;
     a.ring = bc ? 0 : 1;
     a.directed = (bc && directed) ? 1 : 0;
     a.off = (const OffT*)g->offsets;
@@ -1355,10 +1410,10 @@ int launch_batches(sg_graph_t g, bool bc, int32_t nsrc, const int32_t* sources, 
         SG_TRY(sg::graph_buffer(g, "msb_hic", sizeof(HubC) * (size_t)hcslots, &a.hic));
       }
       SG_TRY(sg::graph_buffer(g, "msb_sm", 4 * 64 * (size_t)(n + 1), &a.sm));
-      SG_TRY(sg::graph_buffer(g, "msb_se", 2 * 64 * (size_t)(n + 1), &a.se));
+      if (!a.plain) SG_TRY(sg::graph_buffer(g, "msb_se", 2 * 64 * (size_t)(n + 1), &a.se));
       SG_TRY(sg::graph_buffer(g, "msb_dl", 4 * 64 * (size_t)(n + 1), &a.dl));
       SG_TRY(sg::graph_buffer(g, "msb_pS", 4 * 64 * (size_t)caps.p_cap, &a.pS));
-      SG_TRY(sg::graph_buffer(g, "msb_pE", 4 * 64 * (size_t)caps.p_cap, &a.pE));
+      if (!a.plain) SG_TRY(sg::graph_buffer(g, "msb_pE", 4 * 64 * (size_t)caps.p_cap, &a.pE));
       a.p_cap = caps.p_cap;
       a.bc64 = bc64;
     } else {
@@ -1377,13 +1432,18 @@ int launch_batches(sg_graph_t g, bool bc, int32_t nsrc, const int32_t* sources, 
     ms_seed_kernel<OffT><<<1, 64, 0, s>>>(a);
     SG_HIP(hipGetLastError());
     void* args[] = {&a};
-    SG_HIP(launch_resident(reinterpret_cast<const void*>(ms_kernel<OffT>), grid, kBlock, args, s));
+    const int which = !bc ? 0 : (a.plain ? 2 : 1);
+    SG_HIP(launch_resident(kernels[which], occs[which] * dev->cus, kBlock, args, s));
     SG_HIP(hipMemcpyAsync(hctl, a.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s));
     SG_HIP(hipStreamSynchronize(s));
     const uint32_t fl = hctl->flags;
     SG_CHECK(!(fl & kTimeout), SG_ERR_HIP, "%s: a grid barrier waited longer than the device's wait limit",
              bc ? "sg_bc_batched" : "sg_bfs_multi");
     SG_CHECK(!(fl & kRange), SG_ERR_UNSUPPORTED, "sg_bc_batched: path counts beyond 2^%d", kExpMax);
+    if (fl & kOvPlain) { /* before anything was added to bc */
+      g->msbc_exponents = true;
+      continue;
+    }
     if (fl & (kOvList | kOvHubV | kOvHubC | kOvPart | kOvLevels)) {
       /* grow what overflowed to its bound and run the batch again (the
        * bounds hold for any batch: each (vertex, lane) pair lies at one depth) */

@@ -183,6 +183,17 @@ __device__ __forceinline__ int scan_owner(uint32_t incl, uint32_t t) {
   return (int)lo;
 }
 
+/* Entries a wave takes at a time from a list of cnt: 64, halved (to no fewer
+ * than 8) while the list would leave waves of the grid without any and a
+ * wave's share keeps 256 arcs, by the mean of `arcs` arcs per entry.  A few
+ * thousand lists of a hundred arcs otherwise keep a few dozen waves busy for
+ * tens of steps each; short lists (grids) gain nothing from more waves. */
+__device__ __forceinline__ int group_entries(int64_t cnt, int64_t nwaves, int64_t arcs) {
+  int g = 64;
+  while (g > 8 && cnt <= nwaves * (g / 2) && arcs * (g / 2) >= 256) g >>= 1;
+  return g;
+}
+
 /* The arc range [s, e) of vertex v in one load (its two offsets are adjacent;
  * global loads need only 4-byte alignment). */
 __device__ __forceinline__ void list_bounds(const int64_t* off, uint32_t v, int64_t& s, int64_t& e) {
@@ -638,6 +649,7 @@ template<typename OffT, typename Visit4>
 __device__ __forceinline__ void for_each_queued_arc4(QEntry* const q[3], const QueueHdr* hdr, const int32_t* cols,
                                                      Visit4&& visit4, int variant = 0) {
   const uint32_t n_small = hdr->count[0], n_med = hdr->count[1], n_large = hdr->count[2];
+  const int64_t mean = hdr->nvert ? (int64_t)(hdr->deg / hdr->nvert) : 0; /* arcs per entry, of the queued vertices */
   const int lane = lane_id();
   const int wave_in_block = threadIdx.x >> 6;
   const int64_t gwave = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
@@ -669,13 +681,14 @@ __device__ __forceinline__ void for_each_queued_arc4(QEntry* const q[3], const Q
   for (int cls = 0; cls < (variant == 1 ? 2 : 1); ++cls) {
     const QEntry* qq = q[cls];
     const uint32_t cnt = cls == 0 ? n_small : n_med;
-    for (int64_t base = gwave * 64; base < cnt; base += nwaves * 64) {
+    const int group = group_entries(cnt, nwaves, mean);
+    for (int64_t base = gwave * group; base < cnt; base += nwaves * group) {
       const int64_t i = base + lane;
       QEntry qe;
       qe.start = 0;
       qe.v = 0;
       qe.len = 0;
-      if (i < cnt) qe = qq[i];
+      if (lane < group && i < cnt) qe = qq[i];
       const uint32_t incl = wave_inclusive_scan((uint32_t)qe.len);
       const uint32_t total = wave_lane(incl, 63);
       const uint32_t excl = incl - (uint32_t)qe.len;
@@ -700,6 +713,7 @@ template<typename OffT, typename Visit>
 __device__ __forceinline__ void for_each_queued_arc(QEntry* const q[3], const QueueHdr* hdr, const int32_t* cols,
                                                     Visit&& visit, int variant = 0) {
   const uint32_t n_small = hdr->count[0], n_med = hdr->count[1], n_large = hdr->count[2];
+  const int64_t mean = hdr->nvert ? (int64_t)(hdr->deg / hdr->nvert) : 0; /* arcs per entry, of the queued vertices */
   const int lane = lane_id();
   const int wave_in_block = threadIdx.x >> 6;
   const int64_t gwave = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
@@ -734,13 +748,14 @@ __device__ __forceinline__ void for_each_queued_arc(QEntry* const q[3], const Qu
   for (int cls = 0; cls < (variant == 1 ? 2 : 1); ++cls) {
     const QEntry* qq = q[cls];
     const uint32_t cnt = cls == 0 ? n_small : n_med;
-    for (int64_t base = gwave * 64; base < cnt; base += nwaves * 64) {
+    const int group = group_entries(cnt, nwaves, mean);
+    for (int64_t base = gwave * group; base < cnt; base += nwaves * group) {
       const int64_t i = base + lane;
       QEntry qe;
       qe.start = 0;
       qe.v = 0;
       qe.len = 0;
-      if (i < cnt) qe = qq[i];
+      if (lane < group && i < cnt) qe = qq[i];
       const uint32_t incl = wave_inclusive_scan((uint32_t)qe.len);
       const uint32_t total = wave_lane(incl, 63);
       for (uint32_t t0 = 0; t0 < total; t0 += 64) {

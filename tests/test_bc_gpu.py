@@ -157,10 +157,13 @@ def test_bfs_multi_matches_oracle(sg, device, oracle_mod):
 
 @pytest.mark.parametrize("levels", [30, 200, 1500])
 @pytest.mark.parametrize("directed", [False, True])
-def test_bc_level_grouping_and_hubs(sg, device, oracle_mod, levels, directed):
+@pytest.mark.parametrize("batched", [False, True])
+def test_bc_level_grouping_and_hubs(sg, device, oracle_mod, levels, directed, batched):
     """Level counts on each side of the level grouping's limits (64 levels with bitmaps written by the
     counting pass, 1,024 counted, more sorted), rungs of several shortest paths, and hubs of 700 arcs
-    (a workgroup's share) in the middle and at the end."""
+    (a workgroup's share) in the middle and at the end.  Path counts grow like 1.6^level, so the batched
+    form takes 30 levels without exponents, meets its limit of 2^100 at 200 and starts again with them;
+    a second call on the same graph adds the same sums."""
     a = np.arange(levels - 1)
     u = np.concatenate([2 * a, 2 * a, 2 * a + 1, np.full(700, levels), np.full(700, 2 * levels - 1)])
     v = np.concatenate([2 * a + 2, 2 * a + 3, 2 * a + 2, 2 * levels + np.arange(700), 2 * levels + np.arange(700)])
@@ -175,4 +178,9 @@ def test_bc_level_grouping_and_hubs(sg, device, oracle_mod, levels, directed):
         g = oracle_mod.csr_from_pairs(n, u, v)
         ref = oracle_mod.bc(g, [0, 4])
     G = sg.Graph.from_csr(device, g.offsets, g.cols, directed=directed)
-    assert _close(_bc(sg, G, [0, 4]), ref)
+    b = sg.BC(G)
+    b.init([0, 4])
+    b.run(batched=batched)
+    assert _close(b.get_values(), ref)
+    b.run(batched=batched)
+    assert _close(b.get_values(), 2.0 * ref)
