@@ -306,7 +306,8 @@ typedef struct sg_level_stat {
                                 decision and queue write, and the burst of small levels if one ran */
   int32_t burst;             /* 1: the level ran inside a single-workgroup burst of small push levels,
                                 timed in convert_ms of the level before it; the level at which a burst
-                                stops is counted and decided by the next step, whose times it carries */
+                                stops is counted and decided by the next step, whose times it carries
+                                (a small graph traversed in one launch: the first level's kernel_ms) */
 } sg_level_stat;
 
 typedef struct sg_bfs_stats {

@@ -390,11 +390,28 @@ __device__ __forceinline__ void stage_policy(const DecideParams& p, sg::policy::
  * cleared, and (thread 0) the F0 queue = {src} and the control block for
  * level 0. */
 template<typename OffT>
-__global__ void bfs_start_kernel(BfsArgs<OffT> a, uint64_t* prev, const uint64_t* isolated,
-                                 unsigned long long* stat_words, int64_t n_stat_words, QEntry* q0, QEntry* q1,
-                                 QEntry* q2, QueueHdr* hdr, Tuning t, int32_t src, BfsCtl* ctl, int32_t first_dir,
-                                 int32_t first_lb, int64_t burst_arcs) {
-  const int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+struct StartArgs {
+  BfsArgs<OffT> a;
+  uint64_t* prev;
+  const uint64_t* isolated;
+  unsigned long long* stat_words;
+  int64_t n_stat_words;
+  QEntry* q[3];
+  QueueHdr* hdr;
+  Tuning t;
+  int32_t src, first_dir, first_lb;
+  int64_t burst_arcs;
+};
+template<typename OffT>
+__device__ __forceinline__ void start_body(const StartArgs<OffT>& s, BfsCtl* ctl, int64_t tid, int64_t stride) {
+  const BfsArgs<OffT>& a = s.a;
+  uint64_t* prev = s.prev;
+  const uint64_t* isolated = s.isolated;
+  unsigned long long* stat_words = s.stat_words;
+  const int64_t n_stat_words = s.n_stat_words, burst_arcs = s.burst_arcs;
+  QueueHdr* hdr = s.hdr;
+  const Tuning& t = s.t;
+  const int32_t src = s.src, first_dir = s.first_dir, first_lb = s.first_lb;
   const int64_t sw = src >> 6;
   const uint64_t bit = 1ull << (src & 63);
   for (int64_t i = tid; i < a.n; i += stride) a.depth[i] = i == src ? 0 : (int32_t)(a.n + 1);
@@ -406,8 +423,7 @@ __global__ void bfs_start_kernel(BfsArgs<OffT> a, uint64_t* prev, const uint64_t
   }
   for (int64_t i = tid; i < n_stat_words; i += stride) stat_words[i] = 0ull;
   if (tid != 0) return;
-  QEntry* const q[3] = {q0, q1, q2};
-  enqueue_single(a.off, t, q, hdr, src);
+  enqueue_single(a.off, t, s.q, hdr, src);
   const unsigned long long d = (unsigned long long)(a.off[src + 1] - a.off[src]);
   BfsCtl c{};
   c.dir = first_dir;
@@ -420,6 +436,11 @@ __global__ void bfs_start_kernel(BfsArgs<OffT> a, uint64_t* prev, const uint64_t
    * ahead of the first step) */
   c.burst = (first_dir == 0 && burst_arcs > 0 && (int64_t)d <= burst_arcs) ? 1 : 0;
   *ctl = c;
+}
+
+template<typename OffT>
+__global__ void bfs_start_kernel(StartArgs<OffT> s, BfsCtl* ctl) {
+  start_body(s, ctl, blockIdx.x * (int64_t)blockDim.x + threadIdx.x, (int64_t)gridDim.x * blockDim.x);
 }
 
 /* The traversal of one level, push or pull as the control block says.  Four
@@ -632,6 +653,10 @@ struct BurstArgs {
   QueueHdr* hdr;
   QEntry* list[2][2]; /* burst frontier lists [parity][small / big], kBurstMaxArcs entries each */
   Tuning tune;
+  /* small graphs: both bitmaps in LDS (32-bit words), where the claims of a
+   * whole level on a few words do not queue at one cache line */
+  uint32_t* lds_visited;
+  uint32_t* lds_prev;
 };
 
 struct BurstAcc {
@@ -646,7 +671,7 @@ constexpr int kBurstPiece = 256;  /* arcs per piece of a big list: four per lane
  * counter update per wave and list for all four, then the stores.  A
  * discovery gets depth level + 1 and goes to the small or the big list of the
  * next level by its degree. */
-template<typename OffT>
+template<bool kLds, typename OffT>
 __device__ __forceinline__ void burst_claim4(const BurstArgs<OffT>& a, const uint32_t (&y)[4], const bool (&ok)[4],
                                              int32_t level, QEntry* out_small, QEntry* out_big, uint32_t* cnt2,
                                              BurstAcc& acc) {
@@ -658,7 +683,8 @@ __device__ __forceinline__ void burst_claim4(const BurstArgs<OffT>& a, const uin
     old[k] = ~0ull;
     vs[k] = ve[k] = 0;
     if (ok[k]) {
-      old[k] = atomic_or(&a.visited[y[k] >> 6], 1ull << (y[k] & 63));
+      if (kLds) old[k] = (uint64_t)atomicOr(&a.lds_visited[y[k] >> 5], 1u << (y[k] & 31)) << (y[k] & 32);
+      else old[k] = atomic_or(&a.visited[y[k] >> 6], 1ull << (y[k] & 63));
       vs[k] = (int64_t)a.off[y[k]];
       ve[k] = (int64_t)a.off[y[k] + 1];
     }
@@ -707,7 +733,7 @@ __device__ __forceinline__ void burst_claim4(const BurstArgs<OffT>& a, const uin
 
 /* Short lists: a wave lays 64 entries end to end (merge path) and takes four
  * arcs per lane per round; waves take groups of 64 entries in turn. */
-template<typename OffT>
+template<bool kLds, typename OffT>
 __device__ __forceinline__ void burst_visit_small(const BurstArgs<OffT>& a, const QEntry* ents, uint32_t cnt,
                                                   int32_t level, QEntry* out_small, QEntry* out_big, uint32_t* cnt2,
                                                   BurstAcc& acc) {
@@ -733,7 +759,7 @@ __device__ __forceinline__ void burst_visit_small(const BurstArgs<OffT>& a, cons
         ok[k] = t < total;
         y[k] = ok[k] ? (uint32_t)a.cols[st + (t - before)] : 0u;
       }
-      burst_claim4(a, y, ok, level, out_small, out_big, cnt2, acc);
+      burst_claim4<kLds>(a, y, ok, level, out_small, out_big, cnt2, acc);
     }
   }
 }
@@ -741,7 +767,7 @@ __device__ __forceinline__ void burst_visit_small(const BurstArgs<OffT>& a, cons
 /* Long lists: every list is cut into pieces of kBurstPiece arcs, and the
  * pieces of the level go to the waves in turn, so one hub keeps every wave
  * busy. */
-template<typename OffT>
+template<bool kLds, typename OffT>
 __device__ __forceinline__ void burst_visit_big(const BurstArgs<OffT>& a, const QEntry* ents, uint32_t cnt,
                                                 int32_t level, QEntry* out_small, QEntry* out_big, uint32_t* cnt2,
                                                 BurstAcc& acc) {
@@ -762,7 +788,7 @@ __device__ __forceinline__ void burst_visit_big(const BurstArgs<OffT>& a, const 
         ok[k] = o < qe.len;
         y[k] = ok[k] ? (uint32_t)a.cols[qe.start + o] : 0u;
       }
-      burst_claim4(a, y, ok, level, out_small, out_big, cnt2, acc);
+      burst_claim4<kLds>(a, y, ok, level, out_small, out_big, cnt2, acc);
     }
     pbase += np;
   }
@@ -772,7 +798,7 @@ __device__ __forceinline__ void burst_visit_big(const BurstArgs<OffT>& a, const 
  * buffered by level parity, so a wave may start the next level while others
  * still read this level's sums; every wave evaluates the (deterministic)
  * decision itself. */
-template<typename OffT>
+template<bool kLds, typename OffT>
 __device__ __forceinline__ void burst_body(const BurstArgs<OffT>& a, BfsCtl* ctl, const DecideParams& p,
                                            int32_t step, LevelLog* levlog, StepLog* steplog, bool publish) {
   __shared__ sg::policy::Staged s_pol;
@@ -796,18 +822,19 @@ __device__ __forceinline__ void burst_body(const BurstArgs<OffT>& a, BfsCtl* ctl
     QEntry* out_small = a.list[cur ^ 1][0];
     QEntry* out_big = a.list[cur ^ 1][1];
     if (it == 0) { /* the queues: class 0 lists are short, classes 1 and 2 long */
-      burst_visit_small(a, a.q[0], h0.count[0], level, out_small, out_big, s_count[par], acc);
-      burst_visit_big(a, a.q[1], h0.count[1], level, out_small, out_big, s_count[par], acc);
-      burst_visit_big(a, a.q[2], h0.count[2], level, out_small, out_big, s_count[par], acc);
+      burst_visit_small<kLds>(a, a.q[0], h0.count[0], level, out_small, out_big, s_count[par], acc);
+      burst_visit_big<kLds>(a, a.q[1], h0.count[1], level, out_small, out_big, s_count[par], acc);
+      burst_visit_big<kLds>(a, a.q[2], h0.count[2], level, out_small, out_big, s_count[par], acc);
     } else {
       /* the previous burst level's discoveries join prev (fire and forget:
        * nothing in the burst reads prev) */
       for (uint32_t i = threadIdx.x; i < n_small + n_big; i += kBurstThreads) {
         const uint32_t v = (uint32_t)(i < n_small ? a.list[cur][0][i] : a.list[cur][1][i - n_small]).v;
-        atomic_or(&a.prev[v >> 6], 1ull << (v & 63));
+        if (kLds) atomicOr(&a.lds_prev[v >> 5], 1u << (v & 31));
+        else atomic_or(&a.prev[v >> 6], 1ull << (v & 63));
       }
-      burst_visit_small(a, a.list[cur][0], n_small, level, out_small, out_big, s_count[par], acc);
-      burst_visit_big(a, a.list[cur][1], n_big, level, out_small, out_big, s_count[par], acc);
+      burst_visit_small<kLds>(a, a.list[cur][0], n_small, level, out_small, out_big, s_count[par], acc);
+      burst_visit_big<kLds>(a, a.list[cur][1], n_big, level, out_small, out_big, s_count[par], acc);
     }
     acc.disc = wave_sum_u64(acc.disc);
     acc.deg = wave_sum_u64(acc.deg);
@@ -907,7 +934,52 @@ template<typename OffT>
 __global__ void __launch_bounds__(kBurstThreads) burst_kernel(BurstArgs<OffT> a, BfsCtl* ctl, DecideParams p,
                                                               int32_t step, LevelLog* levlog, StepLog* steplog) {
   if (ctl->done || !ctl->burst) return;
-  burst_body(a, ctl, p, step, levlog, steplog, false);
+  burst_body<false>(a, ctl, p, step, levlog, steplog, false);
+}
+
+/* A graph of at most kSmallArcs arcs and vertices that starts by pushing: the
+ * start and the burst in one launch of one workgroup, whose record the host
+ * waits for before it enqueues anything else.  The burst takes every level
+ * the policy pushes (a burst list fits the whole graph), so a pushing
+ * traversal ends here.  Bound by the rounds' latency: 1,024 vertices of 12
+ * arcs in seven launches and more, the trailing steps' no-ops included, took
+ * 154 us; in this one with the claims at L2, where sixteen words took them
+ * all, 127; with the bitmaps in LDS 69.  The line lies at the capacity of a
+ * burst list, below which every graph tried was faster here: RMAT of 52,628
+ * arcs 198 -> 163 us, 53,982 random arcs 286 -> 158, a 100 x 110 grid
+ * 855 -> 692 (pushing) and 1326 -> 1220 (alternating). */
+constexpr int64_t kSmallArcs = kBurstMaxArcs;
+template<typename OffT>
+__global__ void __launch_bounds__(kBurstThreads) small_kernel(StartArgs<OffT> s, BurstArgs<OffT> a, BfsCtl* ctl,
+                                                              DecideParams p, int32_t step, LevelLog* levlog,
+                                                              StepLog* steplog) {
+  __shared__ uint32_t s_visited[kSmallArcs / 32], s_prev[kSmallArcs / 32];
+  start_body(s, ctl, threadIdx.x, kBurstThreads);
+  const int words = (int)(2 * s.a.w0);
+  const uint32_t* isolated = reinterpret_cast<const uint32_t*>(s.isolated);
+  for (int i = threadIdx.x; i < words; i += kBurstThreads)
+    s_visited[i] = s_prev[i] = isolated[i] | (i == s.src >> 5 ? 1u << (s.src & 31) : 0u);
+  a.lds_visited = s_visited;
+  a.lds_prev = s_prev;
+  wait_stores_complete();
+  __syncthreads();
+  if (!ctl->burst) { /* not a pushing start */
+    if (threadIdx.x == 0) {
+      StepLog sl{};
+      sl.step = step;
+      publish_step(&steplog[step % kRing], sl);
+    }
+    return;
+  }
+  burst_body<true>(a, ctl, p, step, levlog, steplog, true);
+  /* what a handed-back level's count pass reads (after this launch) */
+  __syncthreads();
+  uint32_t* visited = reinterpret_cast<uint32_t*>(a.visited);
+  uint32_t* prev = reinterpret_cast<uint32_t*>(a.prev);
+  for (int i = threadIdx.x; i < words; i += kBurstThreads) {
+    visited[i] = s_visited[i];
+    prev[i] = s_prev[i];
+  }
 }
 
 /* Queue write of a level that the next one pushes.  A workgroup of
@@ -926,7 +998,7 @@ __global__ void __launch_bounds__(kBurstThreads) write_dyn_kernel(CompactArgs<Of
       compact_write_body_at<OffT>(a, 0, (int64_t)blockIdx.x * 2 + (threadIdx.x >> 8), (int)(threadIdx.x & (kBlock - 1)));
   /* a burst level has at most burst_arcs arcs, so few waves write entries and publish them */
   if (!burst || !last_to_arrive<false>(arrive, wrote)) return;
-  burst_body(ba, ctl, p, step, levlog, steplog, true);
+  burst_body<false>(ba, ctl, p, step, levlog, steplog, true);
 }
 
 /* ------------------------------------------------------- grid bursts --- */
@@ -1515,10 +1587,13 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
 
   /* work-mapping variant under the fixed policies (see sg_bfs_options) */
   const int32_t lb_fixed = opt.load_balancer == SG_LB_WORKGROUP ? 1 : (opt.load_balancer == SG_LB_SUBGROUP ? 2 : 0);
-  const int64_t burst_arcs = opt.burst_arcs < 0 ? 0 : (opt.burst_arcs == 0 ? kBurstDefaultArcs : opt.burst_arcs);
+  const bool small = opt.burst_arcs == 0 && opt.grid_burst_arcs <= 0 && g->m <= kSmallArcs && n <= kSmallArcs &&
+                     opt.policy != SG_POLICY_PULL;
+  const int64_t burst_arcs =
+      opt.burst_arcs < 0 ? 0 : (opt.burst_arcs != 0 ? opt.burst_arcs : (small ? kSmallArcs : kBurstDefaultArcs));
   const int64_t gb_arcs = opt.grid_burst_arcs < 0 ? 0 : (opt.grid_burst_arcs == 0 ? kGbDefaultArcs : opt.grid_burst_arcs);
   int gb_grid = 0, gb_stride = 1;
-  if (gb_arcs > 0 && opt.policy != SG_POLICY_PULL) {
+  if (gb_arcs > 0 && opt.policy != SG_POLICY_PULL && !small) { /* a small graph's levels all fit a burst */
     static int occ = 0; /* per offset width (one instantiation each) */
     if (occ == 0) {
       int nb = 0;
@@ -1530,10 +1605,20 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
     gb_stride = gp.stride;
     SG_TRY(gb_buffers(g, ws, gb_arcs, gb_grid));
   }
-  bfs_start_kernel<OffT><<<sg::grid_for(dev, n, 256, 4), 256, 0, s>>>(
-      a, ws->prev, g->isolated, reinterpret_cast<unsigned long long*>(ws->stats),
-      (int64_t)(sizeof(StatSlot) * kSlots * 2 / 8), Q.q[0][0], Q.q[0][1], Q.q[0][2], Q.hdr, tune, src, ws->ctl,
-      opt.policy == SG_POLICY_PULL ? 1 : 0, opt.policy == SG_POLICY_LEARNED ? 0 : lb_fixed, burst_arcs);
+  StartArgs<OffT> start{};
+  start.a = a;
+  start.prev = ws->prev;
+  start.isolated = g->isolated;
+  start.stat_words = reinterpret_cast<unsigned long long*>(ws->stats);
+  start.n_stat_words = (int64_t)(sizeof(StatSlot) * kSlots * 2 / 8);
+  for (int k = 0; k < 3; ++k) start.q[k] = Q.q[0][k];
+  start.hdr = Q.hdr;
+  start.t = tune;
+  start.src = src;
+  start.first_dir = opt.policy == SG_POLICY_PULL ? 1 : 0;
+  start.first_lb = opt.policy == SG_POLICY_LEARNED ? 0 : lb_fixed;
+  start.burst_arcs = burst_arcs;
+  if (!small) bfs_start_kernel<OffT><<<sg::grid_for(dev, n, 256, 4), 256, 0, s>>>(start, ws->ctl);
   SG_HIP(hipGetLastError());
 
   const bool timed = opt.record_levels && stats;
@@ -1626,20 +1711,59 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
   /* no record of an earlier traversal may pass for one of this one (the
    * stream is idle: the previous call ended with a synchronize) */
   for (int k = 0; k < kRing; ++k) __atomic_store_n(&ws->steplog[k].step, -1, __ATOMIC_RELEASE);
+  StepLog last{};
+  int32_t first_level = 0;
+  /* the records of levels first_level .. last.last_level; the times are the
+   * first one's (the step's later levels ran in a burst, timed with the count
+   * and write) */
+  auto take_levels = [&](float k_ms, float c_ms) {
+    for (int32_t L = first_level; stats && L <= last.last_level && L < SG_MAX_LEVELS_RECORDED; ++L) {
+      LevelLog e;
+      std::memcpy(&e, (const void*)&ws->levlog[L], sizeof(e));
+      sg_level_stat& ls = stats->level[L];
+      std::memset(&ls, 0, sizeof(ls));
+      ls.direction = e.dir;
+      ls.load_balancer = opt.load_balancer;
+      ls.frontier_vertices = e.f_vertices;
+      ls.frontier_edges = e.f_edges;
+      ls.discovered = e.disc;
+      ls.edges_inspected = e.edges;
+      ls.vertices_scanned = e.scanned;
+      ls.hint_misses = e.misses;
+      ls.max_degree = e.max_deg;
+      ls.unexplored_edges = e.unexplored;
+      ls.action = e.action;
+      ls.burst = e.burst;
+      if (L == first_level) {
+        ls.kernel_ms = k_ms;
+        ls.convert_ms = c_ms;
+      }
+    }
+  };
   /* a start in a burst: the levels from the source while they stay small,
    * handed back to step 0 (which then only counts and decides) or ending the
    * traversal; the kernel returns at once unless init set ctl->burst */
-  if (burst_arcs > 0 && opt.policy != SG_POLICY_PULL)
+  if (small) {
+    small_kernel<OffT><<<1, kBurstThreads, 0, s>>>(start, burst_args(0), ws->ctl, P, kRing - 1, ws->levlog, ws->steplog);
+    SG_HIP(hipGetLastError());
+    SG_TRY(sg::wait_host_flag(&ws->steplog[kRing - 1].step, kRing - 1, s, "sg_bfs"));
+    std::memcpy(&last, (const void*)&ws->steplog[kRing - 1], sizeof(last));
+    /* the slot is step kRing - 1's again */
+    __atomic_store_n(&ws->steplog[kRing - 1].step, -1, __ATOMIC_RELEASE);
+    if (last.done) take_levels(0.f, 0.f);
+  } else if (burst_arcs > 0 && opt.policy != SG_POLICY_PULL) {
     burst_kernel<OffT><<<1, kBurstThreads, 0, s>>>(burst_args(0), ws->ctl, P, 0, ws->levlog, ws->steplog);
-  SG_TRY(enqueue(0, false));
-  for (int k = 1; k <= lookahead; ++k) SG_TRY(enqueue(k, false));
-  StepLog last{};
-  int32_t first_level = 0;
+  }
+  const bool one_launch = last.done;
+  if (!one_launch) {
+    SG_TRY(enqueue(0, false));
+    for (int k = 1; k <= lookahead; ++k) SG_TRY(enqueue(k, false));
+  }
   /* steps in a row that left a push level of at most gb_arcs arcs (and more
    * than a single-workgroup burst takes) for the next step; from two on, the
    * steps enqueued start with a grid burst */
   int32_t small_push = 0;
-  for (int32_t step = 0;; ++step) {
+  for (int32_t step = 0; !last.done; ++step) {
     const int r = step % kRing;
     if (timed) SG_HIP(hipEventSynchronize(ws->ev_done[r]));
     else SG_TRY(sg::wait_host_flag(&ws->steplog[r].step, step, s, "sg_bfs"));
@@ -1655,36 +1779,13 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
                     last.last_level);
       return SG_ERR_STATE;
     }
-    if (stats) {
-      float k_ms = 0.f, c_ms = 0.f;
-      if (timed) {
-        const hipEvent_t start = step == 0 ? ws->ev_first : ws->ev_done[(step + kRing - 1) % kRing];
-        SG_HIP(hipEventElapsedTime(&k_ms, start, ws->ev_mid[r]));
-        SG_HIP(hipEventElapsedTime(&c_ms, ws->ev_mid[r], ws->ev_done[r]));
-      }
-      for (int32_t L = first_level; L <= last.last_level && L < SG_MAX_LEVELS_RECORDED; ++L) {
-        LevelLog e;
-        std::memcpy(&e, (const void*)&ws->levlog[L], sizeof(e));
-        sg_level_stat& ls = stats->level[L];
-        std::memset(&ls, 0, sizeof(ls));
-        ls.direction = e.dir;
-        ls.load_balancer = opt.load_balancer;
-        ls.frontier_vertices = e.f_vertices;
-        ls.frontier_edges = e.f_edges;
-        ls.discovered = e.disc;
-        ls.edges_inspected = e.edges;
-        ls.vertices_scanned = e.scanned;
-        ls.hint_misses = e.misses;
-        ls.max_degree = e.max_deg;
-        ls.unexplored_edges = e.unexplored;
-        ls.action = e.action;
-        ls.burst = e.burst;
-        if (L == first_level) { /* the step's later levels ran in a burst, timed with the count and write */
-          ls.kernel_ms = k_ms;
-          ls.convert_ms = c_ms;
-        }
-      }
+    float k_ms = 0.f, c_ms = 0.f;
+    if (timed) {
+      const hipEvent_t from = step == 0 ? ws->ev_first : ws->ev_done[(step + kRing - 1) % kRing];
+      SG_HIP(hipEventElapsedTime(&k_ms, from, ws->ev_mid[r]));
+      SG_HIP(hipEventElapsedTime(&c_ms, ws->ev_mid[r], ws->ev_done[r]));
     }
+    take_levels(k_ms, c_ms);
     if (last.done) break;
     if ((int64_t)last.last_level + 1 >= n + 1) { /* more levels than vertices: the control block is corrupt */
       SG_HIP(hipStreamSynchronize(s));
@@ -1710,6 +1811,9 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
     float ms = 0.f;
     SG_HIP(hipEventElapsedTime(&ms, ws->ev_begin, ws->ev_end));
     stats->kernel_ms = ms;
+    /* one launch took every level: its time stands at the first, with no
+     * events around it that the call would wait for */
+    if (timed && one_launch) stats->level[0].kernel_ms = ms;
     stats->levels = last.last_level + 1;
     stats->n_push = last.n_push;
     stats->n_pull = last.n_pull;

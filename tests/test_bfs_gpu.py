@@ -424,3 +424,37 @@ def test_grid_burst_workgroups_and_list_lengths(sg, device, oracle_mod, workgrou
                                  for x in st.level[:st.levels]]))
         assert (sum(x.burst == 2 for x in st.level[:st.levels]) > levels // 2) == (grid >= 0)
     assert runs[0][0] == levels and runs[1] == runs[0] and runs[2] == runs[0]
+
+
+@pytest.mark.parametrize("directed", [False, True])
+@pytest.mark.parametrize("n,arcs", [(1, 0), (2, 2), (63, 200), (64, 900), (65, 65), (1000, 65536), (1000, 65537),
+                                    (65536, 60000), (65537, 60000), (4000, 30000)])
+def test_small_graph_in_one_launch(sg, device, oracle_mod, n, arcs, directed):
+    """Graphs at the edges of a bitmap word and on both sides of the largest that one launch takes: the
+    oracle's depths and the level records of the levels run on their own, for traversals that stay
+    pushing and for those that are handed back for a pull, from a vertex with arcs and from the last."""
+    rng = np.random.default_rng(7 + n + arcs)
+    if directed:
+        key = np.sort(rng.choice(n * n, arcs, replace=False))
+        off = np.concatenate([[0], np.cumsum(np.bincount(key // n, minlength=n))]).astype(np.int64)
+        g = oracle_mod.CSRGraph(n, off, (key % n).astype(np.int32))
+    else:
+        pairs = rng.choice(n * (n - 1) // 2, arcs // 2, replace=False) if arcs else np.zeros(0, dtype=np.int64)
+        v = ((1 + np.sqrt(1 + 8 * pairs.astype(np.float64))) / 2).astype(np.int64)
+        v += (v * (v + 1) // 2 <= pairs).astype(np.int64) - (v * (v - 1) // 2 > pairs).astype(np.int64)
+        g = oracle_mod.csr_from_pairs(n, v, pairs - v * (v - 1) // 2)
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, directed=directed)
+    for src in {int(np.argmax(np.diff(g.offsets))), n - 1}:
+        ref, _ = oracle_mod.bfs(g, src)
+        for policy in (sg.POLICY_PUSH, sg.POLICY_HYBRID):
+            runs = []
+            for tuning in ({}, {}, {"burst_arcs": -1, "grid_burst_arcs": -1}):
+                b = sg.BFS(G)
+                b.init(src)
+                st = b.run(policy, tuning=tuning, record_levels=not runs)
+                assert np.array_equal(b.get_distances(), ref), (src, policy, tuning)
+                runs.append((st.levels, st.reached_vertices, st.reached_edges,
+                             [(x.direction, x.frontier_vertices, x.frontier_edges, x.discovered, x.unexplored_edges)
+                              for x in st.level[:st.levels]]))
+            assert runs[0] == runs[2] and runs[1] == runs[2], (src, policy)
+    G.destroy()
