@@ -388,7 +388,9 @@ typedef struct sg_sssp_options {
                             relaxations buckets save, on sparse long-diameter ones such as grids
                             buckets multiply the iterations.  Below 2^25 arcs, rounds of at most 2^17
                             arcs run back to back in one launch, where putting off the farther
-                            vertices pays: fewer relaxations, other rounds), negative or infinite =
+                            vertices pays: fewer relaxations, other rounds; a graph of at most
+                            16,384 vertices and 2^17 arcs takes every round in one launch of one
+                            workgroup, nothing put off), negative or infinite =
                             none, i.e. every dirty vertex is relaxed each round (the reference's
                             frontier Bellman-Ford, sssp.hpp:152-210) */
   int32_t heavy_pull;    /* direction of a bucket's heavy round on an undirected graph: 0 = automatic

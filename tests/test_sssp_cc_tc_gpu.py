@@ -546,6 +546,46 @@ def test_sssp_grid_bursts(sg, device, oracle_mod, offset_bytes, kind, weight_flo
     assert np.array_equal(got[0].view(np.uint32), got[2].view(np.uint32))
 
 
+@pytest.mark.parametrize("weight_float", [False, True])
+@pytest.mark.parametrize("n,arcs,hubs", [(1, 0, ()), (2, 1, ()), (64, 100, ()), (65, 500, ()), (3000, 9000, (256, 257, 2900)),
+                                         (16384, 40000, (512, 513)), (16385, 40000, ()), (700, 65536, ()),
+                                         (700, 65537, ()), (9000, 2000, (300, 4097))])
+def test_sssp_small_graph_in_one_launch(sg, device, oracle_mod, n, arcs, hubs, weight_float):
+    """Graphs at the edges of a bitmap word and on both sides of the largest that one launch takes, with
+    lists on both sides of the ones cut into pieces: the oracle's distances from the vertex with most arcs
+    and from the last (zero weights among them), directed and not, and records that add up."""
+    rng = np.random.default_rng(n + arcs)
+    pairs = rng.choice(n * (n - 1) // 2, arcs, replace=False) if arcs else np.zeros(0, dtype=np.int64)
+    v = ((1 + np.sqrt(1 + 8 * pairs.astype(np.float64))) / 2).astype(np.int64)
+    v += (v * (v + 1) // 2 <= pairs).astype(np.int64) - (v * (v - 1) // 2 > pairs).astype(np.int64)
+    u = pairs - v * (v - 1) // 2
+    for k, d in enumerate(hubs):
+        u, v = np.concatenate([u, np.full(d, k)]), np.concatenate([v, k + 1 + rng.choice(n - k - 1, d, replace=False)])
+    und = oracle_mod.csr_from_pairs(n, u, v)
+    src, dst = np.repeat(np.arange(n), np.diff(und.offsets)), und.cols
+    one_way = (src < dst) == ((src + dst) % 2 == 0)
+    off = np.concatenate([[0], np.cumsum(np.bincount(src[one_way], minlength=n))]).astype(np.int64)
+    for g, directed in ((und, False), (oracle_mod.CSRGraph(n, off, dst[one_way]), True)):
+        key = np.minimum(np.repeat(np.arange(n), np.diff(g.offsets)), g.cols) * n + np.maximum(
+            np.repeat(np.arange(n), np.diff(g.offsets)), g.cols)
+        w = (key * 2654435761 % 2**32 % 8).astype(np.uint32)
+        G = sg.Graph.from_csr(device, g.offsets, g.cols, weights=w.astype(np.float32) if weight_float else w,
+                              weight_float=weight_float, directed=directed, offset_bytes=4 if n % 2 else 8)
+        for source in {int(np.argmax(np.diff(g.offsets))), n - 1}:
+            ref = oracle_mod.sssp(g, source, w)
+            for _ in range(2):
+                s = sg.SSSP(G)
+                s.init(source)
+                st = s.run()
+                assert np.array_equal(s.get_distances(), ref), (directed, source)
+                assert st.reached_vertices == (ref != n + 1).sum()
+                assert st.reached_edges == np.diff(g.offsets)[ref != n + 1].sum() <= st.relaxations
+                if n <= 16384 and g.m <= 1 << 17:
+                    assert sum(st.round_edges[:st.rounds]) == st.relaxations
+                    assert st.round_vertices[0] == 1 and min(st.round_vertices[:st.rounds]) > 0
+        G.destroy()
+
+
 @pytest.mark.parametrize("graph", ["columns", "random", "two_grids"])
 @pytest.mark.parametrize("noalloc", [False, True])
 def test_cc_first_parents_and_chains(sg, device, oracle_mod, graph, noalloc):
