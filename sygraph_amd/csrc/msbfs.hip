@@ -199,6 +199,14 @@ struct MsArgs {
 __device__ __forceinline__ uint32_t load_flags(const Ctl* c) { return atomic_load(&c->flags); }
 __device__ __forceinline__ void raise_flag(Ctl* c, uint32_t f) { atomic_or(&c->flags, f); }
 
+/* A batch of few (arc, source) pairs runs with one workgroup per CU, whose
+ * barriers cost half those of four or five per CU (6,000 vertices of 5 arcs,
+ * BC of 64 sources 1019 -> 879 us, of 5 sources 547 -> 418; a 40 x 60 grid,
+ * BC 3363 -> 2297, MS-BFS 805 -> 776).  Above, the waves' loads in flight count
+ * more: BC of 64 sources over 500,000 random arcs 747 us with all, 892 with
+ * 256. */
+constexpr int64_t kFewPairs = int64_t(1) << 22;
+
 /* Grid barrier over a launch whose workgroups are all resident.  Arrival
  * counters only grow (barrier t completes at t arrivals per member), so
  * nothing is reset between barriers.  No fences: everything the workgroups
@@ -1433,7 +1441,8 @@ int launch_batches(sg_graph_t g, bool bc, int32_t nsrc, const int32_t* sources, 
     SG_HIP(hipGetLastError());
     void* args[] = {&a};
     const int which = !bc ? 0 : (a.plain ? 2 : 1);
-    SG_HIP(launch_resident(kernels[which], occs[which] * dev->cus, kBlock, args, s));
+    const int per_cu = m * k <= kFewPairs ? 1 : occs[which];
+    SG_HIP(launch_resident(kernels[which], per_cu * dev->cus, kBlock, args, s));
     SG_HIP(hipMemcpyAsync(hctl, a.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s));
     SG_HIP(hipStreamSynchronize(s));
     const uint32_t fl = hctl->flags;
