@@ -270,6 +270,74 @@ __global__ void __launch_bounds__(kBlock) maxprop_kernel(QEntry* q0, QEntry* q1,
   });
 }
 
+/* A small undirected graph in one launch of one workgroup, its trees in LDS:
+ * each thread links an even share of the arcs (a search of the offsets finds
+ * the first one's vertex, then it walks; an edge is linked from its larger
+ * end), then everything is flattened.  Bound by the launch and the threads'
+ * chains of LDS reads, where the sampling below is bound by its dozen launches
+ * and a copy: 1,100 vertices of 13 arcs 112 -> 30 us, a 40 x 60 grid
+ * 100 -> 28.  One workgroup's chains grow with the arcs (a 128 x 128 grid of
+ * 63,000 arcs 111 us, 16,000 vertices of 8 arcs 150) while the sampling stays
+ * near its launches (a 150 x 200 grid of 119,000 arcs 87), so the line lies at
+ * half of where they meet; the vertices are bounded by LDS. */
+constexpr int kSmallVerts = 16384, kSmallThreads = 1024;
+constexpr int64_t kSmallArcs = 1 << 15;
+
+__device__ __forceinline__ uint32_t small_load(const uint32_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+/* root of x, with path halving (a vertex under another one never becomes a root again) */
+__device__ __forceinline__ uint32_t small_root(uint32_t* parent, uint32_t x) {
+  for (;;) {
+    const uint32_t p = small_load(&parent[x]);
+    if (p == x) return x;
+    const uint32_t q = small_load(&parent[p]);
+    if (q == p) return p;
+    __hip_atomic_store(&parent[x], q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    x = q;
+  }
+}
+
+template<typename OffT>
+__global__ void __launch_bounds__(kSmallThreads) cc_small_kernel(const OffT* off, const int32_t* cols, int32_t n,
+                                                                 int32_t m, uint32_t* labels) {
+  __shared__ uint32_t parent[kSmallVerts];
+  for (int i = threadIdx.x; i < n; i += kSmallThreads) parent[i] = (uint32_t)i;
+  __syncthreads();
+  const int32_t share = (m + kSmallThreads - 1) / kSmallThreads;
+  int32_t j = (int32_t)threadIdx.x * share;
+  const int32_t je = min(j + share, m);
+  if (j < je) {
+    int32_t lo = 0, hi = n; /* off[lo] <= j < off[hi] */
+    while (hi - lo > 1) {
+      const int32_t mid = (lo + hi) >> 1;
+      if ((int64_t)off[mid] <= j) lo = mid;
+      else hi = mid;
+    }
+    uint32_t u = (uint32_t)lo;
+    int64_t end = (int64_t)off[u + 1];
+    for (; j < je; ++j) {
+      while (j >= end) end = (int64_t)off[++u + 1];
+      const uint32_t v = (uint32_t)cols[j];
+      if (v >= u) continue;
+      for (uint32_t a = u, b = v;;) {
+        a = small_root(parent, a);
+        b = small_root(parent, b);
+        if (a == b) break;
+        if (atomicCAS(&parent[min(a, b)], min(a, b), max(a, b)) == min(a, b)) break;
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += kSmallThreads) {
+    uint32_t x = (uint32_t)i;
+    for (uint32_t p = parent[x]; p != x; p = parent[x]) x = p;
+    labels[i] = x;
+  }
+}
+
+inline bool cc_small(const sg_graph_s* g) { return g->n <= kSmallVerts && g->m > 0 && g->m <= kSmallArcs; }
+
 /* The forest of an undirected graph's sampled arcs (not flattened). */
 template<typename OffT>
 void sample_forest(sg_device_t dev, hipStream_t s, const OffT* off, const int32_t* cols, int64_t n, uint32_t* parent) {
@@ -302,7 +370,11 @@ int run_cc(sg_graph_t g, uint32_t* labels, int32_t* rounds_out) {
   int32_t rounds = 0;
   bool sym = false;
   if (!(g->flags & SG_GRAPH_DIRECTED)) SG_TRY(graph_symmetric<OffT>(g, reinterpret_cast<unsigned long long*>(roots), &sym));
-  if (sym) {
+  if (sym && cc_small(g)) {
+    cc_small_kernel<OffT><<<1, kSmallThreads, 0, s>>>(off, g->cols, (int32_t)n, (int32_t)g->m, labels);
+    SG_HIP(hipGetLastError());
+    rounds = 1;
+  } else if (sym) {
     const int grid_n = sg::grid_for(dev, n, kBlock, 8);
     sample_forest<OffT>(dev, s, off, g->cols, n, labels);
     flatten_kernel<<<grid_n, kBlock, 0, s>>>(labels, n);
@@ -519,7 +591,11 @@ int run_cc_noalloc(sg_graph_t g, uint32_t* labels, int32_t* rounds_out) {
   int32_t rounds = 0;
   bool sym = false;
   if (!(g->flags & SG_GRAPH_DIRECTED)) SG_TRY(graph_symmetric<OffT>(g, ctr, &sym));
-  if (sym) {
+  if (sym && cc_small(g)) {
+    cc_small_kernel<OffT><<<1, kSmallThreads, 0, s>>>(off, g->cols, (int32_t)n, (int32_t)g->m, labels);
+    SG_HIP(hipGetLastError());
+    rounds = 1;
+  } else if (sym) {
     sample_forest<OffT>(dev, s, off, g->cols, n, labels);
     flatten_kernel<<<grid_n, 256, 0, s>>>(labels, n);
     sample_roots_kernel<<<kRootSamples / 256, 256, 0, s>>>(labels, n, roots);

@@ -418,6 +418,7 @@ def test_cc_sampling_shapes(sg, device, oracle_mod):
         G = sg.Graph.from_csr(device, g.offsets, g.cols)
         c = sg.CC(G)
         c.init()
+        c.init()
         c.run()
         assert np.array_equal(c.get_labels(), oracle_mod.cc(g))
 
@@ -584,6 +585,30 @@ def test_sssp_small_graph_in_one_launch(sg, device, oracle_mod, n, arcs, hubs, w
                     assert sum(st.round_edges[:st.rounds]) == st.relaxations
                     assert st.round_vertices[0] == 1 and min(st.round_vertices[:st.rounds]) > 0
         G.destroy()
+
+
+@pytest.mark.parametrize("offset_bytes", [4, 8])
+@pytest.mark.parametrize("n,arcs", [(1, 0), (2, 1), (1024, 511), (1025, 1024), (16384, 9000), (16384, 16384), (16384, 16385),
+                                    (16385, 9000), (300, 4000)])
+def test_cc_small_graph_in_one_launch(sg, device, oracle_mod, n, arcs, offset_bytes):
+    """Graphs on both sides of the largest that one launch takes, with fewer arcs than threads and a last
+    share that is not full, a hub's list over many shares and vertices without arcs between: the
+    oracle's labels."""
+    rng = np.random.default_rng(n + arcs)
+    pairs = rng.choice(n * (n - 1) // 2, arcs, replace=False) if arcs else np.zeros(0, dtype=np.int64)
+    v = ((1 + np.sqrt(1 + 8 * pairs.astype(np.float64))) / 2).astype(np.int64)
+    v += (v * (v + 1) // 2 <= pairs).astype(np.int64) - (v * (v - 1) // 2 > pairs).astype(np.int64)
+    u = pairs - v * (v - 1) // 2
+    if arcs == 9000:
+        u, v = np.concatenate([u, np.full(5000, n // 2)]), np.concatenate([v, n // 2 + 1 + np.arange(5000)])
+    g = oracle_mod.csr_from_pairs(n, u, v)
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, offset_bytes=offset_bytes)
+    for _ in range(2):
+        c = sg.CC(G)
+        c.init()
+        c.run()
+        assert np.array_equal(c.get_labels(), oracle_mod.cc(g))
+    G.destroy()
 
 
 @pytest.mark.parametrize("graph", ["columns", "random", "two_grids"])
