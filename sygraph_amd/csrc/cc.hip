@@ -298,15 +298,17 @@ __device__ __forceinline__ uint32_t small_root(uint32_t* parent, uint32_t x) {
   }
 }
 
+/* (the arcs are those the offsets name: the array of ids may hold more) */
 template<typename OffT>
 __global__ void __launch_bounds__(kSmallThreads) cc_small_kernel(const OffT* off, const int32_t* cols, int32_t n,
-                                                                 int32_t m, uint32_t* labels) {
+                                                                 uint32_t* labels) {
   __shared__ uint32_t parent[kSmallVerts];
   for (int i = threadIdx.x; i < n; i += kSmallThreads) parent[i] = (uint32_t)i;
   __syncthreads();
-  const int32_t share = (m + kSmallThreads - 1) / kSmallThreads;
-  int32_t j = (int32_t)threadIdx.x * share;
-  const int32_t je = min(j + share, m);
+  const int32_t first = (int32_t)off[0], last = (int32_t)off[n];
+  const int32_t share = (last - first + kSmallThreads - 1) / kSmallThreads;
+  int32_t j = first + (int32_t)threadIdx.x * share;
+  const int32_t je = min(j + share, last);
   if (j < je) {
     int32_t lo = 0, hi = n; /* off[lo] <= j < off[hi] */
     while (hi - lo > 1) {
@@ -371,7 +373,7 @@ int run_cc(sg_graph_t g, uint32_t* labels, int32_t* rounds_out) {
   bool sym = false;
   if (!(g->flags & SG_GRAPH_DIRECTED)) SG_TRY(graph_symmetric<OffT>(g, reinterpret_cast<unsigned long long*>(roots), &sym));
   if (sym && cc_small(g)) {
-    cc_small_kernel<OffT><<<1, kSmallThreads, 0, s>>>(off, g->cols, (int32_t)n, (int32_t)g->m, labels);
+    cc_small_kernel<OffT><<<1, kSmallThreads, 0, s>>>(off, g->cols, (int32_t)n, labels);
     SG_HIP(hipGetLastError());
     rounds = 1;
   } else if (sym) {
@@ -592,7 +594,7 @@ int run_cc_noalloc(sg_graph_t g, uint32_t* labels, int32_t* rounds_out) {
   bool sym = false;
   if (!(g->flags & SG_GRAPH_DIRECTED)) SG_TRY(graph_symmetric<OffT>(g, ctr, &sym));
   if (sym && cc_small(g)) {
-    cc_small_kernel<OffT><<<1, kSmallThreads, 0, s>>>(off, g->cols, (int32_t)n, (int32_t)g->m, labels);
+    cc_small_kernel<OffT><<<1, kSmallThreads, 0, s>>>(off, g->cols, (int32_t)n, labels);
     SG_HIP(hipGetLastError());
     rounds = 1;
   } else if (sym) {

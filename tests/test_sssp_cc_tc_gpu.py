@@ -611,6 +611,24 @@ def test_cc_small_graph_in_one_launch(sg, device, oracle_mod, n, arcs, offset_by
     G.destroy()
 
 
+@pytest.mark.parametrize("offset_bytes", [4, 8])
+@pytest.mark.parametrize("before,after", [(0, 1), (0, 3000), (7, 0), (1500, 1500)])
+@pytest.mark.parametrize("n,arcs", [(2, 1), (1024, 900), (16384, 6000)])
+def test_cc_small_graph_in_a_larger_id_array(sg, device, oracle_mod, n, arcs, before, after, offset_bytes):
+    """Offsets that name a part of the array of ids only (ids ahead of the first list and behind the last, as
+    an array kept with room to grow has them): every call reads the lists, so the labels are the plain graph's."""
+    rng = np.random.default_rng(n + before + after)
+    g = oracle_mod.csr_from_pairs(n, rng.integers(0, n, arcs), rng.integers(0, n, arcs))
+    spare = [rng.integers(0, n, k).astype(np.int32) for k in (before, after)]
+    G = sg.Graph.from_csr(device, g.offsets + before, np.concatenate([spare[0], g.cols, spare[1]]),
+                          offset_bytes=offset_bytes)
+    c = sg.CC(G)
+    c.init()
+    c.run()
+    assert np.array_equal(c.get_labels(), oracle_mod.cc(g))
+    G.destroy()
+
+
 @pytest.mark.parametrize("graph", ["columns", "random", "two_grids"])
 @pytest.mark.parametrize("noalloc", [False, True])
 def test_cc_first_parents_and_chains(sg, device, oracle_mod, graph, noalloc):
