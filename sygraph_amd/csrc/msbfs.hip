@@ -686,8 +686,8 @@ __device__ __forceinline__ void expand_pull(const MsArgs<OffT>& a, const uint64_
       heavy &= heavy - 1;
       const int64_t kb = (int64_t)wave_lane((uint64_t)head, k2), ke = (int64_t)wave_lane((uint64_t)e, k2);
       const uint64_t kwant = wave_lane(want, k2);
-      uint64_t part = lane == 0 ? wave_lane(acc, k2) : 0ull;
-      uint64_t all = 0;
+      const uint64_t got = wave_lane(acc, k2); /* (read by the whole wave: lane k2 has to take part) */
+      uint64_t part = lane == 0 ? got : 0ull, all = 0;
       for (int64_t j0 = kb; j0 < ke; j0 += 4 * 64) {
         int32_t x[4];
         uint64_t m[4];

@@ -90,3 +90,33 @@ def test_msbfs_direction_rules_same_depths(sg, device, oracle_mod, graph):
             assert np.array_equal(d[i], ref[i]), (policy, srcs[i])
     with pytest.raises(sg.SygraphError):
         sg.bfs_multi(G, srcs, policy=sg.POLICY_LEARNED)  # no trained policy given
+
+
+@pytest.mark.parametrize("directed", [False, True])
+def test_pull_of_long_lists_keeps_what_their_head_gave(sg, device, oracle_mod, directed):
+    """In-lists of 64 to 900 arcs whose first 32 name half of the sources and whose last 32 the other half: a
+    lane gathers the head, the whole wave the rest, and the vertex is reached from all of them.  Several such
+    vertices share a wave, some waves have one."""
+    spare = np.concatenate([np.arange(9), [23, 24, 63, 64, 65, 191, 192, 193, 255, 256, 257, 835]])
+    t = len(spare)
+    first = 32 + t + 64  # fillers, then the other half of the sources; the target at 32 + t is on its own
+    n = first + int(spare.max()) + 32
+    u, v = [], []
+    for k, d in enumerate(np.append(spare, 200)):
+        at = 32 + k if k < t else 32 + t + 63
+        ins = np.concatenate([np.arange(32), first + np.arange(d), n - 32 + np.arange(32)])
+        u.append(ins)
+        v.append(np.full(len(ins), at))
+    u, v = np.concatenate(u), np.concatenate(v)
+    if directed:
+        order = np.lexsort((v, u))
+        off = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=n))]).astype(np.int64)
+        g = oracle_mod.CSRGraph(n, off, v[order].astype(np.int32))
+    else:
+        g = oracle_mod.csr_from_pairs(n, u, v)
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, directed=directed)
+    srcs = np.concatenate([np.arange(32), n - 32 + np.arange(32)])
+    d = sg.bfs_multi(G, srcs, policy=sg.POLICY_PULL)
+    for i, s in enumerate(srcs):
+        assert np.array_equal(d[i], oracle_mod.bfs(g, int(s))[0]), i
+    assert (d[:, 32:32 + t] == 1).all() and (d[:, 32 + t + 63] == 1).all()
