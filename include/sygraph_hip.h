@@ -300,14 +300,15 @@ typedef struct sg_level_stat {
   int64_t max_degree;        /* largest degree among the discovered vertices */
   int32_t action;            /* direction * 3 + work-mapping variant (0 bucketing, 1 edge-balanced /
                                 short pull head, 2 wave-split / long pull head) of this level */
-  float kernel_ms;           /* device time of the level's traversal kernel (record_levels; 0 for the
-                                levels of a burst) */
+  float kernel_ms;           /* device time of the level's traversal (record_levels): of its kernel, by
+                                events, or inside a single-workgroup burst, by the device's clock; 0
+                                for the levels of a grid burst after its first */
   float convert_ms;          /* device time of what follows it in the same step: the count, scan,
-                                decision and queue write, and the burst of small levels if one ran */
+                                decision and queue write (0 for the levels inside a burst) */
   int32_t burst;             /* 1: the level ran inside a single-workgroup burst of small push levels,
-                                timed in convert_ms of the level before it; the level at which a burst
-                                stops is counted and decided by the next step, whose times it carries
-                                (a small graph traversed in one launch: the first level's kernel_ms) */
+                                2: inside a grid burst, whose time is in kernel_ms of its first level;
+                                the level at which a single-workgroup burst stops is counted and decided
+                                by the next step */
 } sg_level_stat;
 
 typedef struct sg_bfs_stats {

@@ -299,6 +299,7 @@ struct BfsCtl {
 struct alignas(64) LevelLog {
   int32_t level, dir, done, next_dir, action, burst;
   int64_t f_vertices, f_edges, disc, disc_deg, edges, scanned, misses, max_deg, unexplored;
+  int64_t ticks; /* a level of a burst of one workgroup: its time by the constant-rate clock; others 0 */
 };
 
 /* One step's record (a step = the launches the host enqueues together: one
@@ -311,6 +312,7 @@ struct alignas(64) StepLog {
   int32_t fail;     /* a grid barrier timed out */
   int64_t reached_v, reached_e;
   int64_t next_f_edges; /* its frontier's arcs */
+  int64_t ticks;        /* of the level after last_level, where a burst traversed it and handed it back */
 };
 
 constexpr int kRing = 8; /* steps in the log / event rings (> lookahead + 1) */
@@ -534,6 +536,7 @@ __device__ __forceinline__ void finish_level(const FinishArgs& f, BfsCtl* ctl, c
     e.misses = (int64_t)misses;
     e.max_deg = (int64_t)max_deg;
     e.unexplored = (int64_t)(p.total_degree - vdeg);
+    e.ticks = 0;
     f.levlog[level] = e;
   }
   const int32_t n_push = ctl->n_push + (dir == 0 ? 1 : 0), n_pull = ctl->n_pull + (dir == 0 ? 0 : 1);
@@ -801,6 +804,7 @@ __device__ __forceinline__ void burst_visit_big(const BurstArgs<OffT>& a, const 
 template<bool kLds, typename OffT>
 __device__ __forceinline__ void burst_body(const BurstArgs<OffT>& a, BfsCtl* ctl, const DecideParams& p,
                                            int32_t step, LevelLog* levlog, StepLog* steplog, bool publish) {
+  int64_t mark = (int64_t)wall_clock64(), now = mark; /* the levels' times, which no event stands between */
   __shared__ sg::policy::Staged s_pol;
   __shared__ uint32_t s_count[2][2];
   __shared__ unsigned long long s_red[2][kBurstWaves][5];
@@ -866,6 +870,7 @@ __device__ __forceinline__ void burst_body(const BurstArgs<OffT>& a, BfsCtl* ctl
     act = decide_action(p, &s_pol, 0, disc, disc_deg, unexplored, level + 1, max_deg);
     done = disc == 0 ? 1 : 0;
     const bool more = !done && act / 3 == 0 && (int64_t)disc_deg <= p.burst_arcs;
+    now = (int64_t)wall_clock64();
     if (!more && !done) break; /* the next step counts and decides this level (hand-back) */
     if (threadIdx.x == 0 && level < SG_MAX_LEVELS_RECORDED) {
       LevelLog e;
@@ -884,8 +889,10 @@ __device__ __forceinline__ void burst_body(const BurstArgs<OffT>& a, BfsCtl* ctl
       e.misses = 0;
       e.max_deg = (int64_t)max_deg;
       e.unexplored = (int64_t)unexplored;
+      e.ticks = now - mark;
       levlog[level] = e;
     }
+    mark = now;
     vdeg += disc_deg;
     reached += disc;
     ++n_push;
@@ -921,6 +928,7 @@ __device__ __forceinline__ void burst_body(const BurstArgs<OffT>& a, BfsCtl* ctl
     sl.reached_v = (int64_t)reached;
     sl.reached_e = (int64_t)vdeg;
     sl.next_f_edges = f_edges; /* the level handed back, a push level */
+    sl.ticks = done ? 0 : now - mark;
     /* the step's record, unless the step's own count pass writes it later
      * (a burst ahead of the step that hands a level back) */
     if (publish || done) publish_step(&steplog[step % kRing], sl);
@@ -967,6 +975,7 @@ __global__ void __launch_bounds__(kBurstThreads) small_kernel(StartArgs<OffT> s,
     if (threadIdx.x == 0) {
       StepLog sl{};
       sl.step = step;
+      sl.last_level = -1;
       publish_step(&steplog[step % kRing], sl);
     }
     return;
@@ -1336,6 +1345,7 @@ __global__ void __launch_bounds__(gb::kThreads) gburst_kernel(GbArgs<OffT> a, Bf
             e.misses = 0;
             e.max_deg = (int64_t)t.mx;
             e.unexplored = (int64_t)unexplored;
+            e.ticks = 0;
             a.log[level] = e;
           }
           vdeg += t.deg;
@@ -1713,10 +1723,15 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
   for (int k = 0; k < kRing; ++k) __atomic_store_n(&ws->steplog[k].step, -1, __ATOMIC_RELEASE);
   StepLog last{};
   int32_t first_level = 0;
-  /* the records of levels first_level .. last.last_level; the times are the
-   * first one's (the step's later levels ran in a burst, timed with the count
-   * and write) */
+  /* The records of levels first_level .. last.last_level: the step's own level,
+   * the first whose time the step's events hold, and those of the burst ahead
+   * of it or after it, which timed themselves; what the step's rest spent on
+   * the latter is theirs.  A level that a burst traversed and handed back
+   * (`handed`) gets that time in the step that counts it. */
+  float handed = 0.f;
   auto take_levels = [&](float k_ms, float c_ms) {
+    const float to_ms = 1.0f / (float)dev->wall_khz;
+    sg_level_stat* own = nullptr;
     for (int32_t L = first_level; stats && L <= last.last_level && L < SG_MAX_LEVELS_RECORDED; ++L) {
       LevelLog e;
       std::memcpy(&e, (const void*)&ws->levlog[L], sizeof(e));
@@ -1734,11 +1749,17 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
       ls.unexplored_edges = e.unexplored;
       ls.action = e.action;
       ls.burst = e.burst;
-      if (L == first_level) {
-        ls.kernel_ms = k_ms;
-        ls.convert_ms = c_ms;
+      if (!timed) continue;
+      if (e.ticks > 0) {
+        ls.kernel_ms = (float)e.ticks * to_ms;
+        if (own) c_ms -= ls.kernel_ms;
+      } else if (!own) {
+        own = &ls;
+        ls.kernel_ms = k_ms + handed;
       }
     }
+    handed = timed ? (float)last.ticks * to_ms : 0.f;
+    if (own) own->convert_ms = std::max(c_ms - handed, 0.f);
   };
   /* a start in a burst: the levels from the source while they stay small,
    * handed back to step 0 (which then only counts and decides) or ending the
@@ -1750,12 +1771,12 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
     std::memcpy(&last, (const void*)&ws->steplog[kRing - 1], sizeof(last));
     /* the slot is step kRing - 1's again */
     __atomic_store_n(&ws->steplog[kRing - 1].step, -1, __ATOMIC_RELEASE);
-    if (last.done) take_levels(0.f, 0.f);
+    take_levels(0.f, 0.f);
+    first_level = last.last_level + 1;
   } else if (burst_arcs > 0 && opt.policy != SG_POLICY_PULL) {
     burst_kernel<OffT><<<1, kBurstThreads, 0, s>>>(burst_args(0), ws->ctl, P, 0, ws->levlog, ws->steplog);
   }
-  const bool one_launch = last.done;
-  if (!one_launch) {
+  if (!last.done) {
     SG_TRY(enqueue(0, false));
     for (int k = 1; k <= lookahead; ++k) SG_TRY(enqueue(k, false));
   }
@@ -1811,9 +1832,6 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
     float ms = 0.f;
     SG_HIP(hipEventElapsedTime(&ms, ws->ev_begin, ws->ev_end));
     stats->kernel_ms = ms;
-    /* one launch took every level: its time stands at the first, with no
-     * events around it that the call would wait for */
-    if (timed && one_launch) stats->level[0].kernel_ms = ms;
     stats->levels = last.last_level + 1;
     stats->n_push = last.n_push;
     stats->n_pull = last.n_pull;

@@ -458,3 +458,26 @@ def test_small_graph_in_one_launch(sg, device, oracle_mod, n, arcs, directed):
                               for x in st.level[:st.levels]]))
             assert runs[0] == runs[2] and runs[1] == runs[2], (src, policy)
     G.destroy()
+
+
+@pytest.mark.parametrize("graph", ["small", "small_grid", "rmat", "path"])
+@pytest.mark.parametrize("policy", ["push", "pull", "hybrid"])
+def test_record_levels_times_every_level(sg, device, oracle_mod, graph, policy):
+    """Every level has a time of its own -- by events, or inside a burst of one workgroup by the device's
+    clock, from the source, after a step or in the launch that takes a whole small graph -- and together
+    they are no more than the traversal's."""
+    g = {"small": lambda: oracle_mod.rmat(10, 12, seed=3), "small_grid": lambda: oracle_mod.grid(60, 70, 0.1, seed=4),
+         "rmat": lambda: oracle_mod.rmat(15, 16, seed=5),
+         "path": lambda: oracle_mod.csr_from_pairs(70000, np.arange(66000, 69999), np.arange(66001, 70000))}[graph]()
+    G = sg.Graph.from_csr(device, g.offsets, g.cols)
+    src = 67000 if graph == "path" else int(np.argmax(g.degrees()))
+    b = sg.BFS(G)
+    for _ in range(2):
+        b.init(src)
+        st = b.run(getattr(sg, "POLICY_" + policy.upper()), 15.0, 24.0, tuning={"grid_burst_arcs": -1}, record_levels=True)
+        levels = st.level[:st.levels]
+        assert np.array_equal(b.get_distances(), oracle_mod.bfs(g, src)[0])
+        assert st.levels > 2 and min(x.kernel_ms for x in levels) > 0
+        assert min(x.convert_ms for x in levels) >= 0
+        assert sum(x.kernel_ms + x.convert_ms for x in levels) <= 1.02 * st.kernel_ms + 0.01
+    G.destroy()
