@@ -405,7 +405,8 @@ typedef struct sg_sssp_options {
                             and larger ones of at most 2^17 arcs in one launch of resident
                             workgroups: 0 = default (4,096), negative = neither, at most 8,192 */
   int32_t record_relax;  /* 1: time every relax launch on its own (two events per round; stats must
-                            not be NULL): stats->relax_ms / relax_launches */
+                            not be NULL): stats->relax_ms / relax_launches.  Rounds of more than
+                            burst_arcs arcs then always are launches of their own */
 } sg_sssp_options;
 void sg_sssp_options_default(sg_sssp_options* opt);
 /* sg_sssp with options; the distances do not depend on delta. */

@@ -1622,8 +1622,9 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, double grid_step, int32_t 
   sa.w_max = w_max;
   sa.pull_mode = pull_mode;
   sa.bellman = bellman ? 1 : 0;
-  /* the grid bursts' near and far piles take the small rounds from the start */
-  const bool grid = bellman && burst_arcs > 0, piles = grid && grid_step > 0.0;
+  /* the grid bursts' near and far piles take the small rounds from the start;
+   * a record of the relax launches leaves the rounds to them */
+  const bool grid = bellman && burst_arcs > 0 && !record_relax, piles = grid && grid_step > 0.0;
   sa.burst_arcs = piles ? 0 : burst_arcs;
   SsspBurst<OffT, W> sb{};
   sb.off = off;

@@ -686,3 +686,19 @@ def test_tc_matches_oracle_on_uneven_degrees(sg, device, oracle_mod, seed, n, hu
         u, v = np.concatenate([u, np.full(len(pick), h)]), np.concatenate([v, pick])
     g = oracle_mod.csr_from_pairs(n + 70, u, v)
     assert sg.TC(sg.Graph.from_csr(device, g.offsets, g.cols)).run() == oracle_mod.tc(g)
+
+
+@pytest.mark.parametrize("delta", [0.0, -1.0])
+def test_sssp_record_relax_times_the_launched_rounds(sg, device, oracle_mod, delta):
+    """With the relax launches recorded, every round above the one-workgroup bursts' limit is a launch with its
+    own time, under the automatic schedule too (a 150 x 150 grid: hundreds of rounds, nearly all of them)."""
+    g = oracle_mod.grid(150, 150, 0.05, seed=14)
+    oracle_mod.fill_weights(g, 15)
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, weights=g.weights)
+    src = int(np.nonzero(g.degrees() > 0)[0][0])
+    s = sg.SSSP(G)
+    s.init(src)
+    st = s.run(delta=delta, burst_arcs=64, record_relax=True)
+    assert np.array_equal(s.get_distances(), oracle_mod.sssp(g, src))
+    assert st.rounds > 100 and st.relax_launches > 0.8 * st.rounds
+    assert 0 < st.relax_ms < st.kernel_ms
