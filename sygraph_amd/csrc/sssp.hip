@@ -363,6 +363,16 @@ __global__ void split_slots_reset_kernel(SplitSlot* slots, const SsspCtl* ctl) {
  * round is relaxed again in the next.  The burst stops when a round lowers
  * nothing or the next list is too large: its vertices keep their dirty bits
  * and the next iteration's selection takes them from the bitmap. */
+/* what the bursts tell of their rounds: vertices and arcs of round r at
+ * [2 r] and [2 r + 1], zeros where a round was a launch (the iteration's
+ * record has it).  A round's vertices are its list's entries: a grid burst
+ * lists a vertex again when it is lowered again in the same round. */
+__device__ __forceinline__ void record_round(unsigned long long* rounds, int64_t r, unsigned long long vertices,
+                                             unsigned long long arcs) {
+  if (!rounds || r >= SG_MAX_LEVELS_RECORDED) return;
+  rounds[2 * r] = vertices;
+  rounds[2 * r + 1] = arcs;
+}
 constexpr int kSsspBurstDefault = 4096;
 constexpr int kSsspBurstMax = 8192; /* entries (and arcs) of a burst round; LDS for its scan */
 
@@ -378,6 +388,7 @@ struct SsspBurst {
   QEntry* list[2]; /* kSsspBurstMax entries each */
   int64_t burst_arcs;
   unsigned long long* relax_slots;
+  unsigned long long* rounds; /* record_round's */
   uint32_t* arrive; /* kArriveWords zeroed words */
 };
 
@@ -397,6 +408,7 @@ __device__ __forceinline__ void sssp_burst(const SsspBurst<OffT, W>& b, SsspCtl*
   __syncthreads();
   unsigned long long arcs = 0;
   int32_t rounds = 0;
+  const int32_t first_round = ctl->rounds - 1; /* counted by the selection */
   for (int it = 0;; ++it) {
     const QEntry* in = b.list[(it + 1) & 1];
     QEntry* out = b.list[it & 1];
@@ -422,7 +434,10 @@ __device__ __forceinline__ void sssp_burst(const SsspBurst<OffT, W>& b, SsspCtl*
         s_pref[first + k] = pos;
         pos += (uint32_t)entry(first + k).len;
       }
-    if (threadIdx.x == 0) s_pref[cnt] = total;
+    if (threadIdx.x == 0) {
+      s_pref[cnt] = total;
+      record_round(b.rounds, first_round + rounds, rounds == 0 ? h.nvert : (unsigned long long)cnt, total);
+    }
     __syncthreads();
     for (uint32_t t = threadIdx.x; t < total; t += kBlock) {
       uint32_t lo = 0, hi = cnt; /* s_pref[lo] <= t < s_pref[hi] */
@@ -813,6 +828,7 @@ struct SsspGrid {
   double w_max;
   gb::Exchange x;
   unsigned long long* relax_slots;
+  unsigned long long* rounds; /* record_round's */
   RoundLog* log;
   uint32_t stride; /* the burst's workgroups are those with blockIdx.x % stride == 0 */
 };
@@ -1038,8 +1054,10 @@ __global__ void __launch_bounds__(gb::kThreads) sssp_grid_kernel(SsspGrid<OffT, 
   const int lane = lane_id(), wv = threadIdx.x >> 6;
   const uint32_t gwave = (uint32_t)wv * wgs + rank, nwaves = wgs * gb::kWaves; /* across the workgroups first */
   const bool lead = rank == 0 && threadIdx.x == 0;
-  unsigned long long arcs = h0.deg, relaxed = 0; /* arcs of the round; of the rounds before it (first wave) */
+  /* arcs and entries of the round; arcs of the rounds before it (first wave) */
+  unsigned long long arcs = h0.deg, entries = h0.nvert, relaxed = 0;
   int32_t rounds = 0;
+  const int32_t first_round = ctl->rounds - 1; /* counted by the selection */
   const bool piles = a.step > 0.0;
   double step = a.step;                               /* first wave, like what follows */
   unsigned long long bucket_arcs = 0, bucket_rounds = 0;
@@ -1161,12 +1179,14 @@ __global__ void __launch_bounds__(gb::kThreads) sssp_grid_kernel(SsspGrid<OffT, 
       const unsigned long long extra = !kept ? 0ull : far_pass ? 1ull << 32 | s_far_top : 1ull;
       if (gb::exchange(a.x, &s_local, it, rank, wgs, s_n, t, extra)) {
         if (!far_pass) {
+          if (lead) record_round(a.rounds, first_round + rounds, entries, arcs);
           relaxed += arcs;
           bucket_arcs += arcs;
           ++bucket_rounds;
           ++rounds;
         }
         arcs = t.deg;
+        entries = t.disc;
         const bool fits = (int64_t)t.deg <= a.grid_arcs && t.most <= a.seg_cap && (int64_t)t.npieces <= a.cap_pieces;
         next = t.disc > 0 ? (fits ? 0 : 1) : t.mx ? 3 : 1;
         if (next == 3) { /* the bucket is done: on by a step, or where that found nothing from the smallest left */
@@ -1229,8 +1249,9 @@ __global__ void __launch_bounds__(gb::kThreads) sssp_grid_kernel(SsspGrid<OffT, 
     return;
   }
   if (!lead) return;
-  /* the selection counted the first round; the relax launch has nothing left */
-  ctl->rounds += rounds > 1 ? rounds - 1 : 0;
+  /* the selection counted one round (none, where the first does not fit the
+   * lists); the relax launch has nothing left */
+  ctl->rounds += rounds - 1;
   ctl->relaxed += relaxed - h0.deg;
   ctl->relax = 0;
   atomic_add(&a.relax_slots[0], relaxed);
@@ -1343,9 +1364,11 @@ __global__ void __launch_bounds__(kBlock) sssp_select_kernel(CompactArgs<OffT> c
 
 template<typename OffT>
 __global__ void sssp_init_kernel(const OffT* off, uint32_t* dist, uint32_t unreached, int64_t n, int32_t src,
-                                 QEntry* q0, QEntry* q1, QEntry* q2, QueueHdr* hdr, Tuning t) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    dist[i] = i == src ? 0u : unreached;
+                                 QEntry* q0, QEntry* q1, QEntry* q2, QueueHdr* hdr, Tuning t,
+                                 unsigned long long* rounds) {
+  const int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = tid; i < n; i += stride) dist[i] = i == src ? 0u : unreached;
+  for (int64_t i = tid; rounds && i < 2 * SG_MAX_LEVELS_RECORDED; i += stride) rounds[i] = 0ull;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     QEntry* const q[3] = {q0, q1, q2};
     enqueue_single(off, t, q, hdr, src);
@@ -1400,6 +1423,7 @@ struct SsspWorkspace {
   SplitSlot* slots = nullptr;
   SsspCtl* ctl = nullptr;
   unsigned long long* relax_slots = nullptr; /* kSlots x 16 (one cache line each) */
+  unsigned long long* rounds = nullptr;      /* behind them: record_round's, SG_MAX_LEVELS_RECORDED pairs */
   uint32_t* arrive = nullptr; /* arrival counters of the selection and write launches (kArriveWords each), zero
                                  between launches */
   QEntry* burst_list[2] = {nullptr, nullptr}; /* kSsspBurstMax entries each */
@@ -1462,7 +1486,7 @@ int sssp_workspace_for(sg_graph_t g, SsspWorkspace** out) {
         (st = sg::alloc_device(dev, (void**)&ws->acc, 16)) ||
         (st = sg::alloc_device(dev, (void**)&ws->slots, sizeof(SplitSlot) * kSlots)) ||
         (st = sg::alloc_device(dev, (void**)&ws->ctl, sizeof(SsspCtl))) ||
-        (st = sg::alloc_device(dev, (void**)&ws->relax_slots, 8 * 16 * kSlots)) ||
+        (st = sg::alloc_device(dev, (void**)&ws->relax_slots, 8 * 16 * kSlots + 16 * SG_MAX_LEVELS_RECORDED)) ||
         (st = sg::alloc_device(dev, (void**)&ws->arrive, 8 * kArriveWords)) ||
         (st = sg::zero_async(dev, ws->arrive, 8 * kArriveWords)) ||
         (st = sg::alloc_device(dev, (void**)&ws->burst_list[0], sizeof(QEntry) * kSsspBurstMax)) ||
@@ -1471,6 +1495,7 @@ int sssp_workspace_for(sg_graph_t g, SsspWorkspace** out) {
       sssp_ws_free(ws);
       return st;
     }
+    ws->rounds = ws->relax_slots + 16 * kSlots;
     bool ok = hipHostMalloc((void**)&ws->log, sizeof(RoundLog) * kRing, hipHostMallocCoherent) == hipSuccess;
     if (ok && n <= kSmallVerts && g->m <= kSmallArcs)
       ok = hipHostMalloc((void**)&ws->small_log, sizeof(SmallLog), hipHostMallocCoherent) == hipSuccess;
@@ -1571,11 +1596,12 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, double grid_step, int32_t 
     SG_TRY(sg::zero_async(dev, settled_all, 8 * ws->w0));
   }
   SG_TRY(sg::zero_async(dev, ws->relax_slots, 8 * 16 * kSlots));
+  const bool bellman = !(delta > 0.0) || !std::isfinite(delta);
+  unsigned long long* rounds_log = stats && bellman && burst_arcs > 0 ? ws->rounds : nullptr; /* bursts may run */
   sssp_init_kernel<OffT><<<sg::grid_for(dev, n, 256, 4), 256, 0, s>>>(off, dist, unreached, n, src, Q.q[0][0],
-                                                                       Q.q[0][1], Q.q[0][2], Q.hdr, tune);
+                                                                       Q.q[0][1], Q.q[0][2], Q.hdr, tune, rounds_log);
   set_bit_kernel<<<1, 1, 0, s>>>(dirty, src);
   SG_HIP(hipGetLastError());
-  const bool bellman = !(delta > 0.0) || !std::isfinite(delta);
   const double w_max = DistOps<W>::is_float ? 3.0e38 : 4294967295.0;
   {
     SsspCtl c{};
@@ -1638,6 +1664,7 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, double grid_step, int32_t 
   sb.list[1] = ws->burst_list[1];
   sb.burst_arcs = burst_arcs;
   sb.relax_slots = ws->relax_slots;
+  sb.rounds = rounds_log;
   sb.arrive = ws->arrive + kArriveWords;
   split_slots_reset_kernel<<<1, 64, 0, s>>>(ws->slots, ws->ctl); /* later iterations clear them as they decide */
   /* one iteration, three launches: split + near-set count + decision (relax /
@@ -1675,6 +1702,7 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, double grid_step, int32_t 
     sg_args.x = ws->grid_x;
     sg_args.x.wait_ticks = dev->wait_ticks;
     sg_args.relax_slots = ws->relax_slots;
+    sg_args.rounds = rounds_log;
     sg_args.log = ws->log;
     sg_args.stride = (uint32_t)ws->grid_stride;
   }
@@ -1756,7 +1784,16 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, double grid_step, int32_t 
     {
       unsigned long long rs[16 * kSlots];
       SG_HIP(hipMemcpyAsync(rs, ws->relax_slots, sizeof(rs), hipMemcpyDeviceToHost, s));
+      auto* rl = static_cast<unsigned long long*>(dev->host_scratch);
+      const int32_t recorded = std::min(round, (int32_t)SG_MAX_LEVELS_RECORDED);
+      if (rounds_log && recorded > 0)
+        SG_HIP(hipMemcpyAsync(rl, rounds_log, 16 * (size_t)recorded, hipMemcpyDeviceToHost, s));
       SG_HIP(hipStreamSynchronize(s));
+      for (int32_t r = 0; rounds_log && r < recorded; ++r) {
+        if (rl[2 * r] == 0) continue;
+        stats->round_vertices[r] = (int64_t)rl[2 * r];
+        stats->round_edges[r] = (int64_t)rl[2 * r + 1];
+      }
       unsigned long long t = 0;
       for (int k = 0; k < kSlots; ++k) t += rs[k * 16];
       stats->relaxations = (int64_t)t; /* arcs relaxed in their phase (examined: `relaxed`) */

@@ -702,3 +702,33 @@ def test_sssp_record_relax_times_the_launched_rounds(sg, device, oracle_mod, del
     assert np.array_equal(s.get_distances(), oracle_mod.sssp(g, src))
     assert st.rounds > 100 and st.relax_launches > 0.8 * st.rounds
     assert 0 < st.relax_ms < st.kernel_ms
+
+
+@pytest.mark.parametrize("delta", [0.0, -1.0])
+@pytest.mark.parametrize("burst", [0, 64, -1])
+@pytest.mark.parametrize("graph", ["grid", "rmat", "layers"])
+def test_sssp_round_records_add_up(sg, device, oracle_mod, graph, burst, delta):
+    """Every round has its vertices and arcs, whether it was a launch or ran in a burst of one workgroup or of
+    many: the arcs of the rounds are the relaxations."""
+    if graph == "grid":
+        g = oracle_mod.grid(150, 150, 0.05, seed=16)
+    elif graph == "rmat":
+        g = oracle_mod.rmat(15, 16, seed=17)
+    else:  # a path into a hub and out of it, so that rounds of one arc stand beside large ones
+        tail = np.arange(20000, 20400)
+        g = oracle_mod.csr_from_pairs(20401, np.concatenate([np.full(9000, 20000), tail, np.arange(9000)]),
+                                      np.concatenate([np.arange(9000), tail + 1, 9000 + np.arange(9000)]))
+    oracle_mod.fill_weights(g, 18)
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, weights=g.weights)
+    src = 20400 if graph == "layers" else int(np.nonzero(g.degrees() > 0)[0][0])
+    ref = oracle_mod.sssp(g, src)
+    for _ in range(2):
+        s = sg.SSSP(G)
+        s.init(src)
+        st = s.run(delta=delta, burst_arcs=burst)
+        assert np.array_equal(s.get_distances(), ref)
+        assert 1 < st.rounds <= sg.MAX_LEVELS_RECORDED
+        assert st.round_vertices[0] == 1 and st.round_edges[0] == g.degrees()[src]
+        assert min(st.round_vertices[:st.rounds]) > 0
+        assert sum(st.round_edges[:st.rounds]) == st.relaxations
+    G.destroy()
