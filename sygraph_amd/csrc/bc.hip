@@ -48,6 +48,7 @@ constexpr int kCountLevels = 1024; /* levels up to which the counting sort's his
 constexpr int kMaxSlots = 64;   /* per-level maximum of sigma: slots, one cache line apart */
 constexpr int kSlotStride = 16; /* unsigned long long per 128-byte line */
 constexpr int64_t kLevelBitmapBytes = 1ll << 30; /* per-level bitmaps up to 1 GiB, else depth[] tests */
+constexpr size_t kKeepBytes = size_t(64) << 20;
 
 /* sum over groups of kLanes lanes, in every lane (fixed butterfly) */
 template<int kLanes>
@@ -175,7 +176,18 @@ __global__ void level_bits_kernel(const int32_t* depth, int64_t n, int64_t w0, i
 
 __device__ __forceinline__ bool bit_of(const uint64_t* bm, int32_t v) { return (bm[v >> 6] >> (v & 63)) & 1ull; }
 
-__global__ void bc_source_init_kernel(double* sigma, int32_t s) { sigma[s] = 1.0; }
+/* The largest sigma of a level, in a block of slots: three blocks in turn, the
+ * level's own, the level before's, which is read, and the next level's, which
+ * is cleared meanwhile (a block per level would be 8 KiB times the levels). */
+constexpr int kSlotWords = kMaxSlots * kSlotStride;
+__device__ __forceinline__ unsigned long long* max_slots(unsigned long long* all, int32_t L) {
+  return all + (int64_t)(L % 3) * kSlotWords;
+}
+
+__global__ void bc_source_init_kernel(double* sigma, int32_t s, unsigned long long* level_max) {
+  for (int i = threadIdx.x; i < 3 * kSlotWords; i += blockDim.x) level_max[i] = 0ull;
+  if (threadIdx.x == 0) sigma[s] = 1.0;
+}
 
 /* 2^-e for the exponent e of a level's largest sigma (1 where none was
  * recorded: the source's level).  All threads call; one barrier. */
@@ -262,16 +274,21 @@ __device__ __forceinline__ void gather_level(const int32_t* order, const int64_t
 }
 
 /* prev_bm: bitmap of level L-1 (L2-resident), or nullptr to test depth[]:
- * sigma is only loaded for real parents.  level_max: the slots of level L,
- * the level before's right ahead of them.  The deepest level's R is final
- * here. */
+ * sigma is only loaded for real parents.  scale[L-1] is written here, for the
+ * way back; the deepest level's R is final here. */
 template<typename OffT>
 __global__ void __launch_bounds__(kBlock) sigma_level_kernel(const int32_t* order, const int64_t* lvl, int32_t L,
                                                              int32_t nl, const uint32_t* hub, int hub_blocks,
                                                              const OffT* in_off, const int32_t* in_cols,
                                                              const int32_t* depth, const uint64_t* prev_bm,
-                                                             double* sigma, double* r, unsigned long long* level_max) {
-  const double sc = level_scale(level_max - kMaxSlots * kSlotStride);
+                                                             double* sigma, double* r, unsigned long long* slots,
+                                                             double* scale) {
+  const double sc = level_scale(max_slots(slots, L - 1));
+  unsigned long long *level_max = max_slots(slots, L), *cleared = max_slots(slots, L + 1);
+  if (blockIdx.x == 0) {
+    for (int i = threadIdx.x; i < kMaxSlots; i += kBlock) cleared[i * kSlotStride] = 0ull;
+    if (threadIdx.x == 0) scale[L - 1] = sc;
+  }
   double mx = 0.0;
   gather_level<OffT>(
       order, lvl, L, hub, hub_blocks, in_off, in_cols, depth, prev_bm, L - 1,
@@ -297,15 +314,14 @@ __global__ void __launch_bounds__(kBlock) sigma_level_kernel(const int32_t* orde
   }
 }
 
-/* next_bm: bitmap of level L+1, or nullptr to test depth[]; level_max: the
- * slots of level L */
+/* next_bm: bitmap of level L+1, or nullptr to test depth[] */
 template<typename OffT>
 __global__ void __launch_bounds__(kBlock) delta_level_kernel(const int32_t* order, const int64_t* lvl, int32_t L,
                                                              const uint32_t* hub, int hub_blocks, const OffT* off,
                                                              const int32_t* cols, const int32_t* depth,
                                                              const uint64_t* next_bm, const double* sigma, double* r,
-                                                             const unsigned long long* level_max, double* acc_bc) {
-  const double sc = level_scale(level_max);
+                                                             const double* scale, double* acc_bc) {
+  const double sc = scale[L];
   gather_level<OffT>(
       order, lvl, L, hub, hub_blocks, off, cols, depth, next_bm, L + 1, [&](int32_t w) { return r[w]; },
       [&](int32_t v, double sum) {
@@ -339,10 +355,17 @@ int run_bc(sg_graph_t g, int32_t nsrc, const int32_t* sources, float* out) {
   const OffT* in_off = (const OffT*)(g->inv_offsets ? g->inv_offsets : g->offsets);
   const int32_t* in_cols = g->inv_cols ? g->inv_cols : g->cols;
   const bool directed = in_off != off;
-  /* kept with the graph: repeated calls allocate nothing */
+  /* kept with the graph, so that repeated calls allocate nothing, but no part
+   * of more than kKeepBytes beyond the call: of a graph of 8 M vertices and
+   * more, or of long diameter, the calls take far longer than allocating */
+  struct Trim {
+    sg_graph_t g;
+    ~Trim() { sg::graph_buffers_trim(g, "bc_", kKeepBytes); }
+  } trim{g};
   int32_t *depth = nullptr, *order = nullptr;
   int64_t* lvl = nullptr;
-  double *sigma = nullptr, *r = nullptr, *acc = nullptr;
+  double *sigma = nullptr, *r = nullptr, *acc = nullptr, *scale = nullptr;
+  unsigned long long* level_max = nullptr;
   uint32_t *count = nullptr, *hubs = nullptr, *in_hubs = nullptr;
   const size_t hub_cap = (size_t)(g->m / kHub) + 2;
   SG_TRY(sg::graph_buffer(g, "bc_depth", 4 * (size_t)(n + 1), &depth));
@@ -351,6 +374,7 @@ int run_bc(sg_graph_t g, int32_t nsrc, const int32_t* sources, float* out) {
   SG_TRY(sg::graph_buffer(g, "bc_sigma", 8 * (size_t)(n + 1), &sigma));
   SG_TRY(sg::graph_buffer(g, "bc_r", 8 * (size_t)(n + 1), &r));
   SG_TRY(sg::graph_buffer(g, "bc_acc", 8 * (size_t)(n + 1), &acc));
+  SG_TRY(sg::graph_buffer(g, "bc_level_max", 8 * 3 * kSlotWords, &level_max));
   SG_TRY(sg::graph_buffer(g, "bc_count", 4 * 2 * kCountLevels, &count));
   SG_TRY(sg::graph_buffer(g, "bc_hubs", 4 * hub_cap, &hubs));
   if (directed) SG_TRY(sg::graph_buffer(g, "bc_in_hubs", 4 * hub_cap, &in_hubs));
@@ -381,11 +405,7 @@ int run_bc(sg_graph_t g, int32_t nsrc, const int32_t* sources, float* out) {
     const bool use_lbm = (int64_t)nl * w0 * 8 <= kLevelBitmapBytes;
     uint64_t* lbm = nullptr;
     if (use_lbm) SG_TRY(sg::graph_buffer(g, "bc_lbm", 8 * (size_t)nl * w0, &lbm));
-    const size_t slot_words = (size_t)kMaxSlots * kSlotStride;
-    unsigned long long* level_max = nullptr;
-    SG_TRY(sg::graph_buffer(g, "bc_level_max", 8 * slot_words * (nl + 1), &level_max));
-    fill_i64_kernel<<<sg::grid_for(dev, (int64_t)((nl + 1) * slot_words), kBlock, 4), kBlock, 0, st>>>(
-        (int64_t*)level_max, 0, (int64_t)((nl + 1) * slot_words));
+    SG_TRY(sg::graph_buffer(g, "bc_scale", 8 * (size_t)nl, &scale));
     if (nl <= kCountLevels) {
       uint32_t* cursor = count + kCountLevels;
       fill_i64_kernel<<<1, kBlock, 0, st>>>((int64_t*)count, 0, kCountLevels / 2);
@@ -413,15 +433,15 @@ int run_bc(sg_graph_t g, int32_t nsrc, const int32_t* sources, float* out) {
                                                                                       (int64_t)nl * w0);
       level_bits_kernel<<<sg::grid_for(dev, n, kBlock, 4), kBlock, 0, st>>>(depth, n, w0, nl, lbm);
     }
-    bc_source_init_kernel<<<1, 1, 0, st>>>(sigma, s);
+    bc_source_init_kernel<<<1, kBlock, 0, st>>>(sigma, s, level_max);
     auto lbm_of = [&](int32_t L) -> const uint64_t* { return use_lbm ? lbm + (int64_t)L * w0 : nullptr; };
     for (int32_t L = 1; L < nl; ++L)
       sigma_level_kernel<OffT><<<grid_lvl, kBlock, 0, st>>>(order, lvl, L, nl, in_hubs, hub_blocks, in_off, in_cols,
-                                                            depth, lbm_of(L - 1), sigma, r, level_max + L * slot_words);
+                                                            depth, lbm_of(L - 1), sigma, r, level_max, scale);
     /* the source's own dependency is not counted */
     for (int32_t L = nl - 2; L >= 1; --L)
       delta_level_kernel<OffT><<<grid_lvl, kBlock, 0, st>>>(order, lvl, L, hubs, hub_blocks, off, g->cols, depth,
-                                                            lbm_of(L + 1), sigma, r, level_max + L * slot_words, acc);
+                                                            lbm_of(L + 1), sigma, r, scale, acc);
     SG_HIP(hipGetLastError());
   }
   add_to_float_kernel<<<grid_n, kBlock, 0, st>>>(acc, out, n);

@@ -532,6 +532,19 @@ int graph_buffer(sg_graph_t g, const char* name, size_t bytes, void** out) {
   return SG_OK;
 }
 
+void graph_buffers_trim(sg_graph_t g, const char* prefix, size_t keep) {
+  bool idle = false;
+  for (auto& kv : g->buffers) {
+    auto& e = kv.second;
+    if (!e.first || e.second <= keep || kv.first.compare(0, std::strlen(prefix), prefix) != 0) continue;
+    if (!idle) (void)hipStreamSynchronize(g->dev->stream); /* queued work may still use it */
+    idle = true;
+    (void)hipFree(e.first);
+    e.first = nullptr;
+    e.second = 0;
+  }
+}
+
 void graph_buffers_release(sg_graph_t g) {
   for (auto& kv : g->buffers) (void)hipFree(kv.second.first);
   g->buffers.clear();

@@ -181,6 +181,9 @@ inline int graph_buffer(sg_graph_t g, const char* name, size_t bytes, T** out) {
   *out = static_cast<T*>(p);
   return st;
 }
+/* Free the kept buffers of more than `keep` bytes whose names start with
+ * `prefix`. */
+void graph_buffers_trim(sg_graph_t g, const char* prefix, size_t keep);
 void graph_buffers_release(sg_graph_t g);
 void aux_queues_release(sg_graph_t g);
 

@@ -184,3 +184,35 @@ def test_bc_level_grouping_and_hubs(sg, device, oracle_mod, levels, directed, ba
     assert _close(b.get_values(), ref)
     b.run(batched=batched)
     assert _close(b.get_values(), 2.0 * ref)
+
+
+def test_bc_of_a_long_path_keeps_little_memory(sg, device, oracle_mod):
+    """30,000 levels: what the call keeps with the graph grows with the vertices, not with 8 KiB or a bitmap per
+    level (245 and 112 MB here), and a second call gives the same sums."""
+    import ctypes as C
+    hip = C.CDLL("libamdhip64.so")
+
+    other = sg.BFS(sg.Graph.from_csr(device, np.array([0, 1, 2]), np.array([1, 0])))
+
+    def free_bytes():
+        for _ in range(5):  # the runtime gives memory back with the commands after those that used it
+            other.init(0)
+            other.run(sg.POLICY_PUSH, 15.0, 24.0)
+            other.get_distances()
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    n = 30000
+    g = oracle_mod.csr_from_pairs(n, np.arange(n - 1), np.arange(1, n))
+    ref = oracle_mod.bc(g, [0, 7])
+    G = sg.Graph.from_csr(device, g.offsets, g.cols)
+    b = sg.BC(G)
+    b.init([0, 7])
+    b.run()
+    assert _close(b.get_values(), ref)
+    b.run()
+    assert _close(b.get_values(), 2.0 * ref)
+    held = free_bytes()
+    G.destroy()
+    assert free_bytes() - held < 64 << 20
