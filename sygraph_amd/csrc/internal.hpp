@@ -120,7 +120,8 @@ struct sg_graph_s {
                                     out-degree of the vertex}, or with pull_hint_offsets {that in-neighbour,
                                     low 32 bits of the start of the vertex's list} and entry n = {-1, m} */
   bool pull_hint_offsets = false;
-  double mean_weight = -1.0;     /* mean arc weight, computed on first use (automatic SSSP delta) */
+  bool weight_sum_valid = false; /* the sum of the arc weights is in its buffer (automatic SSSP schedule) */
+  double mean_weight = -1.0;     /* mean arc weight, fetched on first use (automatic SSSP delta) */
   /* SSSP's light-first copy of the adjacency for one bucket width: per vertex
    * the arcs lighter than the width first, then the others */
   int32_t* sssp_cols = nullptr;

@@ -745,6 +745,18 @@ __global__ void __launch_bounds__(kSmallThreads) sssp_small_kernel(SmallArgs<Off
   }
 }
 
+/* automatic delta = half the mean arc weight: of 0.125-1.0 times the mean,
+ * the least geometric mean of time / the run's best (1.026) over the 30
+ * training graphs the rule below sends to buckets (0.25: 1.18; 1.0: 1.19) */
+constexpr double kAutoDeltaFactor = 0.5;
+
+/* The automatic bucket width for a mean arc weight. */
+template<typename W>
+__host__ __device__ inline double auto_delta(double mean) {
+  const double least = DistOps<W>::is_float ? 1e-30 : 1.0, d = kAutoDeltaFactor * mean;
+  return d < least ? least : d;
+}
+
 /* Threshold after a dry iteration: the smallest deferred distance plus
  * delta, at least one representable step above it. */
 template<typename W>
@@ -824,7 +836,7 @@ struct SsspGrid {
   int64_t cap_pieces, grid_arcs;
   uint64_t* far[2]; /* [parity]: far_cap entries per workgroup, vertex | distance << 32 */
   uint32_t far_cap;
-  double step;      /* first step of T; 0: no far list */
+  const double* weight_sum; /* of all arcs, for the first step of T; null: no far list */
   double w_max;
   gb::Exchange x;
   unsigned long long* relax_slots;
@@ -1058,8 +1070,9 @@ __global__ void __launch_bounds__(gb::kThreads) sssp_grid_kernel(SsspGrid<OffT, 
   unsigned long long arcs = h0.deg, entries = h0.nvert, relaxed = 0;
   int32_t rounds = 0;
   const int32_t first_round = ctl->rounds - 1; /* counted by the selection */
-  const bool piles = a.step > 0.0;
-  double step = a.step;                               /* first wave, like what follows */
+  const bool piles = a.weight_sum != nullptr;
+  const double first_step = piles ? 4.0 * auto_delta<W>(*a.weight_sum / (double)a.m) : 0.0;
+  double step = first_step;                           /* first wave, like what follows */
   unsigned long long bucket_arcs = 0, bucket_rounds = 0;
   bool far_pass = piles; /* every thread's; the first sorts the queues into the far lists (T = 0) */
   int fp = 0;            /* the far list in use */
@@ -1192,7 +1205,7 @@ __global__ void __launch_bounds__(gb::kThreads) sssp_grid_kernel(SsspGrid<OffT, 
         if (next == 3) { /* the bucket is done: on by a step, or where that found nothing from the smallest left */
           if (bucket_rounds) {
             if (bucket_arcs < (unsigned long long)kNearFew * bucket_rounds) step *= 2.0;
-            else if (bucket_arcs > (unsigned long long)kNearMany * bucket_rounds && step > a.step / 64) step *= 0.5;
+            else if (bucket_arcs > (unsigned long long)kNearMany * bucket_rounds && step > first_step / 64) step *= 0.5;
           }
           bucket_arcs = bucket_rounds = 0;
           const uint32_t T = next_threshold<W>(far_pass ? ~(uint32_t)t.mx : s_T, step, a.w_max);
@@ -1466,10 +1479,6 @@ void sssp_ws_free(SsspWorkspace* w) {
   delete w;
 }
 
-/* automatic delta = half the mean arc weight: of 0.125-1.0 times the mean,
- * the least geometric mean of time / the run's best (1.026) over the 30
- * training graphs the rule below sends to buckets (0.25: 1.18; 1.0: 1.19) */
-constexpr double kAutoDeltaFactor = 0.5;
 
 int sssp_workspace_for(sg_graph_t g, SsspWorkspace** out) {
   auto* ws = static_cast<SsspWorkspace*>(g->sssp_ws);
@@ -1560,8 +1569,24 @@ int ensure_split(sg_graph_t g, W dlt) {
   return SG_OK;
 }
 
+/* The sum of the arcs' weights in device memory, summed once per graph; no
+ * wait (a host wait for it made a first call on a small graph 2 % longer). */
+template<typename W>
+int weight_sum(sg_graph_t g, const double** out) {
+  double* sum = nullptr;
+  SG_TRY(sg::graph_buffer(g, "sssp_weight_sum", 8, &sum));
+  if (!g->weight_sum_valid) {
+    SG_TRY(sg::zero_async(g->dev, sum, 8));
+    weight_sum_kernel<W><<<sg::grid_for(g->dev, g->m, 256, 4), 256, 0, g->dev->stream>>>((const W*)g->weights, g->m, sum);
+    SG_HIP(hipGetLastError());
+    g->weight_sum_valid = true;
+  }
+  *out = sum;
+  return SG_OK;
+}
+
 template<typename OffT, typename W>
-int run_sssp(sg_graph_t g, int32_t src, double delta, double grid_step, int32_t heavy_pull, int64_t burst_arcs,
+int run_sssp(sg_graph_t g, int32_t src, double delta, bool far_lists, int32_t heavy_pull, int64_t burst_arcs,
              bool record_relax, W* dist_out, sg_sssp_stats* stats) {
   sg_device_t dev = g->dev;
   hipStream_t s = dev->stream;
@@ -1650,7 +1675,7 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, double grid_step, int32_t 
   sa.bellman = bellman ? 1 : 0;
   /* the grid bursts' near and far piles take the small rounds from the start;
    * a record of the relax launches leaves the rounds to them */
-  const bool grid = bellman && burst_arcs > 0 && !record_relax, piles = grid && grid_step > 0.0;
+  const bool grid = bellman && burst_arcs > 0 && !record_relax, piles = grid && far_lists;
   sa.burst_arcs = piles ? 0 : burst_arcs;
   SsspBurst<OffT, W> sb{};
   sb.off = off;
@@ -1696,7 +1721,7 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, double grid_step, int32_t 
     }
     sg_args.cap_pieces = gb::cap_pieces(kSsspGridArcs);
     sg_args.grid_arcs = kSsspGridArcs;
-    sg_args.step = grid_step;
+    if (piles) SG_TRY(weight_sum<W>(g, &sg_args.weight_sum));
     sg_args.far_cap = far_capacity(n, ws->grid_wgs);
     sg_args.w_max = w_max;
     sg_args.x = ws->grid_x;
@@ -1865,20 +1890,14 @@ int run_sssp_small(sg_graph_t g, int32_t src, W* dist, sg_sssp_stats* stats) {
 /* mean arc weight, computed once per graph (automatic delta) */
 template<typename W>
 int mean_weight(sg_graph_t g, double* out) {
-  if (g->mean_weight >= 0.0) {
-    *out = g->mean_weight;
-    return SG_OK;
+  if (!(g->mean_weight >= 0.0)) {
+    const double* sum = nullptr;
+    SG_TRY(weight_sum<W>(g, &sum));
+    double h = 0.0;
+    SG_HIP(hipMemcpyAsync(&h, sum, 8, hipMemcpyDeviceToHost, g->dev->stream));
+    SG_HIP(hipStreamSynchronize(g->dev->stream));
+    g->mean_weight = g->m > 0 ? h / (double)g->m : 1.0;
   }
-  SsspWorkspace* ws = nullptr;
-  SG_TRY(sssp_workspace_for(g, &ws));
-  double* acc = reinterpret_cast<double*>(ws->acc);
-  SG_TRY(sg::zero_async(g->dev, acc, 16));
-  weight_sum_kernel<W><<<sg::grid_for(g->dev, g->m, 256, 4), 256, 0, g->dev->stream>>>((const W*)g->weights, g->m,
-                                                                                       acc);
-  double h = 0.0;
-  SG_HIP(hipMemcpyAsync(&h, acc, 8, hipMemcpyDeviceToHost, g->dev->stream));
-  SG_HIP(hipStreamSynchronize(g->dev->stream));
-  g->mean_weight = g->m > 0 ? h / (double)g->m : 1.0;
   *out = g->mean_weight;
   return SG_OK;
 }
@@ -1905,21 +1924,20 @@ constexpr int64_t kAutoBucketDegree = 8;
 template<typename OffT, typename W>
 int run_sssp_auto(sg_graph_t g, int32_t source, double delta, int32_t heavy_pull, int64_t burst_arcs,
                   bool record_relax, W* dist, sg_sssp_stats* stats) {
-  double grid_step = 0.0;
   /* (an explicit burst length asks for rounds by launches, a record of the
    * relax launches for their times) */
   if (delta == 0.0 && burst_arcs == kSsspBurstDefault && !record_relax && g->n <= kSmallVerts && g->m <= kSmallArcs)
     return run_sssp_small<OffT, W>(g, source, dist, stats);
-  if (delta == 0.0) {
+  bool far_lists = false;
+  if (delta == 0.0 && (g->m < kAutoBucketArcs || g->m < kAutoBucketDegree * (int64_t)g->n)) {
+    far_lists = g->m < kAutoBucketArcs;
+    delta = -1.0;
+  } else if (delta == 0.0) {
     double mw = 1.0;
     SG_TRY(mean_weight<W>(g, &mw));
-    delta = std::max(kAutoDeltaFactor * mw, DistOps<W>::is_float ? 1e-30 : 1.0);
-    if (g->m < kAutoBucketArcs || g->m < kAutoBucketDegree * (int64_t)g->n) {
-      if (g->m < kAutoBucketArcs) grid_step = 4.0 * delta; /* first step of the grid bursts' threshold */
-      delta = -1.0;
-    }
+    delta = auto_delta<W>(mw);
   }
-  return run_sssp<OffT, W>(g, source, delta, grid_step, heavy_pull, burst_arcs, record_relax, dist, stats);
+  return run_sssp<OffT, W>(g, source, delta, far_lists, heavy_pull, burst_arcs, record_relax, dist, stats);
 }
 
 extern "C" {
