@@ -216,3 +216,36 @@ def test_bc_of_a_long_path_keeps_little_memory(sg, device, oracle_mod):
     held = free_bytes()
     G.destroy()
     assert free_bytes() - held < 64 << 20
+
+
+@pytest.mark.parametrize("directed", [False, True])
+@pytest.mark.parametrize("before,after", [(49, 3), (49, 60), (0, 70), (52, 0)])
+def test_batched_bc_goes_on_with_exponents(sg, device, oracle_mod, directed, before, after):
+    """Layers of four vertices, all joined to the next layer's: path counts grow fourfold a level and pass 2^100
+    at the 51st, in lists laid end to end, or in lists of 300 (added up from chunks) where `before` such levels
+    lie ahead of a layer of 300, or at the last level.  A first call, which meets the limit in its first batch
+    and takes that level again with exponents, gives the bits of a second one, which has them from the start."""
+    sizes = [1] + [4] * before + [300] + [4] * after + [1]
+    first = np.concatenate([[0], np.cumsum(sizes)])
+    u, v = [], []
+    for k in range(len(sizes) - 1):
+        a, b = np.meshgrid(first[k] + np.arange(sizes[k]), first[k + 1] + np.arange(sizes[k + 1]), indexing="ij")
+        u.append(a.ravel())
+        v.append(b.ravel())
+    u, v, n = np.concatenate(u), np.concatenate(v), int(first[-1])
+    if directed:
+        off = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=n))]).astype(np.int64)
+        g = oracle_mod.CSRGraph(n, off, v[np.argsort(u, kind="stable")].astype(np.int32))
+    else:
+        g = oracle_mod.csr_from_pairs(n, u, v)
+    srcs = np.concatenate([[0, 0, 1, n - 1], np.arange(70) % n])
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, directed=directed)
+    got = []
+    for _ in range(2):
+        b = sg.BC(G)
+        b.init(srcs)
+        b.run(batched=True)
+        got.append(b.get_values())
+    assert _close(got[0], oracle_mod.bc(g, srcs.tolist(), **({"inverse": oracle_mod.transpose(g)} if directed else {})))
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    G.destroy()
