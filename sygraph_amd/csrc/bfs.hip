@@ -297,9 +297,9 @@ struct BfsCtl {
  * SG_MAX_LEVELS_RECORDED) by finish_level or, inside a burst, by
  * burst_body. */
 struct alignas(64) LevelLog {
-  int32_t level, dir, done, next_dir, action, burst;
+  uint32_t ticks; /* a level of a burst of one workgroup: its time by the constant-rate clock; others 0 */
+  int32_t dir, done, next_dir, action, burst;
   int64_t f_vertices, f_edges, disc, disc_deg, edges, scanned, misses, max_deg, unexplored;
-  int64_t ticks; /* a level of a burst of one workgroup: its time by the constant-rate clock; others 0 */
 };
 
 /* One step's record (a step = the launches the host enqueues together: one
@@ -338,6 +338,7 @@ struct DecideParams {
   const float* mlp;     /* learned policy parameters (SG_POLICY_LEARNED) */
   float f6, f7;         /* the graph's constant features (average degree, vertex count) */
   int64_t burst_arcs;   /* frontier arcs up to which push levels run in a burst (0: never) */
+  int32_t timed;        /* levels are recorded: a burst of one workgroup takes their times */
   unsigned long long learned_gate; /* learned policy: a level whose frontier has fewer arcs than the
                                       graph's arcs / learned_gate pushes (variant 0) without asking the
                                       network; 0: the network decides every level */
@@ -521,7 +522,7 @@ __device__ __forceinline__ void finish_level(const FinishArgs& f, BfsCtl* ctl, c
   const int32_t done = disc == 0 ? 1 : 0;
   if (level < SG_MAX_LEVELS_RECORDED) {
     LevelLog e;
-    e.level = level;
+    e.ticks = 0;
     e.dir = dir;
     e.done = done;
     e.next_dir = next;
@@ -536,7 +537,6 @@ __device__ __forceinline__ void finish_level(const FinishArgs& f, BfsCtl* ctl, c
     e.misses = (int64_t)misses;
     e.max_deg = (int64_t)max_deg;
     e.unexplored = (int64_t)(p.total_degree - vdeg);
-    e.ticks = 0;
     f.levlog[level] = e;
   }
   const int32_t n_push = ctl->n_push + (dir == 0 ? 1 : 0), n_pull = ctl->n_pull + (dir == 0 ? 0 : 1);
@@ -804,12 +804,15 @@ __device__ __forceinline__ void burst_visit_big(const BurstArgs<OffT>& a, const 
 template<bool kLds, typename OffT>
 __device__ __forceinline__ void burst_body(const BurstArgs<OffT>& a, BfsCtl* ctl, const DecideParams& p,
                                            int32_t step, LevelLog* levlog, StepLog* steplog, bool publish) {
-  int64_t mark = (int64_t)wall_clock64(), now = mark; /* the levels' times, which no event stands between */
+  __shared__ int64_t s_mark; /* the levels' times, as no event stands between them: when the last one ended */
   __shared__ sg::policy::Staged s_pol;
   __shared__ uint32_t s_count[2][2];
   __shared__ unsigned long long s_red[2][kBurstWaves][5];
   stage_policy(p, &s_pol);
-  if (threadIdx.x == 0) s_count[0][0] = s_count[0][1] = 0;
+  if (threadIdx.x == 0) {
+    s_count[0][0] = s_count[0][1] = 0;
+    if (p.timed) s_mark = (int64_t)wall_clock64();
+  }
   const int lane = lane_id(), wv = threadIdx.x >> 6;
   int32_t level = ctl->level, lb = ctl->lb;
   int64_t f_vertices = ctl->f_vertices, f_edges = ctl->f_edges;
@@ -870,11 +873,9 @@ __device__ __forceinline__ void burst_body(const BurstArgs<OffT>& a, BfsCtl* ctl
     act = decide_action(p, &s_pol, 0, disc, disc_deg, unexplored, level + 1, max_deg);
     done = disc == 0 ? 1 : 0;
     const bool more = !done && act / 3 == 0 && (int64_t)disc_deg <= p.burst_arcs;
-    now = (int64_t)wall_clock64();
     if (!more && !done) break; /* the next step counts and decides this level (hand-back) */
     if (threadIdx.x == 0 && level < SG_MAX_LEVELS_RECORDED) {
       LevelLog e;
-      e.level = level;
       e.dir = 0;
       e.done = done;
       e.next_dir = act / 3;
@@ -889,10 +890,14 @@ __device__ __forceinline__ void burst_body(const BurstArgs<OffT>& a, BfsCtl* ctl
       e.misses = 0;
       e.max_deg = (int64_t)max_deg;
       e.unexplored = (int64_t)unexplored;
-      e.ticks = now - mark;
+      e.ticks = 0;
+      if (p.timed) {
+        const int64_t now = (int64_t)wall_clock64();
+        e.ticks = (uint32_t)(now - s_mark);
+        s_mark = now;
+      }
       levlog[level] = e;
     }
-    mark = now;
     vdeg += disc_deg;
     reached += disc;
     ++n_push;
@@ -928,7 +933,7 @@ __device__ __forceinline__ void burst_body(const BurstArgs<OffT>& a, BfsCtl* ctl
     sl.reached_v = (int64_t)reached;
     sl.reached_e = (int64_t)vdeg;
     sl.next_f_edges = f_edges; /* the level handed back, a push level */
-    sl.ticks = done ? 0 : now - mark;
+    sl.ticks = done || !p.timed ? 0 : (int64_t)wall_clock64() - s_mark;
     /* the step's record, unless the step's own count pass writes it later
      * (a burst ahead of the step that hands a level back) */
     if (publish || done) publish_step(&steplog[step % kRing], sl);
@@ -1072,8 +1077,13 @@ struct GbOut {
 
 /* Claim the (up to) K arcs y[k] of each lane; new vertices get depth
  * level + 1 and join the workgroup's segment or, cut into pieces, the long
- * list.  Two memory round trips: the visited words with the heads' list
- * bounds, then the claims with the heads of the short lists. */
+ * list.  One arc per lane (small levels) takes two memory round trips: the
+ * visited word with the head's list bounds, then the claim with the heads of
+ * a short list.  Four take three, the bounds with the claims, for the heads
+ * not yet visited only: larger levels wait for their loads (layers of 2,000 to
+ * 32,000 vertices and 4 or 12 arcs each way, 23,000 to 360,000 arcs a level:
+ * 4 to 36 % longer with all bounds loaded first, and up to 35 % longer than
+ * the launched levels and bursts before inline lists). */
 template<int K, typename OffT>
 __device__ __forceinline__ void gb_claim(const GbArgs<OffT>& a, const uint32_t (&y)[K], const bool (&ok)[K],
                                          const GbOut<OffT>& o, gb::Acc& acc) {
@@ -1085,7 +1095,7 @@ __device__ __forceinline__ void gb_claim(const GbArgs<OffT>& a, const uint32_t (
     vs[k] = ve[k] = 0;
     if (ok[k]) {
       w[k] = a.visited[y[k] >> 6];
-      list_bounds(a.off, y[k], vs[k], ve[k]);
+      if constexpr (K == 1) list_bounds(a.off, y[k], vs[k], ve[k]);
     }
   }
   uint64_t old[K];
@@ -1096,8 +1106,19 @@ __device__ __forceinline__ void gb_claim(const GbArgs<OffT>& a, const uint32_t (
     const uint64_t bit = 1ull << (y[k] & 63);
     nw[k] = !(w[k] & bit);
     old[k] = ~0ull;
-    if (nw[k]) old[k] = atomic_or(&a.visited[y[k] >> 6], bit);
-    if (nw[k] && ve[k] - vs[k] <= gb::kInline) load_ids4(a.cols, vs[k], a.m, id[k]);
+    if (nw[k]) {
+      old[k] = atomic_or(&a.visited[y[k] >> 6], bit);
+      if constexpr (K > 1) {
+        list_bounds(a.off, y[k], vs[k], ve[k]);
+      } else if (ve[k] - vs[k] <= gb::kInline) {
+        load_ids4(a.cols, vs[k], a.m, id[k]);
+      }
+    }
+  }
+  if constexpr (K > 1) {
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (nw[k] && ve[k] - vs[k] <= gb::kInline) load_ids4(a.cols, vs[k], a.m, id[k]);
   }
   uint64_t ms[K];
   uint32_t cs = 0;
@@ -1206,13 +1227,31 @@ __device__ __forceinline__ void gb_merge_path(const GbArgs<OffT>& a, int64_t sta
  * entries of segment w, most: of the longest.  Where every list's heads are
  * in its entry, each lane takes one arc: a wave's time is its instructions and
  * divergent loads, a lookup per lane each, and one arc per lane spreads a
- * small level's over four times the waves of four.  An entry's vertex joins
+ * small level's over four times the waves of four.  Where lists are longer on
+ * average and a wave would take several steps (`wide`), it takes 64 entries at
+ * once, which fill its rounds of 256 arcs.  An entry's vertex joins
  * prev last, so that nothing waits for that atomic before the level's end
  * (nothing in the burst reads prev). */
 template<typename OffT>
 __device__ __forceinline__ void gb_visit_list(const GbArgs<OffT>& a, const uint64_t* in, const uint32_t* s_n,
-                                              uint32_t most, const GbOut<OffT>& o, gb::Acc& acc) {
+                                              uint32_t most, bool wide, const GbOut<OffT>& o, gb::Acc& acc) {
   const int lane = lane_id();
+  if (__builtin_expect(wide, 0)) {
+    for (uint32_t k0 = threadIdx.x >> 6; k0 * gb::kGroup < most; k0 += 64 / gb::kGroup * gb::kWaves) {
+      const uint32_t k = k0 + (uint32_t)lane / gb::kGroup * gb::kWaves, w = gb::segment_of(k, o.rank, o.wgs);
+      const uint32_t i = k * gb::kGroup + (uint32_t)lane % gb::kGroup;
+      const int64_t e = gb::entry_at(w, i, o.wgs);
+      const bool has = i < s_n[w];
+      uint64_t e0 = 0;
+      if (has) e0 = atomic_load(in + e);
+      const uint32_t len = (uint32_t)(e0 >> 32);
+      int64_t start = 0;
+      if (has) start = len > (uint32_t)gb::kInline ? (int64_t)atomic_load(in + a.total + e) : (int64_t)a.off[(uint32_t)e0];
+      gb_merge_path(a, start, len, o, acc);
+      if (has) atomic_or(&a.prev[(uint32_t)e0 >> 6], 1ull << (e0 & 63));
+    }
+    return;
+  }
   for (uint32_t k = threadIdx.x >> 6; k * gb::kGroup < most; k += gb::kWaves) {
     const uint32_t w = gb::segment_of(k, o.rank, o.wgs);
     if (k * gb::kGroup >= s_n[w]) continue;
@@ -1227,7 +1266,7 @@ __device__ __forceinline__ void gb_visit_list(const GbArgs<OffT>& a, const uint6
       y[0] = atomic_load(reinterpret_cast<const uint32_t*>(in + 2 * a.total) + gb::kInline * e + sub);
     }
     const uint32_t len = (uint32_t)(e0 >> 32);
-    if (ballot(len > (uint32_t)gb::kInline)) {
+    if (__builtin_expect(ballot(len > (uint32_t)gb::kInline) != 0, 0)) {
       int64_t start = 0; /* the entry's first lane lays its list */
       if (has && sub == 0)
         start = len > (uint32_t)gb::kInline ? (int64_t)atomic_load(in + a.total + e) : (int64_t)a.off[(uint32_t)e0];
@@ -1271,6 +1310,7 @@ __global__ void __launch_bounds__(gb::kThreads) gburst_kernel(GbArgs<OffT> a, Bf
   __shared__ sg::policy::Staged s_pol;
   __shared__ uint32_t s_n[kGbMaxWgs], s_most;
   __shared__ gb::Local s_local;
+  __shared__ int32_t s_wide;
   __shared__ int32_t s_next; /* 0: another level, 1: none, 2: a wait ran out */
   __shared__ int64_t s_pieces;
   if (blockIdx.x % a.stride) return;
@@ -1301,7 +1341,7 @@ __global__ void __launch_bounds__(gb::kThreads) gburst_kernel(GbArgs<OffT> a, Bf
     gb::Acc acc{0, 0, 0, 0};
     const GbOut<OffT> o{a.list[cur ^ 1], rank, wgs, a.pieces[cur ^ 1], a.x.sums + (it % 3), &s_local,
                         first_level + it};
-    if (it == 0) {
+    if (__builtin_expect(it == 0, 0)) {
       for (int64_t base = (int64_t)gwave * 64; base < h0.count[0]; base += (int64_t)nwaves * 64) {
         QEntry qe{0, 0, 0};
         if (base + lane < h0.count[0]) qe = a.q[0][base + lane];
@@ -1310,7 +1350,7 @@ __global__ void __launch_bounds__(gb::kThreads) gburst_kernel(GbArgs<OffT> a, Bf
       gb_visit_pieces(a, a.q[1], h0.count[1], o, acc, gwave, nwaves, false);
       gb_visit_pieces(a, a.q[2], h0.count[2], o, acc, gwave, nwaves, false);
     } else {
-      gb_visit_list(a, a.list[cur], s_n, s_most, o, acc);
+      gb_visit_list(a, a.list[cur], s_n, s_most, s_wide != 0, o, acc);
       gb_visit_pieces(a, a.pieces[cur], s_pieces, o, acc, gwave, nwaves, true);
     }
     gb::add_local(&s_local, acc);
@@ -1330,7 +1370,7 @@ __global__ void __launch_bounds__(gb::kThreads) gburst_kernel(GbArgs<OffT> a, Bf
             /* into device memory: a store to the host's would hold up this
              * wave's next wait for its stores by a trip over the host link */
             LevelLog e;
-            e.level = level;
+            e.ticks = 0;
             e.dir = 0;
             e.done = done;
             e.next_dir = act / 3;
@@ -1345,7 +1385,6 @@ __global__ void __launch_bounds__(gb::kThreads) gburst_kernel(GbArgs<OffT> a, Bf
             e.misses = 0;
             e.max_deg = (int64_t)t.mx;
             e.unexplored = (int64_t)unexplored;
-            e.ticks = 0;
             a.log[level] = e;
           }
           vdeg += t.deg;
@@ -1361,6 +1400,11 @@ __global__ void __launch_bounds__(gb::kThreads) gburst_kernel(GbArgs<OffT> a, Bf
       if (lane == 0) {
         s_next = next;
         s_most = t.most;
+        /* lists longer than an entry carries on average, and more than two
+         * steps of 16 entries for a wave: 64 at once fill its rounds of 256
+         * arcs (layers of 16,000 vertices and 4 arcs each way, 168,000 arcs a
+         * level: 1.72 ms by 16, 1.55 so) */
+        s_wide = t.deg > gb::kInline * t.disc && t.most > 2 * gb::kGroup * gb::kWaves;
         s_pieces = (int64_t)t.npieces;
       }
     }
@@ -1645,6 +1689,7 @@ int run_bfs(sg_graph_t g, int32_t src, const sg_bfs_options& opt, int32_t* depth
   P.f6 = sg::policy::feature(6, 0, 0, 0, 0, 0, (double)n, (double)g->m);
   P.f7 = sg::policy::feature(7, 0, 0, 0, 0, 0, (double)n, (double)g->m);
   P.burst_arcs = burst_arcs;
+  P.timed = timed ? 1 : 0;
   P.learned_gate = opt.learned_gate < 0 ? 0ull
                                         : (unsigned long long)(opt.learned_gate == 0 ? kLearnedGateDefault : opt.learned_gate);
   if (want_total) SG_HIP(hipEventRecord(ws->ev_begin, s));

@@ -481,3 +481,28 @@ def test_record_levels_times_every_level(sg, device, oracle_mod, graph, policy):
         assert min(x.convert_ms for x in levels) >= 0
         assert sum(x.kernel_ms + x.convert_ms for x in levels) <= 1.02 * st.kernel_ms + 0.01
     G.destroy()
+
+
+@pytest.mark.parametrize("offset_bytes", [4, 8])
+@pytest.mark.parametrize("workgroups", [1, 2, 4, 32])
+def test_grid_burst_large_levels(sg, device, oracle_mod, workgroups, offset_bytes):
+    """Levels of about 1,500 lists of 1 to 70 arcs and more, which few workgroups take 64 lists at a time and
+    more workgroups 16: the oracle's depths and the records of the levels run on their own."""
+    u, v, n = _layers(77, layers=40, width=1500)
+    perm = np.random.default_rng(78).permutation(n)
+    g = oracle_mod.csr_from_pairs(n, perm[u], perm[v])
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, offset_bytes=offset_bytes)
+    src = int(perm[:1500][np.nonzero(g.degrees()[perm[:1500]] > 0)[0][0]])
+    ref, levels = oracle_mod.bfs(g, src)
+    runs = []
+    for grid in (-1, 0):
+        b = sg.BFS(G)
+        b.init(src)
+        st = b.run(sg.POLICY_PUSH, tuning={"burst_arcs": -1, "grid_burst_arcs": grid,
+                                           "grid_burst_workgroups": workgroups}, record_levels=False)
+        assert np.array_equal(b.get_distances(), ref), grid
+        runs.append((st.levels, [(x.frontier_vertices, x.frontier_edges, x.discovered, x.unexplored_edges, x.max_degree)
+                                 for x in st.level[:st.levels]]))
+        assert (sum(x.burst == 2 for x in st.level[:st.levels]) > levels // 2) == (grid >= 0)
+    assert runs[0][0] == levels and runs[1] == runs[0]
+    assert max(x[1] / x[0] for x in runs[0][1]) > 8 and max(x[0] for x in runs[0][1]) > 1200
