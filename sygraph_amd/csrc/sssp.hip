@@ -374,6 +374,11 @@ __device__ __forceinline__ void record_round(unsigned long long* rounds, int64_t
   rounds[2 * r + 1] = arcs;
 }
 constexpr int kSsspBurstDefault = 4096;
+/* With far lists the grid bursts take the rounds from the start but for those
+ * of a few arcs, which one workgroup takes faster, to the end on a path
+ * (20,000 vertices: 53.6 ms, in a grid burst 67), and hands over as the queues
+ * of the round that is larger. */
+constexpr int64_t kTinyArcs = 8;
 constexpr int kSsspBurstMax = 8192; /* entries (and arcs) of a burst round; LDS for its scan */
 
 template<typename OffT, typename W>
@@ -387,6 +392,9 @@ struct SsspBurst {
   const QueueHdr* hdr;
   QEntry* list[2]; /* kSsspBurstMax entries each */
   int64_t burst_arcs;
+  int hand_over; /* a round beyond burst_arcs goes to the queues (out_hdr counts them) and not to the bitmap */
+  QueueHdr* out_hdr;
+  Tuning tune;
   unsigned long long* relax_slots;
   unsigned long long* rounds; /* record_round's */
   uint32_t* arrive; /* kArriveWords zeroed words */
@@ -397,6 +405,8 @@ __device__ __forceinline__ void sssp_burst(const SsspBurst<OffT, W>& b, SsspCtl*
   __shared__ uint32_t s_pref[kSsspBurstMax + 1];
   __shared__ uint32_t s_wtot[kBlock / 64];
   __shared__ uint32_t s_next, s_next_arcs;
+  __shared__ uint32_t s_class[3];
+  __shared__ unsigned long long s_deg, s_maxdeg;
   const QueueHdr h = *b.hdr;
   const uint32_t n0 = h.count[0], n1 = h.count[1];
   uint32_t cnt = h.count[0] + h.count[1] + h.count[2];
@@ -484,6 +494,41 @@ __device__ __forceinline__ void sssp_burst(const SsspBurst<OffT, W>& b, SsspCtl*
     }
     __syncthreads();
     cnt = nc;
+  }
+  const uint32_t nc = s_next;
+  if (b.hand_over && nc != 0 && nc <= (uint32_t)kSsspBurstMax) { /* uniform: the same in every thread */
+    const QEntry* out = b.list[(rounds - 1) & 1];
+    if (threadIdx.x < 3) s_class[threadIdx.x] = 0;
+    if (threadIdx.x == 0) s_deg = s_maxdeg = 0;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < nc; i += kBlock) {
+      const QEntry e = out[i];
+      atomic_and(&b.dirty[(uint32_t)e.v >> 6], ~(1ull << (e.v & 63)));
+      const int cls = e.len < b.tune.t_medium ? 0 : e.len < b.tune.t_large ? 1 : 2;
+      const uint32_t pieces = cls < 2 ? 1u : (uint32_t)((e.len + b.tune.chunk - 1) / b.tune.chunk);
+      const uint32_t at = atomicAdd(&s_class[cls], pieces);
+      if (cls < 2) b.q[cls][at] = e;
+      for (uint32_t c = 0; cls == 2 && c < pieces; ++c)
+        b.q[2][at + c] = QEntry{e.start + (int64_t)c * b.tune.chunk, e.v,
+                                min(b.tune.chunk, e.len - (int32_t)c * b.tune.chunk)};
+      atomicAdd(&s_deg, (unsigned long long)e.len);
+      atomicMax(&s_maxdeg, (unsigned long long)e.len);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      QueueHdr o{};
+      for (int k = 0; k < 3; ++k) o.count[k] = s_class[k];
+      o.nvert = nc;
+      o.deg = s_deg;
+      o.maxdeg = s_maxdeg;
+      *b.out_hdr = o;
+      record_round(b.rounds, first_round + rounds, nc, s_deg);
+      ctl->rounds += rounds;
+      ctl->relaxed += arcs + s_deg - (unsigned long long)h.deg;
+      ctl->burst = 0;
+      atomic_add(&b.relax_slots[0], arcs);
+    }
+    return;
   }
   if (threadIdx.x == 0) {
     /* the selection counted the first round; the relax launch has nothing left */
@@ -822,7 +867,7 @@ struct SsspGrid {
   const OffT* off;
   const int32_t* cols;
   const W* w;
-  int64_t m;
+  int64_t m, mean; /* arcs; of a vertex */
   uint32_t* dist;
   uint64_t* dirty;
   QEntry* q[3]; /* the round's queues */
@@ -1062,6 +1107,10 @@ __global__ void __launch_bounds__(gb::kThreads) sssp_grid_kernel(SsspGrid<OffT, 
   const QueueHdr h0 = *a.hdr;
   /* the same for every workgroup */
   if (ctl->done || !ctl->relax || ctl->pull || (int64_t)h0.deg > a.grid_arcs) return;
+  /* a source of so many arcs that the next round, at the mean of arcs per
+   * vertex, is far beyond the burst's: sorting it into the far lists and out
+   * of them again is for nothing (a clique of 1,800: 445 us, without 390) */
+  if (ctl->rounds == 1 && (int64_t)h0.deg * a.mean > 2 * a.grid_arcs) return;
   const uint32_t rank = blockIdx.x / a.stride, wgs = gridDim.x / a.stride;
   const int lane = lane_id(), wv = threadIdx.x >> 6;
   const uint32_t gwave = (uint32_t)wv * wgs + rank, nwaves = wgs * gb::kWaves; /* across the workgroups first */
@@ -1208,7 +1257,10 @@ __global__ void __launch_bounds__(gb::kThreads) sssp_grid_kernel(SsspGrid<OffT, 
             else if (bucket_arcs > (unsigned long long)kNearMany * bucket_rounds && step > first_step / 64) step *= 0.5;
           }
           bucket_arcs = bucket_rounds = 0;
-          const uint32_t T = next_threshold<W>(far_pass ? ~(uint32_t)t.mx : s_T, step, a.w_max);
+          uint32_t from = far_pass ? ~(uint32_t)t.mx : s_T;
+          /* the first bucket counts from the source, wherever the burst starts */
+          if (it == 0 && (double)DistOps<W>::value(from) < step) from = 0;
+          const uint32_t T = next_threshold<W>(from, step, a.w_max);
           if (lane == 0) s_T = T;
         }
       }
@@ -1676,7 +1728,7 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, bool far_lists, int32_t he
   /* the grid bursts' near and far piles take the small rounds from the start;
    * a record of the relax launches leaves the rounds to them */
   const bool grid = bellman && burst_arcs > 0 && !record_relax, piles = grid && far_lists;
-  sa.burst_arcs = piles ? 0 : burst_arcs;
+  sa.burst_arcs = piles ? kTinyArcs : burst_arcs;
   SsspBurst<OffT, W> sb{};
   sb.off = off;
   sb.cols = g->cols;
@@ -1687,7 +1739,10 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, bool far_lists, int32_t he
   sb.hdr = Q.hdr;
   sb.list[0] = ws->burst_list[0];
   sb.list[1] = ws->burst_list[1];
-  sb.burst_arcs = burst_arcs;
+  sb.burst_arcs = sa.burst_arcs;
+  sb.hand_over = piles ? 1 : 0;
+  sb.out_hdr = Q.hdr;
+  sb.tune = tune;
   sb.relax_slots = ws->relax_slots;
   sb.rounds = rounds_log;
   sb.arrive = ws->arrive + kArriveWords;
@@ -1708,6 +1763,7 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, bool far_lists, int32_t he
     sg_args.cols = g->cols;
     sg_args.w = (const W*)g->weights;
     sg_args.m = g->m;
+    sg_args.mean = g->m / n;
     sg_args.dist = dist;
     sg_args.dirty = dirty;
     for (int k = 0; k < 3; ++k) sg_args.q[k] = Q.q[0][k];
@@ -1807,14 +1863,14 @@ int run_sssp(sg_graph_t g, int32_t src, double delta, bool far_lists, int32_t he
     stats->relax_ms = relax_ms;
     stats->relax_launches = relax_launches;
     {
-      unsigned long long rs[16 * kSlots];
-      SG_HIP(hipMemcpyAsync(rs, ws->relax_slots, sizeof(rs), hipMemcpyDeviceToHost, s));
-      auto* rl = static_cast<unsigned long long*>(dev->host_scratch);
-      const int32_t recorded = std::min(round, (int32_t)SG_MAX_LEVELS_RECORDED);
-      if (rounds_log && recorded > 0)
-        SG_HIP(hipMemcpyAsync(rl, rounds_log, 16 * (size_t)recorded, hipMemcpyDeviceToHost, s));
+      /* the relax counts and, behind them, the bursts' rounds, in one copy */
+      const auto* rs = static_cast<const unsigned long long*>(dev->host_scratch);
+      const auto* rl = rs + 16 * kSlots;
+      const int32_t recorded = rounds_log ? std::min(round, (int32_t)SG_MAX_LEVELS_RECORDED) : 0;
+      SG_HIP(hipMemcpyAsync(dev->host_scratch, ws->relax_slots, 8 * 16 * kSlots + 16 * (size_t)recorded,
+                            hipMemcpyDeviceToHost, s));
       SG_HIP(hipStreamSynchronize(s));
-      for (int32_t r = 0; rounds_log && r < recorded; ++r) {
+      for (int32_t r = 0; r < recorded; ++r) {
         if (rl[2 * r] == 0) continue;
         stats->round_vertices[r] = (int64_t)rl[2 * r];
         stats->round_edges[r] = (int64_t)rl[2 * r + 1];

@@ -732,3 +732,37 @@ def test_sssp_round_records_add_up(sg, device, oracle_mod, graph, burst, delta):
         assert min(st.round_vertices[:st.rounds]) > 0
         assert sum(st.round_edges[:st.rounds]) == st.relaxations
     G.destroy()
+
+
+@pytest.mark.parametrize("offset_bytes", [4, 8])
+@pytest.mark.parametrize("directed", [False, True])
+@pytest.mark.parametrize("weight_float", [False, True])
+def test_sssp_tiny_rounds_hand_over(sg, device, oracle_mod, offset_bytes, directed, weight_float):
+    """A path (rounds of a few arcs, which one workgroup takes) into vertices of 3, 70 and 9,000 arcs, one after
+    another with paths between them: what the workgroup hands over holds short lists, long ones and pieces."""
+    u, v, at, fresh = [], [], 0, 400
+    for k, d in enumerate((3, 70, 9000, 12)):
+        step = np.arange(at, at + 60)
+        leaves = fresh + np.arange(d)
+        u += [step, np.full(d, at + 60)]
+        v += [step + 1, leaves]
+        at, fresh = at + 60, fresh + d
+    n = 20000
+    u, v = np.concatenate(u), np.concatenate(v)
+    if directed:
+        off = np.concatenate([[0], np.cumsum(np.bincount(u, minlength=n))]).astype(np.int64)
+        g = oracle_mod.CSRGraph(n, off, v[np.lexsort((v, u))].astype(np.int32))
+    else:
+        g = oracle_mod.csr_from_pairs(n, u, v)
+    w = (oracle_mod.fill_weights(g, 21) % 8 + 1).astype(np.uint32)
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, weights=w.astype(np.float32) if weight_float else w,
+                          weight_float=weight_float, directed=directed, offset_bytes=offset_bytes)
+    for source in (0, 239):
+        ref = oracle_mod.sssp(g, source, w)
+        s = sg.SSSP(G)
+        s.init(source)
+        st = s.run()
+        assert np.array_equal(s.get_distances(), ref)
+        assert st.reached_vertices == (ref != n + 1).sum() > 10
+        assert sum(st.round_edges[:st.rounds]) == st.relaxations >= st.reached_edges
+    G.destroy()
