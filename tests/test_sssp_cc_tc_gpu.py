@@ -766,3 +766,86 @@ def test_sssp_tiny_rounds_hand_over(sg, device, oracle_mod, offset_bytes, direct
         assert st.reached_vertices == (ref != n + 1).sum() > 10
         assert sum(st.round_edges[:st.rounds]) == st.relaxations >= st.reached_edges
     G.destroy()
+
+
+@pytest.mark.parametrize("offset_bytes", [4, 8])
+@pytest.mark.parametrize("weight_float", [False, True])
+@pytest.mark.parametrize("kind", ["grid", "layers", "directed", "overflow", "left"])
+def test_sssp_far_lists(sg, device, oracle_mod, kind, weight_float, offset_bytes):
+    """The automatic schedule's near and far lists, from many threshold moves (a grid), long and short lists in
+    layers, more put off in a round than a workgroup's far list holds (1,024 vertices; `overflow`: 120,000 at
+    once, the rest left to the bitmap), and a round too large for the burst while others are put off (`left`):
+    the distances of the launched rounds of the reference's schedule, bit for bit, and the oracle's."""
+    rng = np.random.default_rng(50)
+    far = None
+    if kind == "grid":
+        g = oracle_mod.grid(260, 300, 0.05, seed=28)
+    elif kind in ("layers", "directed"):
+        layers, width = 60, 900
+        u = np.concatenate([np.repeat(np.arange(k * width, (k + 1) * width), rng.integers(0, 12, width) ** 2 // 8)
+                            for k in range(layers - 1)])
+        v, n = (u // width + 1) * width + rng.integers(0, width, len(u)), layers * width
+        if kind == "layers":
+            g = oracle_mod.csr_from_pairs(n, u, v)
+        else:
+            key = np.unique(u.astype(np.int64) * n + v)
+            off = np.concatenate([[0], np.cumsum(np.bincount(key // n, minlength=n))]).astype(np.int64)
+            g = oracle_mod.CSRGraph(n, off, (key % n).astype(np.int32))
+    else:
+        # 0 -> 100 mids -> 1,200 leaves each, over heavy arcs; elsewhere many light ones keep the mean weight low
+        mids, leaves = np.arange(1, 101), 101 + np.arange(120000)
+        n = 170000
+        u, v = [np.zeros(100, dtype=np.int64), np.repeat(mids, 1200), leaves], [mids, leaves, np.roll(leaves, 17)]
+        if kind == "left":  # ... the first mid has more light arcs than a burst's round, and some leaves are put off by then
+            u += [np.full(40000, 1), np.zeros(50, dtype=np.int64)]
+            v += [125000 + np.arange(40000), leaves[:50]]
+            u.append(125000 + np.repeat(np.arange(40000), 4))
+            v.append(125000 + rng.integers(0, 40000, 160000))
+        u.append(165000 + rng.integers(0, 5000, 900000))
+        v.append(165000 + rng.integers(0, 5000, 900000))
+        u, v = np.concatenate(u), np.concatenate(v)
+        keep = u != v
+        g = oracle_mod.csr_from_pairs(n, u[keep], v[keep])
+        far = (101, 120101)
+    w = oracle_mod.fill_weights(g, 3) if kind != "directed" else rng.integers(1, 256, g.m).astype(np.uint32)
+    if far:
+        row = np.repeat(np.arange(g.n), np.diff(g.offsets))
+        heavy = ((row >= far[0]) & (row < far[1])) | ((g.cols >= far[0]) & (g.cols < far[1]))
+        w = np.where(heavy, 200 + w % 50, 1 + w % 2).astype(np.uint32)
+    wd = (w / 7.0).astype(np.float32) if weight_float else w
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, weights=wd, weight_float=weight_float,
+                          directed=kind == "directed", offset_bytes=offset_bytes)
+    assert g.n > 16384 and g.m < 1 << 25
+    src = 0 if far else int(np.nonzero(g.degrees() > 0)[0][0])
+    got = []
+    for delta, burst in ((-1.0, -1), (0.0, 0), (0.0, 0), (0.0, 64)):
+        s = sg.SSSP(G)
+        s.init(src)
+        st = s.run(delta=delta, burst_arcs=burst)
+        got.append(s.get_distances())
+        assert np.array_equal(got[0].view(np.uint32), got[-1].view(np.uint32)), (delta, burst)
+        if st.rounds <= sg.MAX_LEVELS_RECORDED:
+            assert sum(st.round_edges[:st.rounds]) == st.relaxations
+    if not weight_float:
+        assert np.array_equal(got[0], oracle_mod.sssp(g, src, w))
+    G.destroy()
+
+
+@pytest.mark.parametrize("rows,cols", [(20, 20), (32, 32), (60, 70), (16, 1100), (32, 1200)])
+def test_sssp_distances_beyond_the_vertex_count(sg, device, oracle_mod, rows, cols):
+    """n + 1 is both the value that distances start from and the one that stands for unreached
+    (algorithms/sssp.hpp:43): a vertex whose distance is n + 1 or more stays unreached, in every schedule."""
+    g = oracle_mod.grid(rows, cols, 0.05, seed=30)
+    oracle_mod.fill_weights(g, 31)
+    src = int(np.nonzero(g.degrees() > 0)[0][0])
+    ref = oracle_mod.sssp(g, src)
+    assert (ref == g.n + 1).sum() > 0.3 * g.n
+    G = sg.Graph.from_csr(device, g.offsets, g.cols, weights=g.weights)
+    for delta, burst in ((0.0, 0), (-1.0, 0), (-1.0, -1), (64.0, 0)):
+        s = sg.SSSP(G)
+        s.init(src)
+        st = s.run(delta=delta, burst_arcs=burst)
+        assert np.array_equal(s.get_distances(), ref), (delta, burst)
+        assert st.reached_vertices == (ref != g.n + 1).sum()
+        assert st.reached_edges == g.degrees()[ref != g.n + 1].sum()
+    G.destroy()
