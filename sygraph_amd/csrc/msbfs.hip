@@ -1126,10 +1126,15 @@ __device__ __forceinline__ void load_head(unsigned long long* dst, const LevelIn
  * waves), which costs the power-law graphs' big levels 7 %.  MS-BFS and the
  * batches with exponents fit in three; the plain batches, whose time is row
  * reads, take five (RMAT scale 20, 64 sources: 12.7 ms with three, 11.1 with
- * four, 9.8 with five). */
-constexpr int ms_waves(bool bc, bool plain) { return bc && plain ? 5 : 3; }
-template<bool kBc, bool kPlain, typename OffT>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(ms_waves(kBc, kPlain)))) ms_kernel(MsArgs<OffT> a) {
+ * four, 9.8 with five), at 96 registers and 118 more in scratch.  Batches of
+ * few pairs, one workgroup per CU, have no use for the waves and wait for the
+ * scratch on every level: they take the plain kernel with three and none (a
+ * path of 20,000 vertices, 20 sources: 440 -> 340 ms, 378 before the plain
+ * kernel; a 32 x 32 grid, 3 sources: 1,500 -> 1,195 us, 1,327 before; 6,000
+ * vertices of 6 arcs, 5 sources: 389 -> 351; RMAT of 1,024 vertices: equal). */
+constexpr int kRowWaves = 5, kFewWaves = 3;
+template<bool kBc, bool kPlain, int kWaves, typename OffT>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWaves))) ms_kernel(MsArgs<OffT> a) {
   __shared__ sg::policy::Staged s_pol;
   __shared__ int32_t s_stage[kBlock / 64][kStage];
   __shared__ unsigned long long s_red[2 * (kBlock / 64)];
@@ -1407,16 +1412,17 @@ int launch_batches(sg_graph_t g, bool bc, int32_t nsrc, const int32_t* sources, 
     caps.hc_cap = chunks_bound;
     caps.li_cap = kLiRing;
   }
-  /* MS-BFS; BC with exponents; BC without (per offset width) */
-  const void* const kernels[3] = {reinterpret_cast<const void*>(ms_kernel<false, true, OffT>),
-                                  reinterpret_cast<const void*>(ms_kernel<true, false, OffT>),
-                                  reinterpret_cast<const void*>(ms_kernel<true, true, OffT>)};
-  static int occs[3] = {0, 0, 0};
+  /* MS-BFS; BC with exponents; BC without, many pairs and few (per offset width) */
+  const void* const kernels[4] = {reinterpret_cast<const void*>(ms_kernel<false, true, kFewWaves, OffT>),
+                                  reinterpret_cast<const void*>(ms_kernel<true, false, kFewWaves, OffT>),
+                                  reinterpret_cast<const void*>(ms_kernel<true, true, kRowWaves, OffT>),
+                                  reinterpret_cast<const void*>(ms_kernel<true, true, kFewWaves, OffT>)};
+  static int occs[3] = {0, 0, 0}; /* (the last one runs with one workgroup per CU) */
   for (int k = 0; k < 3; ++k)
     if (occs[k] == 0) {
       int nb = 0;
       SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernels[k], kBlock, 0));
-      occs[k] = std::max(1, std::min(nb, k == 2 ? 5 : 4));
+      occs[k] = std::max(1, std::min(nb, k == 2 ? kRowWaves : 4));
     }
   const int grid_n = sg::grid_for(dev, n, kBlock, 8);
 
@@ -1495,8 +1501,9 @@ int launch_batches(sg_graph_t g, bool bc, int32_t nsrc, const int32_t* sources, 
     SG_HIP(hipGetLastError());
     auto launch = [&]() -> int {
       void* args[] = {&a};
-      const int which = !bc ? 0 : (a.plain ? 2 : 1);
-      const int per_cu = m * k <= kFewPairs ? 1 : occs[which];
+      const bool few = m * k <= kFewPairs;
+      const int which = !bc ? 0 : (!a.plain ? 1 : (few ? 3 : 2));
+      const int per_cu = few ? 1 : occs[which];
       SG_HIP(launch_resident(kernels[which], per_cu * dev->cus, kBlock, args, s));
       SG_HIP(hipMemcpyAsync(hctl, a.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s));
       SG_HIP(hipStreamSynchronize(s));
