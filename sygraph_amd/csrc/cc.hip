@@ -108,13 +108,20 @@ __global__ void __launch_bounds__(kBlock) shorten_kernel(uint32_t* parent, int64
   }
 }
 
-/* Every stride-th vertex links its first kSampleArcs arcs; equal parents need
- * no look at the root (an older parent is an ancestor too, so a cached one
- * will do).  Run over a 64th of the vertices first: the arcs between two large
- * trees are a good part of the graph's, and while the trees are apart every
- * one of them chases and tries to hook the same root (2.7 ms on RMAT scale 20
- * in one go).  Once a sample has joined them the rest finds equal parents. */
-constexpr int kFirstStride = 64;
+/* Every stride-th vertex links its first kSampleArcs arcs.  Two that lead to
+ * the same ancestor by ordinary loads need no look at the root (an older
+ * parent is an ancestor too, so a cached one will do): what the roots' words
+ * cost is that every find of a root reads them past the caches.  The arcs
+ * between two large trees are a good part of the graph's, and while the trees
+ * are apart every one of them chases and tries to hook the same root (2.7 ms
+ * on RMAT scale 20 in one go), so the vertices come in steps, a 64th, a 16th,
+ * a fourth and all, the chains shortened between; most arcs of a step then
+ * find equal ancestors.  One step of a 64th ahead of all, without the cached
+ * climb, and these: 60,000 vertices of 6 random arcs 620-930 -> 170 us (410
+ * with every vertex hooked at once), a 1000 x 1000 grid of random ids 2,900 ->
+ * 515 (13,000), a path of 4 M random ids 1,830 -> 925 (1,010), a binary tree
+ * of 60,000 240 -> 145 (110; the launches), RMAT scale 20 equal. */
+constexpr int kLinkStrides[] = {64, 16, 4, 1}, kCachedHops = 8;
 template<typename OffT>
 __global__ void __launch_bounds__(kBlock) sample_link_kernel(const OffT* off, const int32_t* cols, int64_t n,
                                                              uint32_t* parent, int stride) {
@@ -128,8 +135,16 @@ __global__ void __launch_bounds__(kBlock) sample_link_kernel(const OffT* off, co
 #pragma unroll
     for (int k = 0; k < kSampleArcs; ++k) pv[k] = parent[v[k]];
 #pragma unroll
-    for (int k = 0; k < kSampleArcs; ++k)
-      if (pv[k] != pu) hook(parent, (uint32_t)u, v[k]);
+    for (int k = 0; k < kSampleArcs; ++k) {
+      uint32_t x = pu, y = pv[k];
+      for (int h = 0; h < kCachedHops && x != y; ++h) {
+        const uint32_t px = parent[x], py = parent[y];
+        if (px == x && py == y) break;
+        x = px;
+        y = py;
+      }
+      if (x != y) hook(parent, x, y);
+    }
   }
 }
 
@@ -346,10 +361,10 @@ void sample_forest(sg_device_t dev, hipStream_t s, const OffT* off, const int32_
   const int grid = sg::grid_for(dev, n, kBlock, 8);
   first_parent_kernel<OffT><<<grid, kBlock, 0, s>>>(off, cols, n, parent);
   for (int k = 0; k < kShortenPasses; ++k) shorten_kernel<<<grid, kBlock, 0, s>>>(parent, n);
-  sample_link_kernel<OffT><<<sg::grid_for(dev, n / kFirstStride + 1, kBlock, 8), kBlock, 0, s>>>(off, cols, n, parent,
-                                                                                               kFirstStride);
-  shorten_kernel<<<grid, kBlock, 0, s>>>(parent, n);
-  sample_link_kernel<OffT><<<grid, kBlock, 0, s>>>(off, cols, n, parent, 1);
+  for (int stride : kLinkStrides) {
+    sample_link_kernel<OffT><<<sg::grid_for(dev, n / stride + 1, kBlock, 8), kBlock, 0, s>>>(off, cols, n, parent, stride);
+    if (stride > 1) shorten_kernel<<<grid, kBlock, 0, s>>>(parent, n);
+  }
 }
 
 template<typename OffT>

@@ -629,18 +629,25 @@ def test_cc_small_graph_in_a_larger_id_array(sg, device, oracle_mod, n, arcs, be
     G.destroy()
 
 
-@pytest.mark.parametrize("graph", ["columns", "random", "two_grids"])
+@pytest.mark.parametrize("graph", ["columns", "random", "two_grids", "tree", "path", "forest"])
 @pytest.mark.parametrize("noalloc", [False, True])
 def test_cc_first_parents_and_chains(sg, device, oracle_mod, graph, noalloc):
     """Forests whose first parents form chains longer than the passes that shorten them reach (one
-    column of 9,000 vertices), none at all, and several components of the same size; unsorted lists."""
+    column of 9,000 vertices), none at all, and several components of the same size, trees that are joined
+    late, and paths of ids in any order; unsorted lists."""
     import ctypes as C
     if graph == "columns":
         g = oracle_mod.grid(9000, 3, 0.0)
     elif graph == "random":
         g = oracle_mod.erdos_renyi(30000, 25000, seed=9)
-    else:
+    elif graph == "two_grids":
         g = oracle_mod.grid(400, 300, 0.35, seed=12)
+    elif graph == "tree":  # the largest id alone under a leaf of the last level but one: every tree hooks to it late
+        g = oracle_mod.csr_from_pairs(1 << 17, np.arange(1, 1 << 17), (np.arange(1, 1 << 17) - 1) // 2)
+    else:  # a path of ids in any order, whole, or cut into pieces of a thousand
+        p = np.random.default_rng(13).permutation(150001)
+        keep = np.ones(150000, dtype=bool) if graph == "path" else np.arange(150000) % 1000 != 7
+        g = oracle_mod.csr_from_pairs(150001, p[:-1][keep], p[1:][keep])
     cols = g.cols.copy()
     rng = np.random.default_rng(5)
     for v in rng.integers(0, g.n, 2000):  # arcs in any order
