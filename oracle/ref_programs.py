@@ -77,7 +77,7 @@ def _jobs(ref: str):
 def build(ref: str = DEFAULT_REF, workers: int = 8) -> list[str]:
     """Compile every program; returns the names that failed (empty on success,
     and where the reference tree is absent or empty)."""
-    if not os.path.isdir(os.path.join(ref, "examples")):
+    if not os.path.isdir(ref) or not os.listdir(ref):
         return []
     os.makedirs(os.path.join(OUT, "examples"), exist_ok=True)
     os.makedirs(os.path.join(OUT, "tests"), exist_ok=True)

@@ -378,3 +378,17 @@ def test_bc_path_length_identity_on_long_grids(oracle_mod):
     b20 = oracle_mod.bc(g2, srcs20)
     ref = sum(oracle_mod.bc(g2, [s]) for s in srcs20)
     assert np.allclose(b20, ref, rtol=1e-12, atol=1e-12)
+
+
+def test_reference_programs_of_a_partial_tree_fail(tmp_path, monkeypatch):
+    """An absent or empty reference tree has nothing to build; one that lacks sources fails, by name."""
+    from oracle import ref_programs
+
+    monkeypatch.setattr(ref_programs, "OUT", str(tmp_path / "out"))
+    monkeypatch.setattr(ref_programs, "HIPCC", "/bin/false")
+    empty, partial = tmp_path / "empty", tmp_path / "partial"
+    empty.mkdir()
+    (partial / "tests").mkdir(parents=True)
+    assert ref_programs.build(str(tmp_path / "absent")) == [] == ref_programs.build(str(empty))
+    failed = ref_programs.build(str(partial))
+    assert {"bfs", "bfs_shared", "algorithms_bc"} <= set(failed)
