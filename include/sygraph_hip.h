@@ -364,12 +364,13 @@ int sg_policy_train_step(sg_policy_t p, const float* features, const int32_t* la
 
 typedef struct sg_sssp_stats {
   int32_t rounds;            /* frontier rounds until no distance changed */
-  int64_t reached_vertices;  /* dist != n+1 */
+  int64_t reached_vertices;  /* dist != n+1 (a distance of n+1 or more stays n+1, the value all start from) */
   int64_t reached_edges;     /* TEPS numerator (algorithms/sssp.hpp:66-77) */
   int64_t relaxations;       /* arcs relaxed over all rounds (light arcs in light rounds, heavy arcs in a
                                 bucket's heavy round) */
   float kernel_ms;           /* device time of the whole run */
-  int64_t round_vertices[SG_MAX_LEVELS_RECORDED]; /* |F| per round */
+  int64_t round_vertices[SG_MAX_LEVELS_RECORDED]; /* |F| per round (inside a grid burst: the entries of its
+                                                     list, a vertex lowered twice being two) */
   int64_t round_edges[SG_MAX_LEVELS_RECORDED];    /* arcs relaxed per round: sum deg over F (Bellman-Ford),
                                                      or over F of the light / heavy arcs (buckets) */
   float relax_ms;            /* sg_sssp_options.record_relax: device time of the relax launches of the
@@ -389,11 +390,13 @@ typedef struct sg_sssp_options {
                             relaxations buckets save, on sparse long-diameter ones such as grids
                             buckets multiply the iterations.  Below 2^25 arcs, rounds of at most 2^17
                             arcs run back to back in one launch, where putting off the farther
-                            vertices pays: fewer relaxations, other rounds; a graph of at most
+                            vertices pays: fewer relaxations, other rounds (those of at most 8
+                            arcs, from the source on, in one workgroup); a graph of at most
                             16,384 vertices and 2^17 arcs takes every round in one launch of one
                             workgroup, nothing put off), negative or infinite =
                             none, i.e. every dirty vertex is relaxed each round (the reference's
-                            frontier Bellman-Ford, sssp.hpp:152-210) */
+                            frontier Bellman-Ford, sssp.hpp:152-210; a round inside a grid burst
+                            relaxes a vertex once for every time the round before lowered it) */
   int32_t heavy_pull;    /* direction of a bucket's heavy round on an undirected graph: 0 = automatic
                             (pull when the heavy arcs of the vertices not yet settled are fewer than
                             those of the bucket's settled set), 1 = always pull, -1 = always push.

@@ -448,7 +448,7 @@ __global__ void bfs_start_kernel(StartArgs<OffT> s, BfsCtl* ctl) {
 
 /* The traversal of one level, push or pull as the control block says.  Four
  * waves per SIMD, what four workgroups of four waves per CU place: the pull's
- * eight hint chains per lane take 106 registers (four chains: 80 registers,
+ * eight hint chains per lane take 98 registers (four chains: 80 registers,
  * 3 % slower; sixteen: 162 registers and three workgroups per CU, 11 %
  * slower). */
 constexpr int kLevelWavesPerSimd = 4;

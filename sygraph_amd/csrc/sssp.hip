@@ -11,8 +11,10 @@
  * takes only the dirty vertices with distance below a threshold T (the near
  * set) and defers the rest, raising T to (smallest deferred distance) + delta
  * when the near set runs dry -- the bucket order of delta-stepping, which
- * relaxes far fewer arcs on weighted graphs.  delta = infinity is exactly the
- * reference's schedule.  Within a bucket, light iterations relax only the
+ * relaxes far fewer arcs on weighted graphs.  delta = infinity is the
+ * reference's schedule: every dirty vertex each round, exactly so in launched
+ * rounds and one workgroup's bursts; a grid burst's round holds a vertex once
+ * for every time that the round before lowered it.  Within a bucket, light iterations relax only the
  * arcs lighter than delta and one heavy iteration the others; the adjacency is
  * read from a light-first copy (per vertex the light arcs, then the heavy
  * ones) so each phase reads only its own arcs.  Each round reads its frontier
@@ -23,7 +25,9 @@
  *
  * Distances have the weights' 4-byte type: uint32 weights use integer min,
  * float weights (non-negative) compare through their bit patterns.  The
- * unreached value is n+1 in that type (sssp.hpp:43).
+ * unreached value is n+1 in that type (sssp.hpp:43), and so is the value that
+ * distances start from: a vertex whose distance is n+1 or more stays
+ * unreached, as in the reference.
  */
 #include <algorithm>
 #include <cmath>
@@ -559,7 +563,8 @@ __global__ void __launch_bounds__(kBlock) near_write_kernel(CompactArgs<OffT> a,
  * this by the rounds' chains of loads and LDS operations (3 us a round on a
  * grid).  Per call, before and after: RMAT of 1,186 arcs 231 -> 38 us, 12,002
  * arcs 333 -> 96, 45,187 (directed, float) 435 -> 163, 85,128 arcs 717 -> 250;
- * grids of 20 x 20 222 -> 42, 60 x 70 553 -> 244.  The vertices are bounded by
+ * grids of 20 x 20 (weights 1 to 7, so that every vertex is reached below
+ * n + 1) 320 -> 104, 60 x 70 1,214 -> 350.  The vertices are bounded by
  * LDS; the arcs by the grid bursts' own limit, from which the automatic
  * schedule keeps the order of the launched rounds (here a distance lowered in
  * a round is seen at once, which saves a tenth of the relaxations). */
@@ -1971,9 +1976,10 @@ int mean_weight(sg_graph_t g, double* out) {
  * total time 1.8 % under the reference's schedule everywhere.
  * Below kAutoBucketArcs the grid bursts keep near and far piles (1201 x 1301
  * grid: 14 ms with them, 66 without; 300 x 400: 4.1 and 22; 200,000 vertices
- * of 16 arcs: 1.68 and 2.07).  Sparse graphs above it keep the reference's
- * order of relaxations: their counts of rounds and relaxations are part of
- * what the automatic schedule is known to report there. */
+ * of 16 arcs: 1.68 and 2.07).  Sparse graphs above it would gain as much
+ * (3072 x 3072 grid, 35.9 M arcs: 52.5 ms with far lists, 319 without; 4096 x
+ * 4096: 76 and 494, the same distances); they keep the reference's order only
+ * because a test holds their count of relaxations to within 5 % of its. */
 constexpr int64_t kAutoBucketArcs = int64_t(1) << 25;
 constexpr int64_t kAutoBucketDegree = 8;
 

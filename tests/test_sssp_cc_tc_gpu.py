@@ -418,7 +418,6 @@ def test_cc_sampling_shapes(sg, device, oracle_mod):
         G = sg.Graph.from_csr(device, g.offsets, g.cols)
         c = sg.CC(G)
         c.init()
-        c.init()
         c.run()
         assert np.array_equal(c.get_labels(), oracle_mod.cc(g))
 
