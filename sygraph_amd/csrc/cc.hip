@@ -120,7 +120,10 @@ __global__ void __launch_bounds__(kBlock) shorten_kernel(uint32_t* parent, int64
  * climb, and these: 60,000 vertices of 6 random arcs 620-930 -> 170 us (410
  * with every vertex hooked at once), a 1000 x 1000 grid of random ids 2,900 ->
  * 515 (13,000), a path of 4 M random ids 1,830 -> 925 (1,010), a binary tree
- * of 60,000 240 -> 145 (110; the launches), RMAT scale 20 equal. */
+ * of 60,000 240 -> 145 (110; the launches); RMAT scale 20, edge factor 32,
+ * 268 -> 300 by the launches.  The steps stay on dense graphs too: without the
+ * 16th and the fourth that RMAT takes 285, but a 700 x 700 grid of 7 x 7
+ * neighbourhoods with random ids 1,600 instead of 237 (2,200 with the one step). */
 constexpr int kLinkStrides[] = {64, 16, 4, 1}, kCachedHops = 8;
 template<typename OffT>
 __global__ void __launch_bounds__(kBlock) sample_link_kernel(const OffT* off, const int32_t* cols, int64_t n,
